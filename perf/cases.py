@@ -70,8 +70,9 @@ def draw(rng):
         return {"kind": kind, "rows": rows, "columns": rng.choice(["ssb", "ssb", "mixed"]),
                 "pred_load": rng.random() < 0.25}
     if kind == "star":
-        return {"kind": kind, "query": rng.choice(["q21", "q21_pht", "q31", "q41"]), "rows": rows,
-                "columns": rng.choice(["ssb", "ssb", "ssb", "mixed"])}
+        query = rng.choice(["q21", "q21_pht", "q31", "q41"])  # hash-table probes take bit-packed columns only
+        columns = "ssb" if query == "q21_pht" else rng.choice(["ssb", "ssb", "ssb", "mixed"])
+        return {"kind": kind, "query": query, "rows": rows, "columns": columns}
     if kind == "unpack":
         return {"kind": kind, "bw": rng.randint(1, 32), "values": rows, "checksum": rng.random() < 0.5}
     if kind == "decode":
