@@ -262,8 +262,7 @@ __global__ __launch_bounds__(kBlock) void features_kernel(const uint32_t* __rest
 __global__ __launch_bounds__(kBlock) void mixed_plan_kernel(const uint32_t* __restrict in, uint64_t n, uint64_t n_vec,
                                                             uint8_t* __restrict cls, const float* __restrict conf,
                                                             float conf_min, uint32_t* __restrict words,
-                                                            uint32_t* __restrict encw, uint64_t* __restrict aux,
-                                                            uint32_t* __restrict fallbacks) {
+                                                            uint32_t* __restrict encw, uint64_t* __restrict aux) {
     const uint64_t v = (uint64_t)blockIdx.x * kVecPerBlock + (threadIdx.x >> 5);
     if (v >= n_vec) return;
     uint32_t x[32];
@@ -281,12 +280,9 @@ __global__ __launch_bounds__(kBlock) void mixed_plan_kernel(const uint32_t* __re
     if (dev::lane32() == 0) {
         const uint32_t w = enc_width(enc, st);
         words[v] = (mix_bytes(enc, st) - 16u) / 4u;
-        encw[v] = (enc << 6) | w;
+        encw[v] = (enc << 6) | w | (fallback ? kScanFlag : 0u);  // the offset scan counts the flags
         aux[v] = enc_aux(enc, st);
-        if (fallback) {
-            cls[v] = (uint8_t)mix_class(enc, w);
-            if (fallbacks) atomicAdd(fallbacks, 1u);
-        }
+        if (fallback) cls[v] = (uint8_t)mix_class(enc, w);
     }
 }
 
@@ -465,6 +461,7 @@ constexpr uint32_t kSpinMax = 1u << 26;
 struct EncodeLds {
     PackLds pack;
     uint32_t words[kVecPerBlock];
+    uint32_t fallback[kVecPerBlock];
     uint64_t base;
     uint32_t ticket;
 };
@@ -490,7 +487,10 @@ __global__ __launch_bounds__(kBlock) void mixed_encode_kernel(const uint32_t* __
         p = plan_vector(r, cls[v], conf, conf_min, v);
     }
     const uint32_t words = live ? (mix_bytes(p.enc, p.st) - 16u) / 4u : 0u;
-    if (dev::lane32() == 0) lds.words[slot] = words;
+    if (dev::lane32() == 0) {
+        lds.words[slot] = words;
+        lds.fallback[slot] = live && p.fallback;
+    }
     __syncthreads();
     if (threadIdx.x < 64) {  // the first wave: publish, look back, publish
         const uint32_t lane = threadIdx.x;
@@ -538,10 +538,13 @@ __global__ __launch_bounds__(kBlock) void mixed_encode_kernel(const uint32_t* __
     if (live && dev::lane32() == 0) {
         vmeta[v] = FLS_VMETA(off, (p.enc << 6) | p.w);
         aux[v] = enc_aux(p.enc, p.st);
-        if (p.fallback) {
-            cls[v] = (uint8_t)mix_class(p.enc, p.w);
-            if (fallbacks) atomicAdd(fallbacks, 1u);
-        }
+        if (p.fallback) cls[v] = (uint8_t)mix_class(p.enc, p.w);
+    }
+    if (fallbacks && threadIdx.x == 0) {  // one atomic per block, not per vector: they share an address
+        uint32_t c = 0;
+#pragma unroll
+        for (int k = 0; k < kVecPerBlock; ++k) c += lds.fallback[k];
+        if (c) atomicAdd(fallbacks, c);
     }
     pack_vector(r, live, p.enc, p.w, off, enc_aux(p.enc, p.st), lds.pack.tile[slot], lds.pack.cnt[slot], out);
 }
@@ -724,9 +727,9 @@ int fls_mixed_plan_device(const uint32_t* d_in, uint64_t n, uint8_t* d_class, co
     uint64_t* bsum = reinterpret_cast<uint64_t*>(static_cast<char*>(d_scratch) + (2 * n_vec * 4 + 255) / 256 * 256);
     hipStream_t s = as_stream(stream);
     hipLaunchKernelGGL(mixed_plan_kernel, dim3((uint32_t)ceil_div(n_vec, kVecPerBlock)), dim3(kBlock), 0, s, d_in, n,
-                       n_vec, d_class, d_conf, conf_min, words, encw, d_aux, d_fallbacks);
+                       n_vec, d_class, d_conf, conf_min, words, encw, d_aux);
     if (const int rc = check_launch()) return rc;
-    return scan_offsets(words, encw, n_vec, bsum, d_vmeta, d_total_words, s);
+    return scan_offsets(words, encw, n_vec, bsum, d_vmeta, d_total_words, s, d_fallbacks);
 }
 
 int fls_mixed_encode_device(const uint32_t* d_in, uint64_t n, uint8_t* d_class, const float* d_conf, float conf_min,
