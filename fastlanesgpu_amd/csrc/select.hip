@@ -14,18 +14,14 @@
 //    plan (chosen encoding's statistics -> size) -> scan -> pack.
 //
 // Work-item t of a 256-work-item block serves lane t%32 of vector
-// blockIdx.x*8 + t/32.  Loads are coalesced: lane l reads rows 32j + l
-// (j = 0..31), i.e. element l of every 32-row chain j -- FastLanes delta's
-// chains are 32 consecutive rows, chain c owned in the packed format by the
-// lane l with 2*(l%16) + l/16 = c, its element j in register row rsum_row(j)
-// (rsum.cuh:8-106).  Chain deltas are therefore neighbour-lane differences
-// (one shuffle), and the pack step moves chains to their owning lanes
-// through a padded LDS tile.  Every exchange stays inside one wave.
+// blockIdx.x*8 + t/32 in the coalesced layout of fls_rows.hpp.  Every exchange
+// stays inside one wave.
 #include "fls/device/unpack.hpp"
 #include "fls/device/wave.hpp"
 #include "fls_columns.hpp"
 #include "fls_encode.hpp"
 #include "fls_rng.hpp"
+#include "fls_rows.hpp"
 #include "fls_runtime.hpp"
 #include "fls_select.hpp"
 
@@ -34,58 +30,6 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kVecPerBlock = kBlock / 32;
-
-__device__ __forceinline__ uint32_t wid(uint32_t x) { return x ? 32u - __clz(x) : 0u; }
-// Half-wave (32-lane) reductions.  Within a 16-lane row DPP moves data at
-// VALU speed (quad_perm swaps at distance 1 and 2, then row_ror:4 and
-// row_ror:8 -- after the quad steps each lane holds its quad, and each
-// rotation doubles the span, so every row lane ends with the row total, for
-// sums too); one lane exchange then joins the two rows of the half-wave.
-template <int CTRL>
-__device__ __forceinline__ uint32_t dpp(uint32_t x) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, false);
-}
-constexpr int kQuadXor1 = 0xB1, kQuadXor2 = 0x4E, kRowRor4 = 0x124, kRowRor8 = 0x128;
-constexpr int kWaveShr1 = 0x138;  // lane i <- lane i-1
-
-template <typename Op>
-__device__ __forceinline__ uint32_t half_reduce(uint32_t x, Op op) {
-    x = op(x, dpp<kQuadXor1>(x));
-    x = op(x, dpp<kQuadXor2>(x));
-    x = op(x, dpp<kRowRor4>(x));
-    x = op(x, dpp<kRowRor8>(x));
-    return op(x, (uint32_t)__shfl_xor(x, 16, 64));
-}
-__device__ __forceinline__ uint32_t h_or(uint32_t x) {
-    return half_reduce(x, [](uint32_t a, uint32_t b) { return a | b; });
-}
-__device__ __forceinline__ uint32_t h_min(uint32_t x) {
-    return half_reduce(x, [](uint32_t a, uint32_t b) { return min(a, b); });
-}
-__device__ __forceinline__ uint32_t h_max(uint32_t x) {
-    return half_reduce(x, [](uint32_t a, uint32_t b) { return max(a, b); });
-}
-__device__ __forceinline__ uint32_t h_sum(uint32_t x) {
-    return half_reduce(x, [](uint32_t a, uint32_t b) { return a + b; });
-}
-
-__device__ __forceinline__ uint32_t chain_slot(uint32_t l) { return 2u * (l & 15u) + (l >> 4); }
-
-__device__ __forceinline__ uint32_t padded(const uint32_t* __restrict in, uint64_t n, uint64_t k) {
-    return in[k < n ? k : n - 1];
-}
-
-// Coalesced load of vector v: x[j] = row 32j + l (rows past n repeat row n-1).
-__device__ __forceinline__ void load_rows(const uint32_t* __restrict in, uint64_t n, uint64_t v, uint32_t (&x)[32]) {
-    const uint64_t base = v * 1024u + dev::lane32();
-    if (v * 1024u + 1024u <= n) {
-#pragma unroll
-        for (int j = 0; j < 32; ++j) x[j] = __builtin_nontemporal_load(in + base + 32u * j);
-    } else {
-#pragma unroll
-        for (int j = 0; j < 32; ++j) x[j] = padded(in, n, base + 32u * j);
-    }
-}
 
 // Statistics of the vector from the coalesced layout (half-wave reductions).
 // ALL: every encoding's; otherwise only those of encoding `enc`.
@@ -262,7 +206,9 @@ __global__ __launch_bounds__(kBlock) void features_kernel(const uint32_t* __rest
 __global__ __launch_bounds__(kBlock) void mixed_plan_kernel(const uint32_t* __restrict in, uint64_t n, uint64_t n_vec,
                                                             uint8_t* __restrict cls, const float* __restrict conf,
                                                             float conf_min, uint32_t* __restrict words,
-                                                            uint32_t* __restrict encw, uint64_t* __restrict aux) {
+                                                            uint32_t* __restrict encw, uint64_t* __restrict aux,
+                                                            ScanState state) {
+    scan_clear(state);
     const uint64_t v = (uint64_t)blockIdx.x * kVecPerBlock + (threadIdx.x >> 5);
     if (v >= n_vec) return;
     uint32_t x[32];
@@ -293,14 +239,6 @@ __global__ __launch_bounds__(kBlock) void mixed_plan_kernel(const uint32_t* __re
 // over the chains before the lane's and the run values, both through LDS.
 // A vector lives in one half-wave, so every exchange is wave-local: the
 // kernel has no block barrier.
-constexpr int kTile = 32 * 33;
-
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 struct PackLds {
     uint32_t tile[kVecPerBlock][kTile];  // transpose tile, then the RLE run values
     uint32_t cnt[kVecPerBlock][32];
@@ -316,10 +254,7 @@ __device__ __forceinline__ void pack_vector(const uint32_t (&r)[32], bool live, 
     const uint32_t l = dev::lane32();
     const uint32_t c = chain_slot(l);  // the chain this lane packs
     uint32_t x[32];
-    if (live) {
-#pragma unroll
-        for (int j = 0; j < 32; ++j) tile[33 * j + l] = r[j];  // element l of chain j
-    }
+    if (live) rows_to_tile(r, tile);
     wave_sync();
     uint32_t before = 0;
     if (live) {
@@ -576,7 +511,9 @@ struct Candidates {
 };
 
 __global__ void trial_choose_kernel(Candidates c, uint64_t n_vec, uint8_t* __restrict cls, uint32_t* __restrict words,
-                                    uint32_t* __restrict encw, uint64_t* __restrict aux, uint8_t* __restrict pick) {
+                                    uint32_t* __restrict encw, uint64_t* __restrict aux, uint8_t* __restrict pick,
+                                    ScanState state) {
+    scan_clear(state);
     for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n_vec; v += (uint64_t)gridDim.x * blockDim.x) {
         uint32_t best = 0;
         uint64_t best_size = ~0ull;
@@ -722,14 +659,12 @@ int fls_mixed_plan_device(const uint32_t* d_in, uint64_t n, uint8_t* d_class, co
     if (n == 0) return zero_u64(d_total_words, 1, as_stream(stream));
     FLS_RETURN_IF(!d_in || !d_class || !d_vmeta || !d_aux || !d_total_words || !d_scratch, FLS_ERR_NULL);
     const uint64_t n_vec = ceil_div(n, 1024);
-    uint32_t* encw = static_cast<uint32_t*>(d_scratch);
-    uint32_t* words = encw + n_vec;
-    uint64_t* bsum = reinterpret_cast<uint64_t*>(static_cast<char*>(d_scratch) + (2 * n_vec * 4 + 255) / 256 * 256);
+    const EncodeScratch e = encode_scratch(d_scratch, n_vec);
     hipStream_t s = as_stream(stream);
     hipLaunchKernelGGL(mixed_plan_kernel, dim3((uint32_t)ceil_div(n_vec, kVecPerBlock)), dim3(kBlock), 0, s, d_in, n,
-                       n_vec, d_class, d_conf, conf_min, words, encw, d_aux);
+                       n_vec, d_class, d_conf, conf_min, e.words, e.bws, d_aux, e.state);
     if (const int rc = check_launch()) return rc;
-    return scan_offsets(words, encw, n_vec, bsum, d_vmeta, d_total_words, s, d_fallbacks);
+    return scan_offsets(e, n_vec, d_vmeta, d_total_words, s, d_fallbacks);
 }
 
 int fls_mixed_encode_device(const uint32_t* d_in, uint64_t n, uint8_t* d_class, const float* d_conf, float conf_min,
@@ -812,13 +747,11 @@ int fls_mixed_encode_trial(const uint32_t* d_in, uint64_t n, uint8_t* d_class, f
         c.total[e] = ct;
         c.words[e] = cw;
     }
-    uint32_t* encw = static_cast<uint32_t*>(scratch);
-    uint32_t* words = encw + n_vec;
-    uint64_t* bsum = reinterpret_cast<uint64_t*>(static_cast<char*>(scratch) + (2 * n_vec * 4 + 255) / 256 * 256);
+    const EncodeScratch sc = encode_scratch(scratch, n_vec);
     hipLaunchKernelGGL(trial_choose_kernel, dim3((uint32_t)ceil_div(n_vec, 256)), dim3(256), 0, s, c, n_vec, d_class,
-                       words, encw, d_aux, pick);
+                       sc.words, sc.bws, d_aux, pick, sc.state);
     if (const int rc = check_launch()) return rc;
-    if (const int rc = scan_offsets(words, encw, n_vec, bsum, d_vmeta, d_total_words, s)) return rc;
+    if (const int rc = scan_offsets(sc, n_vec, d_vmeta, d_total_words, s)) return rc;
     hipLaunchKernelGGL(trial_gather_kernel, dim3(vblocks), dim3(kBlock), 0, s, c, n_vec, pick, d_vmeta, d_out);
     return check_launch();
 }

@@ -94,3 +94,58 @@ def test_rle_roundtrip_gpu(case):
     padded = np.full(n_vec * 1024, x[-1], np.uint32)
     padded[:n] = x
     np.testing.assert_array_equal(u32(out), T.transpose_vectors(padded))
+
+
+@pytest.mark.parametrize("n", [1, 31, 33, 1023, 1024, 1025, 8 * 1024 - 1, 8 * 1024 + 1])
+def test_encoders_at_vector_and_block_edges(n):
+    """Sizes around a chain, a vector and a block of 8 vectors: bit-pack in both
+    orders with a base, delta against the host encoder, RLE by round trip."""
+    torch = T.torch_cuda()
+    rng = np.random.default_rng(n)
+    x = rng.integers(50, 50 + 2**13, n).astype(np.uint32)
+    d = T.to_dev(x)
+    for transposed in (False, True):
+        want = fls.pack_column((x - 50).astype(np.uint32), 13, transpose=transposed)
+        got = u32(fls.pack_column_device(d, n, 13, base=50, transposed=transposed))[: want.size]
+        np.testing.assert_array_equal(got, want, err_msg=f"transposed={transposed}")
+    words, vmeta, bases = fls.delta_encode_column(x)
+    dw, dv, db = fls.delta_encode_device(d, n)
+    np.testing.assert_array_equal(T.from_dev(dv, np.uint64)[: vmeta.size], vmeta)
+    np.testing.assert_array_equal(u32(db)[: bases.size], bases)
+    np.testing.assert_array_equal(u32(dw)[: words.size], words)
+    x = np.repeat(x[: n // 3 + 1], 3)[:n]
+    words, vmeta, rmeta, bases = fls.rle_encode_device(T.to_dev(x), n)
+    n_vec = (n + 1023) // 1024
+    out = torch.empty(n_vec * 1024, dtype=torch.int32, device="cuda")
+    fls.rle_decode(words, vmeta, rmeta, bases, n_vec, out)
+    padded = np.full(n_vec * 1024, x[-1], np.uint32)
+    padded[:n] = x
+    np.testing.assert_array_equal(u32(out), T.transpose_vectors(padded))
+
+
+@pytest.mark.parametrize("n_vec", [4095, 4096, 4097, 2 * 4096 + 3])
+def test_offsets_over_several_scan_blocks(n_vec):
+    """Offsets, total and fallback count where the scan runs in one block, in
+    exactly one, and in several (4,096 vectors each)."""
+    import fastlanesgpu_amd.selector as sel
+    torch = T.torch_cuda()
+    n = n_vec * 1024 - 5
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n_vec)
+    # a width of its own for every vector: 1-bit to 16-bit steps between neighbours
+    top = torch.randint(1, 17, (n_vec,), generator=g, device="cuda", dtype=torch.int32).repeat_interleave(1024)[:n]
+    d = torch.randint(0, 1 << 30, (n,), generator=g, device="cuda", dtype=torch.int32) & ((1 << top) - 1)
+    words, vmeta, _ = fls.delta_encode_device(d, n)
+    vm = T.from_dev(vmeta, np.uint64)
+    sizes = 32 * (vm & np.uint64(255))
+    want = np.concatenate([[0], np.cumsum(sizes)])
+    np.testing.assert_array_equal(vm >> np.uint64(8), want[:-1])
+    assert words.numel() == want[-1]
+    ws = sel.MixedWorkspace(n)
+    conf = torch.rand(n_vec, generator=g, device="cuda")
+    ws.cls.zero_()
+    ws.fallbacks.zero_()
+    sel.mixed_plan(d, n, ws, conf=conf, conf_min=0.3)
+    assert int(ws.fallbacks.item()) == int((conf < 0.3).sum())
+    sel.mixed_plan(d, n, ws, conf=conf, conf_min=0.3)  # the counter is added to
+    assert int(ws.fallbacks.item()) == 2 * int((conf < 0.3).sum())
