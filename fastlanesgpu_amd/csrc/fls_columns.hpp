@@ -91,14 +91,6 @@ __device__ __forceinline__ void decode_fixed(const ColDev& c, uint64_t v, uint32
     }
 }
 
-// FastLanes delta column: unpack at the vector's own width, then the
-// in-register rsum seeded with the lane's base.
-__device__ __forceinline__ void decode_delta(const ColDev& c, uint64_t v, uint32_t (&x)[32]) {
-    const fls_vmeta m = c.vmeta[v];
-    dev::unpack_device(c.words + FLS_VMETA_OFFSET(m), x, FLS_VMETA_BW(m));
-    dev::rsum_lane(x, c.bases[v * 32u + dev::lane32()]);
-}
-
 // Value k of a linear LSB-first bit-packing at width bw (bw <= 32).
 __device__ __forceinline__ uint32_t linear_extract(const uint32_t* __restrict w, uint32_t k, uint32_t bw) {
     if (bw == 0) return 0u;
@@ -116,6 +108,8 @@ __device__ __forceinline__ uint32_t linear_extract(const uint32_t* __restrict w,
 // of the run values straight from the column (a vector's run values are at
 // most 1024 packed values, so the gathers hit the cache after the first).
 // Row order: normal for BITPACK unless c.transposed, transposed otherwise.
+// RLE = false leaves the gather out, for callers that take RLE vectors apart.
+template <bool RLE = true>
 __device__ __forceinline__ void decode_regs(const ColDev& c, uint64_t v, uint32_t (&x)[32]) {
     const uint32_t l = dev::lane32();
     const uint32_t* p;
@@ -164,7 +158,7 @@ __device__ __forceinline__ void decode_regs(const ColDev& c, uint64_t v, uint32_
     }
     dev::unpack_device(p, x, w);
     if (rsum) dev::rsum_lane(x, seed);
-    if (vals) {
+    if (RLE && vals) {
         const uint32_t last = nr ? nr - 1u : 0u;
 #pragma unroll
         for (int r = 0; r < 32; ++r) {
@@ -359,95 +353,6 @@ __device__ __forceinline__ uint32_t live_row_mask(uint32_t live, bool transposed
     const uint32_t part = 0x11111111u & ((1u << (4u * s)) - 1u);  // s <= 7
     const uint32_t sh = q < 4 ? (0x3120u >> (4u * q)) & 3u : 0u;
     return m | (part << sh);
-}
-
-// FastLanes RLE decode of vector v, one lane, into 32 rows (transposed order).
-// `stage` is this vector's 1024-entry LDS slice; the 32 lanes of the vector
-// first unpack the run values into it (about 4 per lane at 128 runs), then
-// each row reads its value by run index.  All 64 work-items of the wave must
-// call it (it waits on the wave's own LDS writes only).
-__device__ __forceinline__ void decode_rle(const ColDev& c, const fls_rle_meta* __restrict rmeta, uint64_t v,
-                                           uint32_t* __restrict stage, bool live, uint32_t (&x)[32]) {
-    fls_vmeta m = 0;
-    fls_rle_meta rm{};
-    if (live) {
-        m = c.vmeta[v];
-        rm = rmeta[v];
-        const uint32_t* vals = c.words + FLS_VMETA_OFFSET(m) + 32u * FLS_VMETA_BW(m);
-        const uint32_t nr = rm.n_runs < 1024u ? rm.n_runs : 1024u;  // the stage holds one vector's runs
-        for (uint32_t k = dev::lane32(); k < nr; k += 32u) stage[k] = rm.vbase + linear_extract(vals, k, rm.vbw);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (!live) return;
-    dev::unpack_device(c.words + FLS_VMETA_OFFSET(m), x, FLS_VMETA_BW(m));
-    dev::rsum_lane(x, c.bases[v * 32u + dev::lane32()]);
-    const uint32_t last = rm.n_runs ? min((uint32_t)rm.n_runs, 1024u) - 1u : 0u;  // inside this vector's stage
-#pragma unroll
-    for (int r = 0; r < 32; ++r) x[r] = stage[min(x[r], last)];
-}
-
-// MIXED column: vector v decoded with its own encoding (fls.h FLS_ENC_MIXED),
-// transposed order.  Like decode_rle, every work-item of the wave calls it.
-__device__ __forceinline__ void decode_mixed(const ColDev& c, uint64_t v, uint32_t* __restrict stage, bool live,
-                                             uint32_t (&x)[32]) {
-    uint32_t enc = 0, w = 0;
-    uint64_t ax = 0;
-    const uint32_t* p = c.words;
-    if (live) {
-        const fls_vmeta m = c.vmeta[v];
-        enc = (uint32_t)(m >> 6) & 3u;
-        w = (uint32_t)m & 63u;
-        ax = c.aux[v];
-        p = c.words + FLS_VMETA_OFFSET(m);
-    }
-    const uint32_t ibw = (uint32_t)(ax >> 48) & 1u, nr_field = (uint32_t)(ax >> 32) & 0xffffu;
-    const uint32_t nr = nr_field < 1024u ? nr_field : 1024u;  // the stage holds one vector's runs
-    if (live && enc == FLS_MIX_RLE) {
-        const uint32_t* vals = p + 32u + 32u * ibw;
-        for (uint32_t k = dev::lane32(); k < nr; k += 32u) stage[k] = (uint32_t)ax + linear_extract(vals, k, w);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (!live) return;
-    const uint32_t l = dev::lane32();
-    switch (enc) {
-        case FLS_MIX_BITPACK: dev::unpack_device(p, x, w); break;
-        case FLS_MIX_FOR:
-            dev::unpack_device(p, x, w);
-#pragma unroll
-            for (int r = 0; r < 32; ++r) x[r] += (uint32_t)ax;
-            break;
-        case FLS_MIX_DELTA:
-            dev::unpack_device(p + 32, x, w);
-            dev::rsum_lane(x, p[l]);
-            break;
-        default: {
-            dev::unpack_device(p + 32, x, ibw);
-            dev::rsum_lane(x, p[l]);
-            const uint32_t last = nr ? nr - 1u : 0u;
-#pragma unroll
-            for (int r = 0; r < 32; ++r) x[r] = stage[min(x[r], last)];
-        }
-    }
-}
-
-// Any column encoding, width known at run time.  `stage` is this vector's
-// 1024-entry LDS slice (RLE / MIXED); every work-item of the wave calls it.
-__device__ __forceinline__ void decode_col(const ColDev& c, uint64_t v, uint32_t* __restrict stage, bool live,
-                                           uint32_t (&x)[32]) {
-    switch (c.enc) {
-        case FLS_ENC_BITPACK:
-            if (live) decode_fixed<-1>(c, v, x);
-            break;
-        case FLS_ENC_DELTA:
-            if (live) decode_delta(c, v, x);
-            break;
-        case FLS_ENC_RLE: decode_rle(c, reinterpret_cast<const fls_rle_meta*>(c.aux), v, stage, live, x); break;
-        default: decode_mixed(c, v, stage, live, x); break;
-    }
 }
 
 // Predicate-fused FastLanes delta walk of one lane at compile-time width BW:

@@ -20,6 +20,7 @@
 #include "fls/device/wave.hpp"
 #include "fls_columns.hpp"
 #include "fls_encode.hpp"
+#include "fls_materialize.hpp"
 #include "fls_rng.hpp"
 #include "fls_rows.hpp"
 #include "fls_runtime.hpp"
@@ -484,22 +485,6 @@ __global__ __launch_bounds__(kBlock) void mixed_encode_kernel(const uint32_t* __
     pack_vector(r, live, p.enc, p.w, off, enc_aux(p.enc, p.st), lds.pack.tile[slot], lds.pack.cnt[slot], out);
 }
 
-__global__ __launch_bounds__(kBlock) void mixed_decode_kernel(const uint32_t* __restrict words,
-                                                              const fls_vmeta* __restrict vmeta,
-                                                              const uint64_t* __restrict aux, uint64_t n_vec,
-                                                              uint32_t* __restrict out) {
-    __shared__ uint32_t stage[kVecPerBlock][1024];
-    const uint64_t v = (uint64_t)blockIdx.x * kVecPerBlock + (threadIdx.x >> 5);
-    const bool live = v < n_vec;
-    ColDev c{FLS_ENC_MIXED, 0, 0, 1, words, vmeta, nullptr, aux};
-    uint32_t x[32];
-    decode_mixed(c, v, stage[threadIdx.x >> 5], live, x);
-    if (!live) return;
-    uint32_t* o = out + v * 1024u + dev::lane32();
-#pragma unroll
-    for (int r = 0; r < 32; ++r) o[32 * r] = x[r];
-}
-
 // Try-all-encodings search, last two steps: every vector has been encoded
 // four times (candidate columns cand[e]); keep the smallest (ties to the
 // lower encoding number) ...
@@ -614,9 +599,8 @@ int fls_mixed_decode_u32(const uint32_t* d_words, const fls_vmeta* d_vmeta, cons
     using namespace fls;
     if (n_vec == 0) return FLS_OK;
     FLS_RETURN_IF(!d_words || !d_vmeta || !d_aux || !d_out, FLS_ERR_NULL);
-    hipLaunchKernelGGL(mixed_decode_kernel, dim3((uint32_t)ceil_div(n_vec, kVecPerBlock)), dim3(kBlock), 0,
-                       as_stream(stream), d_words, d_vmeta, d_aux, n_vec, d_out);
-    return check_launch();
+    const ColDev c{FLS_ENC_MIXED, 0, 0, 1, d_words, d_vmeta, nullptr, d_aux};
+    return materialize(c, n_vec * 1024u, false, d_out, as_stream(stream));
 }
 
 int fls_gen_train_vectors(uint64_t seed, uint64_t first_vector, uint64_t n_vec, const uint32_t* d_zipf_cdf,

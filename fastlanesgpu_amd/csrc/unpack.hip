@@ -10,6 +10,7 @@
 #include "fls/device/unpack.hpp"
 #include "fls/device/wave.hpp"
 #include "fls_columns.hpp"
+#include "fls_materialize.hpp"
 #include "fls_runtime.hpp"
 
 namespace fls {
@@ -161,24 +162,6 @@ __global__ __launch_bounds__(kBlock) void delta_decode_kernel(const uint32_t* __
     for (int r = 0; r < 32; ++r) __builtin_nontemporal_store(vals[r], o + 32 * r);
 }
 
-// FastLanes RLE decode (run values staged per vector in LDS), transposed order.
-__global__ __launch_bounds__(kBlock) void rle_decode_kernel(const uint32_t* __restrict words,
-                                                            const fls_vmeta* __restrict vmeta,
-                                                            const fls_rle_meta* __restrict rmeta,
-                                                            const uint32_t* __restrict bases, uint64_t n_vec,
-                                                            uint32_t* __restrict out) {
-    __shared__ uint32_t stage[kVecPerBlock][1024];
-    const uint64_t v = (uint64_t)blockIdx.x * kVecPerBlock + (threadIdx.x >> 5);
-    const bool live = v < n_vec;
-    const ColDev c{FLS_ENC_RLE, 0, 0, 1, words, vmeta, bases, nullptr};
-    uint32_t x[32];
-    decode_rle(c, rmeta, v, stage[threadIdx.x >> 5], live, x);
-    if (!live) return;
-    uint32_t* o = out + v * 1024u + dev::lane32();
-#pragma unroll
-    for (int r = 0; r < 32; ++r) __builtin_nontemporal_store(x[r], o + 32 * r);
-}
-
 template <bool WRITE, bool CHECKSUM>
 struct UnpackTable {
     using Fn = void (*)(const uint32_t*, uint32_t*, uint64_t, uint64_t, uint64_t*);
@@ -238,11 +221,8 @@ int fls_rle_decode_u32(const uint32_t* d_words, const fls_vmeta* d_vmeta, const 
                        const uint32_t* d_bases, uint64_t n_vec, uint32_t* d_out, void* stream) {
     if (n_vec == 0) return FLS_OK;
     FLS_RETURN_IF(!d_words || !d_vmeta || !d_rmeta || !d_bases || !d_out, FLS_ERR_NULL);
-    const uint64_t blocks = fls::ceil_div(n_vec, fls::kVecPerBlock);
-    FLS_RETURN_IF(blocks > 0x7fffffffu, FLS_ERR_SIZE);
-    hipLaunchKernelGGL(fls::rle_decode_kernel, dim3((uint32_t)blocks), dim3(fls::kBlock), 0, fls::as_stream(stream),
-                       d_words, d_vmeta, d_rmeta, d_bases, n_vec, d_out);
-    return fls::check_launch();
+    const fls::ColDev c{FLS_ENC_RLE, 0, 0, 1, d_words, d_vmeta, d_bases, reinterpret_cast<const uint64_t*>(d_rmeta)};
+    return fls::materialize(c, n_vec * 1024u, false, d_out, fls::as_stream(stream));
 }
 
 }  // extern "C"

@@ -126,3 +126,84 @@ def test_errors():
     with pytest.raises(fls.FlsError):  # vectors are moved 16 bytes at a time
         d = T.to_dev(np.arange(2048, dtype=np.uint32))
         fls.transpose_vectors(d[1:1025], 1)
+
+
+def rle_vector_column(run_counts, ibw=1, vbw=32):
+    """An RLE column made by hand: vector v has run_counts[v] runs, index deltas
+    packed at ibw bits, run values at vbw bits (reference words only)."""
+    words, vmeta, rmeta, bases, rows, off = [], [], [], [], [], 0
+    for nr in run_counts:
+        starts = np.zeros(1024, np.int64)
+        starts[1 + RNG.choice(1023, nr - 1, replace=False)] = 1
+        idx = np.cumsum(starts).astype(np.uint32)
+        vals = RNG.integers(0, 2**vbw, nr, dtype=np.uint64).astype(np.uint32)
+        vbase = np.uint32(RNG.integers(0, 2**32 - 2**vbw + 1, dtype=np.uint64))
+        t = fls.transpose_i(idx)
+        index_words = fls.pack(fls.unrsum(t), ibw)
+        bits = np.zeros(-(-nr * vbw // 32) * 32, np.uint8)
+        bits[: nr * vbw] = ((vals[:, None] >> np.arange(vbw, dtype=np.uint32)) & 1).ravel()
+        value_words = np.packbits(bits, bitorder="little").view(np.uint32)
+        words += [index_words, value_words]
+        vmeta.append(off << 8 | ibw)
+        rmeta.append(int(vbase) | nr << 32 | vbw << 48 | ibw << 56)
+        bases.append(t[:32])
+        rows.append((vals[idx] + vbase).astype(np.uint32))
+        off += index_words.size + value_words.size
+    host = fls.HostColumn(fls.ENC_RLE, 1024 * len(run_counts), np.concatenate(words + [np.zeros(2, np.uint32)]),
+                          vmeta=np.array(vmeta, np.uint64), bases=np.concatenate(bases),
+                          aux=np.array(rmeta, np.uint64))
+    return host.to_device(), np.concatenate(rows)
+
+
+@pytest.mark.parametrize("ibw,vbw", [(1, 32), (1, 7), (3, 20), (32, 1)])
+def test_decode_rle_run_counts(ibw, vbw):
+    """Run counts around a half-wave, a load step (128) and the stage (512),
+    and index deltas wider than a bit, in both orders, aligned and not."""
+    torch = T.torch_cuda()
+    counts = [1, 2, 31, 32, 33, 127, 128, 129, 511, 512, 513, 700, 1023, 1024, 5]
+    col, rows = rle_vector_column(counts, ibw, vbw)
+    stored = T.transpose_vectors(rows)
+    n = rows.size - 300  # the last vector is partial in row order
+    for shift in (0, 1):
+        buf = torch.full((rows.size + 8,), -1, dtype=torch.int32, device="cuda")
+        fls.decode_column(col, n, fls.ORDER_ROWS, out=buf[shift:shift + n])
+        got = T.from_dev(buf)
+        np.testing.assert_array_equal(got[shift:shift + n], rows[:n])
+        assert np.all(got[shift + n:] == 0xFFFFFFFF)
+        buf.fill_(-1)
+        fls.decode_column(col, rows.size, fls.ORDER_STORED, out=buf[shift:shift + rows.size])
+        np.testing.assert_array_equal(T.from_dev(buf)[shift:shift + rows.size], stored)
+        buf.fill_(-1)
+        fls.rle_decode(col.words, col.vmeta, col.aux, col.bases, len(counts), buf[shift:shift + rows.size])
+        got = T.from_dev(buf)
+        np.testing.assert_array_equal(got[shift:shift + rows.size], stored)
+        assert np.all(got[shift + rows.size:] == 0xFFFFFFFF)
+
+
+def test_decode_mixed_column_with_rle_vectors():
+    """RLE vectors of every run count beside other encodings in one column."""
+    import fastlanesgpu_amd.selector as sel
+    torch = T.torch_cuda()
+    parts = []
+    for k, runs in enumerate([3, 600, 0, 512, 513, 0, 1024, 40, 0]):
+        if runs:
+            cuts = np.sort(RNG.choice(1023, runs - 1, replace=False)) + 1
+            parts.append(np.repeat(RNG.integers(0, 2**20, runs), np.diff(np.concatenate([[0], cuts, [1024]]))))
+        else:
+            parts.append(np.arange(1024) * (k + 1) + RNG.integers(0, 3, 1024))
+    x = np.concatenate(parts).astype(np.uint32)[:-77]
+    ws = sel.MixedWorkspace(x.size)
+    ws.cls[:] = torch.tensor([30 if r else 20 for r in [3, 600, 0, 512, 513, 0, 1024, 40, 0]], dtype=torch.uint8)
+    sel.mixed_encode_classes(T.to_dev(x), x.size, ws)
+    col = ws.column(x.size)
+    padded = np.full(9 * 1024, x[-1], np.uint32)
+    padded[: x.size] = x
+    stored = T.transpose_vectors(padded)
+    for shift in (0, 1):
+        buf = torch.full((9 * 1024 + 8,), -1, dtype=torch.int32, device="cuda")
+        fls.decode_column(col, x.size, fls.ORDER_ROWS, out=buf[shift:shift + x.size])
+        got = T.from_dev(buf)
+        np.testing.assert_array_equal(got[shift:shift + x.size], x)
+        assert np.all(got[shift + x.size:] == 0xFFFFFFFF)
+        sel.mixed_decode(col, out=buf[shift:])
+        np.testing.assert_array_equal(T.from_dev(buf)[shift:shift + 9 * 1024], stored)
