@@ -101,6 +101,120 @@ __device__ __forceinline__ uint32_t linear_extract(const uint32_t* __restrict w,
     return __builtin_amdgcn_alignbit(hi, lo, s) & mask;
 }
 
+// ------------------------------------------------- any encoding, one vector
+// A vector's metadata, loaded ahead of its payload: its vmeta and, for RLE and
+// MIXED columns, its aux word (RLE: vbase | n_runs << 32 | vbw << 48).
+struct VecMeta {
+    fls_vmeta m;
+    uint32_t aux_lo, aux_hi;
+};
+__device__ __forceinline__ VecMeta load_meta(const ColDev& c, uint64_t v) {
+    VecMeta t{0, 0, 0};
+    if (c.enc != FLS_ENC_BITPACK) t.m = ldg(c.vmeta + v);
+    if (c.enc == FLS_ENC_RLE || c.enc == FLS_ENC_MIXED) {  // RLE metadata is 4-byte aligned
+        const uint32_t* ax = reinterpret_cast<const uint32_t*>(c.aux) + 2u * v;
+        t.aux_lo = ldg(ax);
+        t.aux_hi = ldg(ax + 1);
+    }
+    return t;
+}
+
+// Where a vector's parts lie.  Every encoding is one unpack at width w, then a
+// base added (add), or the in-register rsum from the lane's seed (chain: delta,
+// and the run index of RLE), and for RLE a look-up among n_runs values packed
+// at vbw bits (vals; add is their base).
+struct VecParts {
+    const uint32_t* p;     // packed words
+    const uint32_t* seed;  // the vector's 32 chain seeds, or null
+    const uint32_t* vals;  // RLE run values, or null
+    uint32_t w, add, n_runs, vbw;
+    const uint32_t* first;  // the vector's words in the column's words array ...
+    uint32_t words;         // ... and how many
+};
+__device__ __forceinline__ VecParts vec_parts(const ColDev& c, uint64_t v, const VecMeta& t) {
+    VecParts q{};
+    uint32_t w = (uint32_t)t.m & 255u, rle = c.enc == FLS_ENC_RLE, chain = rle || c.enc == FLS_ENC_DELTA;
+    q.first = c.words + FLS_VMETA_OFFSET(t.m);
+    if (c.enc == FLS_ENC_BITPACK) {
+        w = c.bw;
+        q.first = c.words + v * (32u * c.bw);
+        q.add = c.base;
+    }
+    q.p = q.first;
+    if (chain) q.seed = c.bases + v * 32u;
+    q.vbw = (t.aux_hi >> 16) & 255u;
+    if (c.enc == FLS_ENC_MIXED) {
+        const uint32_t enc = (w >> 6) & 3u;
+        w &= 63u;
+        rle = enc == FLS_MIX_RLE;
+        chain = rle || enc == FLS_MIX_DELTA;
+        if (enc == FLS_MIX_FOR) q.add = t.aux_lo;
+        q.vbw = w;
+        if (rle) w = (t.aux_hi >> 16) & 1u;
+        if (chain) {
+            q.seed = q.p;
+            q.p += 32;
+        }
+    }
+    q.w = w;
+    q.words = (uint32_t)(q.p - q.first) + 32u * w;
+    if (rle) {
+        q.add = t.aux_lo;
+        q.n_runs = min(t.aux_hi & 0xffffu, 1024u);
+        q.vals = q.p + 32u * w;
+        q.words += (q.n_runs * q.vbw + 31u) / 32u;
+    }
+    return q;
+}
+
+// One word of each line of the vector's payload, all of them asked for with
+// one or two load instructions whatever its width: brings the payload into the
+// cache while other columns are decoded.  The caller keeps the results alive
+// (asm) up to where it wants them to have arrived.
+__device__ __forceinline__ void touch_payload(const VecParts& q, uint32_t& t0, uint32_t& t1) {
+    const uint32_t at = 32u * dev::lane32(), last = q.words - 1u;
+    t0 = q.words && at < q.words + 31u ? ldg(q.first + min(at, last)) : 0u;
+    t1 = q.words && at + 1024u < q.words + 31u ? ldg(q.first + min(at + 1024u, last)) : 0u;
+}
+
+// Run values staged at a time for a vector's look-ups.
+constexpr uint32_t kLookRuns = 512;
+
+// The vector decoded into the lane's 32 rows.  `stage`: kLookRuns words of LDS
+// of this half-wave, for RLE vectors (more runs than that are read from the
+// column a row at a time).  Exchanges stay inside the half-wave.
+__device__ __forceinline__ void decode_parts(const VecParts& q, uint32_t* __restrict stage, uint32_t (&x)[32]) {
+    const uint32_t l = dev::lane32();
+    const uint32_t seed = q.seed ? ldg(q.seed + l) : 0u;
+    const bool staged = q.vals && q.n_runs <= kLookRuns;
+    if (staged)
+        for (uint32_t k = l; k < q.n_runs; k += 32u) stage[k] = q.add + linear_extract(q.vals, k, q.vbw);
+    dev::unpack_device(q.p, x, q.w);
+    if (q.seed) dev::rsum_lane(x, seed);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (!q.vals) {
+#pragma unroll
+        for (int r = 0; r < 32; ++r) x[r] += q.add;
+    } else {
+        const uint32_t last = q.n_runs ? q.n_runs - 1u : 0u;
+        if (staged) {
+#pragma unroll
+            for (int r = 0; r < 32; ++r) {
+                x[r] = stage[min(x[r], last)];
+                if ((r & 7) == 7) __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 32; ++r) {
+                x[r] = q.add + linear_extract(q.vals, min(x[r], last), q.vbw);
+                __builtin_amdgcn_sched_barrier(0);  // one row's gather at a time: 32 hoisted addresses spill
+            }
+        }
+    }
+}
+
 // Any column encoding (BITPACK, DELTA, RLE, MIXED) decoded into registers with
 // no LDS and no wave barrier, for kernels whose LDS holds dimension tables.
 // Every encoding reduces to one unpack at a run-time width, then a FOR add, or
@@ -429,23 +543,7 @@ __device__ __forceinline__ uint32_t delta_mask(const ColDev& c, uint64_t v, Pred
 // register row r (a compile-time constant after unrolling, so a caller's
 // per-row arrays stay in registers), with only the packed words of the
 // vector's width held -- no 32-row decoded array is needed by the walk
-// itself.  Row masks are the walk with f = "set bit r if pred(value)"; a
-// kernel that handles every width and encoding this way stays near 40-80
-// VGPRs.
-
-// fixed width (bit-pack, + FOR base); lane_in = first word of this lane
-template <int BW, typename F>
-__device__ __forceinline__ void walk_fixed_lane(const uint32_t* __restrict lane_in, uint32_t base, F& f) {
-    if constexpr (BW == 0) {
-#pragma unroll
-        for (int r = 0; r < 32; ++r) f(r, base);
-    } else {
-        uint32_t w[BW];
-        load_lane_g<BW>(lane_in, w);
-#pragma unroll
-        for (int r = 0; r < 32; ++r) f(r, dev::extract_at<BW>(w, r) + base);
-    }
-}
+// itself.
 
 // FastLanes delta: the running sum visits the rows in chain order
 template <int BW, typename F>
@@ -471,18 +569,6 @@ __device__ __forceinline__ void walk_delta_lane(const uint32_t* __restrict lane_
         X(20) X(21) X(22) X(23) X(24) X(25) X(26) X(27) X(28) X(29) X(30) X(31) X(32)
 
 template <typename F>
-__device__ __forceinline__ void walk_fixed(const uint32_t* __restrict lane_in, uint32_t bw, uint32_t base, F& f) {
-    switch (bw) {
-#define FLS_WF_CASE(B)                               \
-    case B: walk_fixed_lane<B>(lane_in, base, f); \
-        break;
-        FLS_WIDTH_CASES(FLS_WF_CASE)
-#undef FLS_WF_CASE
-        default: break;
-    }
-}
-
-template <typename F>
 __device__ __forceinline__ void walk_delta(const uint32_t* __restrict lane_in, uint32_t bw, uint32_t first, F& f) {
     switch (bw) {
 #define FLS_WD_CASE(B)                                \
@@ -492,109 +578,6 @@ __device__ __forceinline__ void walk_delta(const uint32_t* __restrict lane_in, u
 #undef FLS_WD_CASE
         default: break;
     }
-}
-
-// FastLanes RLE: the run index of the lane's rows is a delta chain of width
-// ibw (0: the whole lane is one run; 1: one word, bit r = 1 where row r starts
-// a run); `stage` holds the vector's run values, `last` = n_runs - 1.
-template <typename F>
-__device__ __forceinline__ void walk_rle(const uint32_t* __restrict idx_lane, uint32_t ibw, uint32_t first_idx,
-                                         const uint32_t* __restrict stage, uint32_t last, F& f) {
-    if (ibw == 0) {
-        const uint32_t x = stage[min(first_idx, last)];
-#pragma unroll
-        for (int r = 0; r < 32; ++r) f(r, x);
-        return;
-    }
-    const uint32_t starts = ldg_nt(idx_lane);
-    uint32_t acc = first_idx;
-#pragma unroll
-    for (int j = 0; j < 32; ++j) {
-        const int r = dev::rsum_row(j);
-        acc += (starts >> r) & 1u;
-        f(r, stage[min(acc, last)]);
-    }
-}
-
-// Stage the n_runs (<= 1024) run values of a vector into LDS; every
-// work-item of the wave calls it (`active` = this half-wave has a vector).
-__device__ __forceinline__ void stage_runs(const uint32_t* __restrict vals, uint32_t n_runs, uint32_t vbw,
-                                           uint32_t vbase, uint32_t* __restrict stage, bool active) {
-    if (active) {
-        const uint32_t nr = n_runs < 1024u ? n_runs : 1024u;
-        for (uint32_t k = dev::lane32(); k < nr; k += 32u) stage[k] = vbase + linear_extract(vals, k, vbw);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Walk vector v of any column encoding (run-time width and encoding).  Every
-// work-item of the wave calls it (RLE run values are staged in `stage`, this
-// vector's 1024-entry LDS slice); f is called only when `live`.  `rmeta`:
-// the RLE metadata (c.aux of an RLE column).
-template <typename F>
-__device__ __forceinline__ void column_walk(const ColDev& c, const fls_rle_meta* __restrict rmeta, uint64_t v,
-                                            uint32_t* __restrict stage, bool live, F& f) {
-    const uint32_t l = dev::lane32();
-    if (c.enc == FLS_ENC_BITPACK) {
-        if (live) walk_fixed(c.words + v * (32u * c.bw) + l, c.bw, c.base, f);
-        return;
-    }
-    if (c.enc == FLS_ENC_DELTA) {
-        if (!live) return;
-        const fls_vmeta m = ldg(c.vmeta + v);
-        walk_delta(c.words + FLS_VMETA_OFFSET(m) + l, FLS_VMETA_BW(m), ldg(c.bases + v * 32u + l), f);
-        return;
-    }
-    if (c.enc == FLS_ENC_RLE) {
-        fls_vmeta m = 0;
-        fls_rle_meta rm{};
-        if (live) {
-            m = ldg(c.vmeta + v);
-            rm = ldg(rmeta + v);
-        }
-        const uint32_t* p = c.words + FLS_VMETA_OFFSET(m);
-        const uint32_t ibw = FLS_VMETA_BW(m) ? 1u : 0u;
-        stage_runs(p + 32u * ibw, rm.n_runs, rm.vbw, rm.vbase, stage, live);
-        if (!live) return;
-        const uint32_t last = rm.n_runs ? min((uint32_t)rm.n_runs, 1024u) - 1u : 0u;
-        walk_rle(p + l, ibw, ldg(c.bases + v * 32u + l), stage, last, f);
-        return;
-    }
-    // MIXED
-    uint32_t enc = 0, w = 0;
-    uint64_t ax = 0;
-    const uint32_t* p = c.words;
-    if (live) {
-        const fls_vmeta m = ldg(c.vmeta + v);
-        enc = (uint32_t)(m >> 6) & 3u;
-        w = (uint32_t)m & 63u;
-        ax = ldg(c.aux + v);
-        p = c.words + FLS_VMETA_OFFSET(m);
-    }
-    const uint32_t ibw = (uint32_t)(ax >> 48) & 1u, nr = (uint32_t)(ax >> 32) & 0xffffu;
-    stage_runs(p + 32u + 32u * ibw, nr, w, (uint32_t)ax, stage, live && enc == FLS_MIX_RLE);
-    if (!live) return;
-    switch (enc) {
-        case FLS_MIX_BITPACK: walk_fixed(p + l, w, 0u, f); break;
-        case FLS_MIX_FOR: walk_fixed(p + l, w, (uint32_t)ax, f); break;
-        case FLS_MIX_DELTA: walk_delta(p + 32u + l, w, ldg(p + l), f); break;
-        default: {
-            const uint32_t last = nr ? min(nr, 1024u) - 1u : 0u;
-            walk_rle(p + 32u + l, ibw, ldg(p + l), stage, last, f);
-        }
-    }
-}
-
-// Row mask {r : pred(value of row r)} of vector v, any encoding.
-template <typename Pred>
-__device__ __forceinline__ uint32_t column_mask(const ColDev& c, const fls_rle_meta* __restrict rmeta, uint64_t v,
-                                                uint32_t* __restrict stage, bool live, Pred pred) {
-    uint32_t m = 0;
-    auto f = [&](int r, uint32_t x) { m |= (uint32_t)pred(x) << r; };
-    column_walk(c, rmeta, v, stage, live, f);
-    return m;
 }
 
 }  // namespace fls

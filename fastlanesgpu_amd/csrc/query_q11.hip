@@ -32,7 +32,7 @@ constexpr int kBlock = 256;
 constexpr int kVecPerBlock = kBlock / 32;
 
 struct Q11Dev {
-    ColDev date, qty, disc, price;
+    ColDev cols[4];  // orderdate, quantity, discount, price
     uint64_t n_rows, n_vec, n_groups;
     uint32_t date_gt, date_lt, qty_lt, disc_lo, disc_hi;
     int64_t* revenue;
@@ -95,52 +95,82 @@ __device__ __forceinline__ void q11_block_finish(const Q11Dev& a, const uint64_t
     }
 }
 
+// 0 or 1 in a register, so that shifting it into a row mask is one
+// v_lshl_or_b32 (left to itself the compiler selects between 0 and 32
+// constants that it keeps in 32 registers).
+__device__ __forceinline__ uint32_t row_bit(bool f) {
+    uint32_t b = f;
+    asm("" : "+v"(b));
+    return b;
+}
+
 // Generic path: any encoding per column (bit-pack + FOR, delta, RLE, mixed),
-// run-time widths.  Every column is walked row by row at its own width
-// (column_walk): orderdate and quantity reduce straight to row masks,
-// discount is kept as 32 values (it is both filtered and multiplied), and
-// price is multiplied in place during its walk -- one 32-value array live,
-// not one per column.  RLE / MIXED columns stage run values in LDS.
+// run-time widths.  The four columns of a vector go through one copy of the
+// decoder (decode_parts) in a rolled loop: four inlined copies of 33 widths
+// were 1.3 MB of code, and their loop-invariant constants took 220 VGPRs, two
+// waves per SIMD.  Bound by the round trips from metadata to payload to the
+// next column, so all columns' lines are asked for before the first is decoded
+// (touch_payload) and four waves per SIMD run.  59,986,214 mixed rows: 103.1 us
+// with the inlined copies, 95.2 rolled, 59.3 with the lines asked for ahead
+// (4.5 TB/s).  As in the fast path, a wave whose rows have all failed leaves
+// the rest of the vector's ALU work out after its lines have been read; PRED
+// does not read them (34.1 -> 31.1 us).
 template <bool PRED>
-__global__ __launch_bounds__(kBlock) void q11_kernel(const Q11Dev a) {
-    __shared__ uint32_t stage[kVecPerBlock][1024];
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void q11_kernel(const Q11Dev a) {
+    __shared__ uint32_t stage[kVecPerBlock][kLookRuns];
     uint32_t* st = stage[threadIdx.x >> 5];
     uint64_t acc = 0;
     uint32_t cnt = 0;
-    const bool transposed = a.price.transposed != 0;
+    const bool transposed = a.cols[3].transposed != 0;
     const uint32_t dlo = a.date_gt + 1u, dspan = a.date_lt - a.date_gt - 1u;
     const bool ok = a.date_lt > a.date_gt && a.disc_hi >= a.disc_lo;
     const uint32_t span = a.disc_hi - a.disc_lo, qty_lt = a.qty_lt, disc_lo = a.disc_lo;
-    const auto* date_rm = reinterpret_cast<const fls_rle_meta*>(a.date.aux);
-    const auto* qty_rm = reinterpret_cast<const fls_rle_meta*>(a.qty.aux);
-    const auto* disc_rm = reinterpret_cast<const fls_rle_meta*>(a.disc.aux);
-    const auto* price_rm = reinterpret_cast<const fls_rle_meta*>(a.price.aux);
-    for (uint64_t g = blockIdx.x; g < a.n_groups; g += gridDim.x) {
-        const uint64_t v = g * kVecPerBlock + (threadIdx.x >> 5);
-        const bool live = v < a.n_vec;  // RLE / MIXED staging needs the whole wave, so no early exit
-        uint32_t m = 0;
-        if (live && ok) {
-            const uint64_t first = v * 1024u;
-            m = first + 1024u <= a.n_rows ? 0xffffffffu : live_row_mask((uint32_t)(a.n_rows - first), transposed);
-        }
-        m &= column_mask(a.date, date_rm, v, st, live, [dlo, dspan](uint32_t x) { return (x - dlo) < dspan; });
-        if (PRED && !__any(m != 0)) continue;
-        m &= column_mask(a.qty, qty_rm, v, st, live, [qty_lt](uint32_t x) { return x < qty_lt; });
-        if (PRED && !__any(m != 0)) continue;
-        uint32_t d[32];
-        auto keep_disc = [&](int r, uint32_t x) { d[r] = x; };
-        column_walk(a.disc, disc_rm, v, st, live, keep_disc);
-        if (live) {
+    const uint64_t v0 = (uint64_t)blockIdx.x * kVecPerBlock + (threadIdx.x >> 5);
+    for (uint64_t v = v0; v < a.n_vec; v += (uint64_t)gridDim.x * kVecPerBlock) {
+        uint32_t t[6];
+        if constexpr (!PRED) {
 #pragma unroll
-            for (int r = 0; r < 32; ++r) {
-                m &= ~((uint32_t)((d[r] - disc_lo) > span) << r);
-                d[r] &= 0u - ((m >> r) & 1u);  // rows that fail contribute 0
-            }
+            for (int k = 1; k < 4; ++k)
+                touch_payload(vec_parts(a.cols[k], v, load_meta(a.cols[k], v)), t[2 * k - 2], t[2 * k - 1]);
         }
-        if (PRED && !__any(m != 0)) continue;
-        auto mac = [&](int r, uint32_t x) { acc += (uint64_t)x * (uint64_t)d[r]; };
-        column_walk(a.price, price_rm, v, st, live, mac);
-        cnt += (uint32_t)__builtin_popcount(m);
+        const uint64_t first = v * 1024u;
+        uint32_t m = first + 1024u <= a.n_rows ? 0xffffffffu : live_row_mask((uint32_t)(a.n_rows - first), transposed);
+        if (!ok) m = 0;
+        uint32_t d[32];
+        // the columns in turn through one copy of the decoder
+#pragma unroll 1
+        for (int k = 0; k < 4; ++k) {
+            const ColDev& c = a.cols[k];
+            uint32_t x[32];
+            decode_parts(vec_parts(c, v, load_meta(c, v)), st, x);
+            uint32_t f = 0;
+            if (k == 0) {
+#pragma unroll
+                for (int r = 0; r < 32; ++r) f |= row_bit(x[r] - dlo < dspan) << r;
+                m &= f;
+                if constexpr (!PRED) {
+#pragma unroll
+                    for (int i = 0; i < 6; ++i) asm volatile("" : : "v"(t[i]));
+                }
+            } else if (k == 1) {
+#pragma unroll
+                for (int r = 0; r < 32; ++r) f |= row_bit(x[r] < qty_lt) << r;
+                m &= f;
+            } else if (k == 2) {
+#pragma unroll
+                for (int r = 0; r < 32; ++r) {
+                    f |= row_bit(x[r] - disc_lo <= span) << r;
+                    d[r] = x[r];
+                }
+                m &= f;
+            } else {
+#pragma unroll
+                for (int r = 0; r < 32; ++r)  // rows that fail contribute 0
+                    acc += (uint64_t)x[r] * (uint64_t)(d[r] & (uint32_t)__builtin_amdgcn_sbfe((int)m, r, 1));
+                cnt += (uint32_t)__builtin_popcount(m);
+            }
+            if (!__any(m != 0)) break;
+        }
     }
     __shared__ uint64_t s_acc[kBlock / 64];
     __shared__ uint64_t s_cnt[kBlock / 64];
@@ -194,8 +224,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     {
         const uint64_t v0 = (uint64_t)blockIdx.x * kVecPerBlock + (threadIdx.x >> 5);
         if (v0 < a.n_vec) {
-            next_m = a.date.vmeta[v0];
-            next_b = a.date.bases[v0 * 32u + l];
+            next_m = a.cols[0].vmeta[v0];
+            next_b = a.cols[0].bases[v0 * 32u + l];
         }
     }
     for (uint64_t g = blockIdx.x; g < a.n_groups; g += gridDim.x) {
@@ -204,20 +234,20 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         const uint32_t cur_b = next_b;
         const uint64_t vn = v + (uint64_t)gridDim.x * kVecPerBlock;
         if (vn < a.n_vec) {
-            next_m = a.date.vmeta[vn];
-            next_b = a.date.bases[vn * 32u + l];
+            next_m = a.cols[0].vmeta[vn];
+            next_b = a.cols[0].bases[vn * 32u + l];
         }
         if (v >= a.n_vec) continue;
         uint32_t qw[QBW > 0 ? QBW : 1], dw[DBW > 0 ? DBW : 1], pw[PBW > 0 ? PBW : 1];
         if constexpr (!PRED) {
-            dev::load_lane<QBW>(a.qty.words + v * (32u * QBW) + l, qw);
-            dev::load_lane<DBW>(a.disc.words + v * (32u * DBW) + l, dw);
-            dev::load_lane<PBW>(a.price.words + v * (32u * PBW) + l, pw);
+            dev::load_lane<QBW>(a.cols[1].words + v * (32u * QBW) + l, qw);
+            dev::load_lane<DBW>(a.cols[2].words + v * (32u * DBW) + l, dw);
+            dev::load_lane<PBW>(a.cols[3].words + v * (32u * PBW) + l, pw);
         }
         // orderdate: its per-vector width makes this a (half-wave divergent)
         // switch; widths above 16 take the run-time walk, so at most 16 of
         // its words are live next to the other columns' words
-        uint32_t m = delta_mask_pre(a.date, cur_m, cur_b, [=](uint32_t x) { return (x - dlo) < dspan; });
+        uint32_t m = delta_mask_pre(a.cols[0], cur_m, cur_b, [=](uint32_t x) { return (x - dlo) < dspan; });
         if (v == a.n_vec - 1) m &= tail;
         if (!date_ok || !disc_ok) m = 0;
         if constexpr (!PRED) {
@@ -227,18 +257,18 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             if (!__any(m != 0)) continue;
         } else {
             if (!__any(m != 0)) continue;
-            dev::load_lane<QBW>(a.qty.words + v * (32u * QBW) + l, qw);
-            dev::load_lane<DBW>(a.disc.words + v * (32u * DBW) + l, dw);
-            dev::load_lane<PBW>(a.price.words + v * (32u * PBW) + l, pw);
+            dev::load_lane<QBW>(a.cols[1].words + v * (32u * QBW) + l, qw);
+            dev::load_lane<DBW>(a.cols[2].words + v * (32u * DBW) + l, dw);
+            dev::load_lane<PBW>(a.cols[3].words + v * (32u * PBW) + l, pw);
         }
 #pragma unroll
         for (int r = 0; r < 32; ++r) {
             // branch-free: every term is a 0/1 integer, so the row loop stays
             // one straight-line block
-            const uint32_t q = dev::extract_at<QBW>(qw, r) + a.qty.base;
-            const uint32_t d = dev::extract_at<DBW>(dw, r) + a.disc.base;
+            const uint32_t q = dev::extract_at<QBW>(qw, r) + a.cols[1].base;
+            const uint32_t d = dev::extract_at<DBW>(dw, r) + a.cols[2].base;
             const uint32_t f = ((m >> r) & 1u) & (uint32_t)(q < a.qty_lt) & (uint32_t)((d - a.disc_lo) <= span);
-            const uint32_t p = dev::extract_at<PBW>(pw, r) + a.price.base;
+            const uint32_t p = dev::extract_at<PBW>(pw, r) + a.cols[3].base;
             acc += (uint64_t)p * (uint64_t)(d * f);
             cnt += f;
         }
@@ -310,14 +340,12 @@ extern "C" int fls_query_q11(const fls_column* orderdate, const fls_column* quan
     FLS_RETURN_IF(!orderdate || !quantity || !discount || !price || !p || !d_revenue, FLS_ERR_NULL);
     Q11Dev a{};
     int st;
-    if ((st = to_dev_column(*orderdate, n_rows, &a.date, true)) != FLS_OK) return st;
-    if ((st = to_dev_column(*quantity, n_rows, &a.qty, true)) != FLS_OK) return st;
-    if ((st = to_dev_column(*discount, n_rows, &a.disc, true)) != FLS_OK) return st;
-    if ((st = to_dev_column(*price, n_rows, &a.price, true)) != FLS_OK) return st;
+    const fls_column* cols[4] = {orderdate, quantity, discount, price};
+    for (int k = 0; k < 4; ++k)
+        if ((st = to_dev_column(*cols[k], n_rows, &a.cols[k], true)) != FLS_OK) return st;
     // every column must use the same row order (delta / RLE / mixed imply transposed)
-    const uint32_t tr = a.price.transposed != 0;
-    FLS_RETURN_IF((a.date.transposed != 0) != tr || (a.qty.transposed != 0) != tr || (a.disc.transposed != 0) != tr,
-                  FLS_ERR_ARG);
+    const uint32_t tr = a.cols[3].transposed != 0;
+    for (int k = 0; k < 3; ++k) FLS_RETURN_IF((a.cols[k].transposed != 0) != tr, FLS_ERR_ARG);
     a.n_rows = n_rows;
     a.n_vec = ceil_div(n_rows, 1024);
     a.n_groups = ceil_div(a.n_vec, kVecPerBlock);
@@ -337,8 +365,9 @@ extern "C" int fls_query_q11(const fls_column* orderdate, const fls_column* quan
     }
     if ((st = q11_slot(&a.slot)) != FLS_OK) return st;
     const bool pred = (flags & FLS_Q_PRED_LOAD) != 0;
-    const bool fast = a.date.enc == FLS_ENC_DELTA && a.qty.enc == FLS_ENC_BITPACK && a.disc.enc == FLS_ENC_BITPACK &&
-                      a.price.enc == FLS_ENC_BITPACK && a.qty.bw == 6 && a.disc.bw == 4 && a.price.bw == 24;
+    const ColDev &q = a.cols[1], &d = a.cols[2], &x = a.cols[3];
+    const bool fast = a.cols[0].enc == FLS_ENC_DELTA && q.enc == FLS_ENC_BITPACK && d.enc == FLS_ENC_BITPACK &&
+                      x.enc == FLS_ENC_BITPACK && q.bw == 6 && d.bw == 4 && x.bw == 24;
     if (fast) return launch_fast<6, 4, 24>(a, pred, s);
     return launch_generic(a, pred, s);
 }

@@ -158,3 +158,22 @@ def test_q11_zero_rows():
     out.fill_(7)
     fls.query_q11(*dev, 0, accumulate=True, d_out=out)
     assert out.cpu().tolist() == [7, 7]
+
+
+@pytest.mark.parametrize("pred", [False, True])
+@pytest.mark.parametrize("mean_run", [1, 1.6, 3])
+def test_q11_columns_of_many_runs(mean_run, pred):
+    # RLE columns whose vectors hold more runs than are looked up in LDS
+    # (512), about that many, and fewer, beside a delta and a wide FOR column
+    n = 9 * 1024 + 77
+    rng = np.random.default_rng(int(10 * mean_run))
+    idx = np.cumsum(rng.random(n) < 1 / mean_run)
+    od = T.o_gen_c2(21, n)[0]
+    q = (1 + rng.integers(0, 50, n)).astype(np.uint32)
+    d = rng.integers(0, 11, n).astype(np.uint32)[idx - idx[0]]
+    p = rng.integers(0, 2**32, n, dtype=np.uint64).astype(np.uint32)[idx - idx[0]]
+    cols = [T.encode_any(od, "delta"), T.encode_any(q, "bitpack_t"), T.encode_any(d, "rle"), T.encode_any(p, "rle")]
+    params = (19920000, 19990000, 40, 1, 9)
+    gt, lt, ql, lo, hi = params
+    got = fls.query_q11(*cols, n, gt, lt, ql, lo, hi, pred_load=pred)
+    assert got == T.o_q11([od, q, d, p], n, params)
