@@ -9,11 +9,9 @@
 // order: W1[16][64], b1[64], W2[64][64], b2[64], W3[64][40], b3[40]
 // (W[in][out]); 7,848 values.
 //
-// A wave computes 16 samples at a time (one 16-row MFMA tile).  Training:
-// weights staged once per block in LDS as BF16, activations through per-wave
-// LDS tiles, so every product -- including the transposed ones of the
-// backward pass -- reads its operands with plain strides.  Inference keeps
-// activations in registers between layers (see mlp_forward_kernel).
+// 16 samples at a time (one 16-row MFMA tile): a wave's in inference, which
+// keeps activations in registers between layers (see mlp_forward_kernel), four
+// waves' in training, which exchange activations through LDS (mlp_grad_kernel).
 //
 // MFMA operand layouts used here (lane L of the wave):
 //   16x16x16: A[L % 16][4*(L/16) + i], B[4*(L/16) + i][L % 16], i < 4
@@ -107,79 +105,6 @@ __device__ __forceinline__ f32x4 tile_mm(const View& A, const View& B, int m0, i
 // row of item i of the D tile held by this lane, and its column
 __device__ __forceinline__ int d_row(int i) { return 4 * (lane64() >> 4) + i; }
 __device__ __forceinline__ int d_col() { return lane64() & 15; }
-
-// Per-block LDS: BF16 weights (transposed copies for the backward products
-// are not needed: strides do it) + per-wave activation tiles.
-struct WaveTiles {
-    uint16_t x[16 * kIn];        // X tile, row-major [16][16]
-    uint16_t h1[16 * kH];        // relu(X W1 + b1)
-    uint16_t h2[16 * kH];        // relu(H1 W2 + b2)
-    uint16_t dz[16 * kOutPad];   // dL/dZ (bf16), padded columns zero
-    uint16_t dh2[16 * kH];       // dL/dH2 (masked)
-    uint16_t dh1[16 * kH];       // dL/dH1 (masked)
-    float z[16 * kOutPad];       // logits
-};
-struct MlpLds {
-    uint16_t w1[kIn * kH], w2[kH * kH], w3[kH * kOutPad];
-    float b1[kH], b2[kH], b3[kOutPad];
-    WaveTiles t[1];  // the gradient kernel runs one wave per block
-};
-
-__device__ void stage_weights(const uint16_t* __restrict wb, MlpLds& s) {
-    for (int i = threadIdx.x; i < kIn * kH; i += blockDim.x) s.w1[i] = wb[oW1 + i];
-    for (int i = threadIdx.x; i < kH * kH; i += blockDim.x) s.w2[i] = wb[oW2 + i];
-    for (int i = threadIdx.x; i < kH * kOutPad; i += blockDim.x) {
-        const int r = i / kOutPad, c = i % kOutPad;
-        s.w3[i] = c < kOut ? wb[oW3 + r * kOut + c] : (uint16_t)0;
-    }
-    for (int i = threadIdx.x; i < kH; i += blockDim.x) {
-        s.b1[i] = from_bf16(wb[oB1 + i]);
-        s.b2[i] = from_bf16(wb[oB2 + i]);
-    }
-    for (int i = threadIdx.x; i < kOutPad; i += blockDim.x) s.b3[i] = i < kOut ? from_bf16(wb[oB3 + i]) : 0.f;
-}
-
-// forward of one 16-sample tile (rows >= valid are zero inputs)
-__device__ void forward_tile(const float* __restrict feat, uint64_t s0, uint64_t n, MlpLds& s, WaveTiles& t) {
-    const int L = lane64();
-    for (int i = L; i < 16 * kIn; i += 64) {
-        const uint64_t row = s0 + i / kIn;
-        t.x[i] = to_bf16(row < n ? feat[row * kIn + (i % kIn)] : 0.f);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const View X{t.x, kIn, 1}, W1{s.w1, kH, 1}, W2{s.w2, kH, 1}, W3{s.w3, kOutPad, 1};
-    for (int n0 = 0; n0 < kH; n0 += 16) {
-        const f32x4 acc = tile_mm(X, W1, 0, n0, kIn);
-        for (int i = 0; i < 4; ++i) {
-            const float h = acc[i] + s.b1[n0 + d_col()];
-            t.h1[d_row(i) * kH + n0 + d_col()] = to_bf16(h > 0.f ? h : 0.f);
-        }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const View H1{t.h1, kH, 1};
-    for (int n0 = 0; n0 < kH; n0 += 16) {
-        const f32x4 acc = tile_mm(H1, W2, 0, n0, kH);
-        for (int i = 0; i < 4; ++i) {
-            const float h = acc[i] + s.b2[n0 + d_col()];
-            t.h2[d_row(i) * kH + n0 + d_col()] = to_bf16(h > 0.f ? h : 0.f);
-        }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const View H2{t.h2, kH, 1};
-    for (int n0 = 0; n0 < kOutPad; n0 += 16) {
-        const f32x4 acc = tile_mm(H2, W3, 0, n0, kH);
-        for (int i = 0; i < 4; ++i) t.z[d_row(i) * kOutPad + n0 + d_col()] = acc[i] + s.b3[n0 + d_col()];
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // ------------------------------------------------------------- inference
 // The forward holds the weights and the activations in registers and runs
@@ -351,139 +276,219 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void m
 }
 
 // -------------------------------------------------------------- gradients
-// Softmax cross-entropy, scaled by inv_batch.  Every wave accumulates the
-// gradients of its tiles in registers and writes them, with its summed loss,
-// to its own row of `part` (kPart floats); grad_reduce_kernel then adds the
-// rows in wave order, so a step's gradient is bit-reproducible.  One wave per
-// block and one 16-sample tile per wave up to kGradMaxWaves waves: a 4,096-
-// sample batch is 256 blocks, one per CU (the kernel's chain of dependent
-// products and LDS round trips is latency-bound, so spreading the tiles over
-// the CUs is what shortens it).
+// Softmax cross-entropy, scaled by inv_batch.  Every block accumulates the
+// gradients of its 16-sample tiles in registers and writes them, with its
+// summed loss, to its own row of `part` (kPart floats); grad_reduce_kernel then
+// adds the rows in a fixed order, so a step's gradient is bit-reproducible.
+// One tile per block up to kGradMaxBlocks blocks: a 4,096-sample batch is 256
+// blocks, one per CU.
+//
+// Bound by the chain of dependent products, so a tile is spread over four waves
+// (wave w computes columns 16w .. 16w + 15 of every layer and of the gradients
+// that come back to it) and everything off the chain is kept off it: a wave's
+// weight fragments go from memory straight to its registers, all loads in
+// flight at once, and the D tile of a product (lane L: samples 4 (L / 16) + i of
+// unit L % 16) is already the operand that the weight gradients need, whose
+// depth is the samples.  Activations cross waves through LDS, by sample and by
+// unit, in rows padded for 8- and 16-byte reads; a sample's softmax takes 16
+// lanes, which add its 40 terms in class order.  4,096 samples: 47.8 us with
+// one wave per tile, weights staged in LDS two bytes at a time and the softmax
+// on 16 lanes; 12.2 us this way (65,536 samples: 107.5 and 39.2).
 constexpr int kPart = kParams + 8;  // [kParams] = loss, rest padding
-constexpr int kGradMaxWaves = 1024;
+constexpr int kGradMaxBlocks = 1024;
 
-__global__ __launch_bounds__(64) void mlp_grad_kernel(const uint16_t* __restrict wb, const float* __restrict feat,
+struct GradLds {
+    alignas(16) uint16_t h1[16][72], h2[16][72], dh2[16][72];  // by sample: relu(X W1 + b1), relu(H1 W2 + b2), dL/dH2
+    alignas(16) float z[16][52], e[16][52];                    // logits, exp(logit - largest)
+    alignas(8) uint16_t x[16][20], dz[16][52];                 // by sample: features, dL/dZ
+    alignas(8) uint16_t xt[16][20], dzt[kOutPad][20], dh2t[kH][20], dh1t[kH][20];  // by feature / class / unit
+    float loss[16];
+};
+__device__ __forceinline__ bf16x4 ld4(const uint16_t* p) { return *reinterpret_cast<const bf16x4*>(p); }
+__device__ __forceinline__ s16x8 ld8(const uint16_t* p) { return *reinterpret_cast<const s16x8*>(p); }
+
+__global__ __launch_bounds__(256) void mlp_grad_kernel(const uint16_t* __restrict wb, const float* __restrict feat,
                                                        const uint8_t* __restrict label, uint64_t n, float inv_batch,
                                                        float* __restrict part) {
-    __shared__ MlpLds s;
-    stage_weights(wb, s);
-    __syncthreads();
-    WaveTiles& t = s.t[0];
-    const int L = lane64();
-    // register accumulators of this wave's weight gradients (D-tile layout)
-    f32x4 gw1[4], gw2[16], gw3[12];
-    for (int i = 0; i < 4; ++i) gw1[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int i = 0; i < 16; ++i) gw2[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int i = 0; i < 12; ++i) gw3[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float gb1 = 0.f, gb2 = 0.f, gb3 = 0.f, lsum = 0.f;  // lane L owns column L of each bias
+    __shared__ GradLds s;
+    const int t = threadIdx.x, w = t >> 6, L = lane64(), m = L & 15, q = L >> 4;
+    const int col = 16 * w + m;  // this lane's column of every product
+    // weight fragments: layers 1 to 3 forward, then W3^T and W2^T
+    bf16x4 w1, w3t[3];
+    s16x8 w2[2], w3[2], w2t[2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w1[i] = (short)wb[oW1 + (4 * q + i) * kH + col];
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int k = 32 * c + 8 * q + j;
+            w2[c][j] = (short)wb[oW2 + k * kH + col];
+            w2t[c][j] = (short)wb[oW2 + col * kH + k];
+            w3[c][j] = col < kOut ? (short)wb[oW3 + k * kOut + col] : (short)0;
+        }
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int k = 16 * c + 4 * q + i;
+            w3t[c][i] = k < kOut ? (short)wb[oW3 + col * kOut + k] : (short)0;
+        }
+    const float b1 = from_bf16(wb[oB1 + col]), b2 = from_bf16(wb[oB2 + col]);
+    const float b3 = col < kOut ? from_bf16(wb[oB3 + col]) : 0.f;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    // weight gradients of this wave: dW1 columns 16w.., dW2 and dW3 rows 16w..
+    f32x4 gw1 = zero, gw2[4] = {zero, zero, zero, zero}, gw3[3] = {zero, zero, zero};
+    float gb = 0.f, lsum = 0.f;  // wave 0: column L of b1, wave 1: of b2, wave 2: of b3
     const uint64_t n_tiles = ceil_div(n, 16);
+    const int smp = t >> 4, sub = t & 15;  // the sample and the feature / classes of this work-item
     for (uint64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        const uint64_t s0 = tile * 16;
-        forward_tile(feat, s0, n, s, t);
+        const uint64_t row = tile * 16 + smp;
+        const bool in = row < n;
+        const uint16_t xv = to_bf16(in ? feat[row * kIn + sub] : 0.f);  // rows past n are zero inputs
+        const int y = in ? label[row] : 0;
+        s.x[smp][sub] = xv;
+        s.xt[sub][smp] = xv;
+        __syncthreads();
+        bf16x4 h1, h2, d2, d1;
+        f32x4 acc = mfma(ld4(&s.x[m][4 * q]), w1, zero);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float h = acc[i] + b1;
+            h1[i] = (short)to_bf16(h > 0.f ? h : 0.f);
+            s.h1[4 * q + i][col] = (uint16_t)h1[i];
+        }
+        __syncthreads();
+        acc = mfma32(ld8(&s.h1[m][8 * q]), w2[0], zero);
+        acc = mfma32(ld8(&s.h1[m][32 + 8 * q]), w2[1], acc);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float h = acc[i] + b2;
+            h2[i] = (short)to_bf16(h > 0.f ? h : 0.f);
+            s.h2[4 * q + i][col] = (uint16_t)h2[i];
+        }
+        __syncthreads();
+        if (w < 3) {
+            acc = mfma32(ld8(&s.h2[m][8 * q]), w3[0], zero);
+            acc = mfma32(ld8(&s.h2[m][32 + 8 * q]), w3[1], acc);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s.z[4 * q + i][col] = acc[i] + b3;
+        }
+        __syncthreads();
         // softmax + dZ = (p - onehot) * inv_batch, rows past n contribute nothing
-        if (L < 16) {
-            const uint64_t row = s0 + L;
-            float* z = t.z + L * kOutPad;
-            uint16_t* dz = t.dz + L * kOutPad;
-            if (row < n) {
-                float mx = z[0];
-                for (int c = 1; c < kOut; ++c) mx = fmaxf(mx, z[c]);
-                float sum = 0.f;
-                for (int c = 0; c < kOut; ++c) sum += expf(z[c] - mx);
-                const int y = label[row];
-                lsum += logf(sum) + mx - z[y];
-                for (int c = 0; c < kOut; ++c) {
-                    const float p = expf(z[c] - mx) / sum;
-                    dz[c] = to_bf16((p - (c == y ? 1.f : 0.f)) * inv_batch);
-                }
-            } else {
-                for (int c = 0; c < kOut; ++c) dz[c] = 0;
+        {
+            float z[3], e[3], mx = s.z[smp][sub];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                z[k] = s.z[smp][sub + 16 * k];
+                if (sub + 16 * k < kOut) mx = fmaxf(mx, z[k]);
             }
-            for (int c = kOut; c < kOutPad; ++c) dz[c] = 0;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const View DZ{t.dz, kOutPad, 1};
-        const View H2T{t.h2, 1, kH}, H1T{t.h1, 1, kH}, XT{t.x, 1, kIn};
-        // dW3 += H2^T dZ   (64 x 48, K = 16 samples)
-        for (int mi = 0; mi < 4; ++mi)
-            for (int ni = 0; ni < 3; ++ni)
-                gw3[mi * 3 + ni] = mfma(frag_a(H2T, 16 * mi, 0), frag_b(DZ, 0, 16 * ni), gw3[mi * 3 + ni]);
-        // dH2 = dZ W3^T, masked by H2 > 0
-        const View W3T{s.w3, 1, kOutPad};
-        for (int n0 = 0; n0 < kH; n0 += 16) {
-            const f32x4 acc = tile_mm(DZ, W3T, 0, n0, kOutPad);
-            for (int i = 0; i < 4; ++i) {
-                const int r = d_row(i), c = n0 + d_col();
-                t.dh2[r * kH + c] = to_bf16(from_bf16(t.h2[r * kH + c]) > 0.f ? acc[i] : 0.f);
+#pragma unroll
+            for (int off = 8; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                e[k] = expf(z[k] - mx);
+                s.e[smp][sub + 16 * k] = e[k];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            float sum = 0.f;
+#pragma unroll
+            for (int c = 0; c < kOut; c += 4) {
+                const f32x4 v = *reinterpret_cast<const f32x4*>(&s.e[smp][c]);
+                sum += v[0];
+                sum += v[1];
+                sum += v[2];
+                sum += v[3];
+            }
+            if (in && sub == 0) lsum += logf(sum) + mx - s.z[smp][y];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const int c = sub + 16 * k;
+                const float p = e[k] / sum;
+                const uint16_t d = in && c < kOut ? to_bf16((p - (c == y ? 1.f : 0.f)) * inv_batch) : (uint16_t)0;
+                s.dz[smp][c] = d;
+                s.dzt[c][smp] = d;
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const View DH2{t.dh2, kH, 1};
-        // dW2 += H1^T dH2
-        for (int mi = 0; mi < 4; ++mi)
-            for (int ni = 0; ni < 4; ++ni)
-                gw2[mi * 4 + ni] = mfma(frag_a(H1T, 16 * mi, 0), frag_b(DH2, 0, 16 * ni), gw2[mi * 4 + ni]);
-        // dH1 = dH2 W2^T, masked by H1 > 0
-        const View W2T{s.w2, 1, kH};
-        for (int n0 = 0; n0 < kH; n0 += 16) {
-            const f32x4 acc = tile_mm(DH2, W2T, 0, n0, kH);
-            for (int i = 0; i < 4; ++i) {
-                const int r = d_row(i), c = n0 + d_col();
-                t.dh1[r * kH + c] = to_bf16(from_bf16(t.h1[r * kH + c]) > 0.f ? acc[i] : 0.f);
-            }
+        __syncthreads();
+        // dH2 = dZ W3^T, masked by H2 > 0; dW3 += H2^T dZ
+        acc = zero;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) acc = mfma(ld4(&s.dz[m][16 * c + 4 * q]), w3t[c], acc);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            d2[i] = (short)to_bf16(h2[i] > 0 ? acc[i] : 0.f);
+            s.dh2[4 * q + i][col] = (uint16_t)d2[i];
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const View DH1{t.dh1, kH, 1};
-        // dW1 += X^T dH1  (16 x 64)
-        for (int ni = 0; ni < 4; ++ni) gw1[ni] = mfma(frag_a(XT, 0, 0), frag_b(DH1, 0, 16 * ni), gw1[ni]);
-        // bias gradients: column sums over the tile's 16 rows
-        for (int r = 0; r < 16; ++r) {
-            gb1 += from_bf16(t.dh1[r * kH + L]);
-            gb2 += from_bf16(t.dh2[r * kH + L]);
-            if (L < kOutPad) gb3 += from_bf16(t.dz[r * kOutPad + L]);
+        *reinterpret_cast<bf16x4*>(&s.dh2t[col][4 * q]) = d2;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) gw3[c] = mfma(h2, ld4(&s.dzt[16 * c + m][4 * q]), gw3[c]);
+        __syncthreads();
+        // dH1 = dH2 W2^T, masked by H1 > 0; dW2 += H1^T dH2, dW1 += X^T dH1
+        acc = mfma32(ld8(&s.dh2[m][8 * q]), w2t[0], zero);
+        acc = mfma32(ld8(&s.dh2[m][32 + 8 * q]), w2t[1], acc);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d1[i] = (short)to_bf16(h1[i] > 0 ? acc[i] : 0.f);
+        *reinterpret_cast<bf16x4*>(&s.dh1t[col][4 * q]) = d1;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) gw2[c] = mfma(h1, ld4(&s.dh2t[16 * c + m][4 * q]), gw2[c]);
+        gw1 = mfma(ld4(&s.xt[m][4 * q]), d1, gw1);
+        __syncthreads();
+        // bias gradients: column sums over the tile's 16 samples, in order
+        if (w < 2 || (w == 2 && L < kOutPad)) {
+            const uint16_t* v = w == 0 ? s.dh1t[L] : w == 1 ? s.dh2t[L] : s.dzt[L];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) gb += from_bf16(v[r]);
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    // this wave's row of partial sums: every parameter written exactly once
+    // this block's row of partial sums: every parameter written exactly once
     float* p = part + (uint64_t)blockIdx.x * kPart;
-    for (int mi = 0; mi < 4; ++mi)
-        for (int ni = 0; ni < 3; ++ni)
-            for (int i = 0; i < 4; ++i) {
-                const int r = 16 * mi + d_row(i), c = 16 * ni + d_col();
-                if (c < kOut) p[oW3 + r * kOut + c] = gw3[mi * 3 + ni][i];
-            }
-    for (int mi = 0; mi < 4; ++mi)
-        for (int ni = 0; ni < 4; ++ni)
-            for (int i = 0; i < 4; ++i) p[oW2 + (16 * mi + d_row(i)) * kH + 16 * ni + d_col()] = gw2[mi * 4 + ni][i];
-    for (int ni = 0; ni < 4; ++ni)
-        for (int i = 0; i < 4; ++i) p[oW1 + d_row(i) * kH + 16 * ni + d_col()] = gw1[ni][i];
-    p[oB1 + L] = gb1;
-    p[oB2 + L] = gb2;
-    if (L < kOut) p[oB3 + L] = gb3;
-    const float wl = dev::wave_sum(lsum);
-    if (L == 0) p[kParams] = wl;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = 16 * w + 4 * q + i;
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            if (16 * c + m < kOut) p[oW3 + r * kOut + 16 * c + m] = gw3[c][i];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) p[oW2 + r * kH + 16 * c + m] = gw2[c][i];
+        p[oW1 + (4 * q + i) * kH + col] = gw1[i];
+    }
+    if (w == 0) p[oB1 + L] = gb;
+    if (w == 1) p[oB2 + L] = gb;
+    if (w == 2 && L < kOut) p[oB3 + L] = gb;
+    if (sub == 0) s.loss[smp] = lsum;
+    __syncthreads();
+    if (w == 0) {
+        const float wl = dev::wave_sum(L < 16 ? s.loss[L] : 0.f);
+        if (L == 0) p[kParams] = wl;
+    }
 }
 
-// grad[i] += sum over waves of part[w][i]; *loss likewise (i = kParams).  A
-// block serves 16 parameters with 16 slices each: slice s adds waves
+// grad[i] += sum over blocks of part[w][i]; *loss likewise (i = kParams).  A
+// block serves 16 parameters with 16 slices each: slice s adds rows
 // s, s+16, s+32, ... in order, then slice sums are added in slice order --
-// a fixed order, so the result is bit-reproducible.
-__global__ __launch_bounds__(256) void grad_reduce_kernel(const float* __restrict part, uint32_t n_waves,
+// a fixed order, so the result is bit-reproducible.  Sixteen rows' loads are in
+// flight at a time (one after another: 7.3 us for 256 rows, XX this way).
+__global__ __launch_bounds__(256) void grad_reduce_kernel(const float* __restrict part, uint32_t n_rows,
                                                           float* __restrict grad, float* __restrict loss) {
     __shared__ float red[16][17];
     const int col = threadIdx.x & 15, sl = threadIdx.x >> 4;
     const int i = blockIdx.x * 16 + col;
     float acc = 0.f;
     if (i <= kParams)
-        for (uint32_t w = sl; w < n_waves; w += 16) acc += part[(uint64_t)w * kPart + i];
+        for (uint32_t w0 = sl; w0 < n_rows; w0 += 16 * 16) {
+            float v[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                const uint32_t w = w0 + 16 * k;
+                v[k] = part[(uint64_t)(w < n_rows ? w : w0) * kPart + i];
+            }
+#pragma unroll
+            for (int k = 0; k < 16; ++k)
+                if (w0 + 16 * k < n_rows) acc += v[k];
+        }
     red[sl][col] = acc;
     __syncthreads();
     if (sl == 0 && i <= kParams) {
@@ -496,7 +501,7 @@ __global__ __launch_bounds__(256) void grad_reduce_kernel(const float* __restric
 
 uint32_t grad_blocks(uint64_t n) {
     const uint64_t tiles = ceil_div(n, 16);
-    return (uint32_t)(tiles < 1 ? 1 : tiles > kGradMaxWaves ? kGradMaxWaves : tiles);
+    return (uint32_t)(tiles < 1 ? 1 : tiles > kGradMaxBlocks ? kGradMaxBlocks : tiles);
 }
 
 // Adam on the FP32 master weights; refreshes the BF16 copy and zeroes grad
@@ -575,7 +580,7 @@ int fls_mlp_grad(const uint16_t* d_wb, const float* d_feat, const uint8_t* d_lab
     FLS_RETURN_IF(!d_wb || !d_feat || !d_label || !d_work || !d_grad, FLS_ERR_NULL);
     const uint32_t blocks = grad_blocks(n);
     float* part = static_cast<float*>(d_work);
-    hipLaunchKernelGGL(mlp_grad_kernel, dim3(blocks), dim3(64), 0, as_stream(stream), d_wb, d_feat, d_label, n,
+    hipLaunchKernelGGL(mlp_grad_kernel, dim3(blocks), dim3(256), 0, as_stream(stream), d_wb, d_feat, d_label, n,
                        inv_batch, part);
     if (const int rc = check_launch()) return rc;
     hipLaunchKernelGGL(grad_reduce_kernel, dim3((uint32_t)ceil_div(kParams + 1, 16)), dim3(256), 0,

@@ -326,6 +326,27 @@ def test_mlp_grad_matches_oracle():
     np.testing.assert_allclose(mlp.grad.cpu().numpy(), g1.cpu().numpy(), rtol=1e-4, atol=1e-6)
 
 
+@pytest.mark.parametrize("n", [1, 16, 17, 16 * 1024 + 33])
+def test_mlp_grad_at_tile_and_block_edges(n):
+    """One sample, a full tile, one sample past it, and more tiles than blocks
+    (a block then adds several tiles); the bounds are those of the test above."""
+    torch = torch_cuda()
+    w = rand_weights(15)
+    mlp = sel.Mlp(weights=w)
+    rng = np.random.default_rng(n)
+    feat = rng.random((n, 16)).astype(np.float32)
+    label = rng.integers(0, 40, n).astype(np.uint8)
+    loss = torch.zeros(1, dtype=torch.float32, device="cuda")
+    mlp.grad.zero_()
+    mlp.accumulate_grad(torch.from_numpy(feat).cuda(), torch.from_numpy(label).cuda(), n, 1.0 / n, loss)
+    g = mlp.grad.cpu().numpy().astype(np.float64)
+    ref_loss, ref = o_mlp_grad(w.astype(np.float64), feat, label, True)
+    assert float(loss.item()) == pytest.approx(ref_loss, rel=2e-3)
+    for a, b in [(0, 1024), (1024, 1088), (1088, 5184), (5184, 5248), (5248, 7808), (7808, 7848)]:
+        scale = np.max(np.abs(ref[a:b]))
+        assert np.max(np.abs(g[a:b] - ref[a:b])) <= 2e-2 * scale + 1e-7, (a, b)
+
+
 def test_adam_step():
     torch = torch_cuda()
     w = rand_weights(7)
