@@ -208,6 +208,8 @@ SIGNATURES.update({
     "fls_exhaustive_select": (c_int, [c_vp, c_u64, c_vp, c_vp, c_vp]),
     "fls_vector_features": (c_int, [c_vp, c_u64, c_vp, c_vp]),
     "fls_mixed_max_words": (c_u64, [c_u64]),
+    "fls_mixed_stats_device": (c_int, [c_vp, c_u64, c_vp, c_vp, c_vp, c_vp, c_vp]),
+    "fls_mixed_resolve_device": (c_int, [c_u64, c_vp, c_vp, ctypes.c_float, c_u32, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp]),
     "fls_mixed_plan_device": (c_int, [c_vp, c_u64, c_vp, c_vp, ctypes.c_float, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp]),
     "fls_trial_workspace_bytes": (c_u64, [c_u64]),
     "fls_mixed_encode_trial": (c_int, [c_vp, c_u64, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp]),

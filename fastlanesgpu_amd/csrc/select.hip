@@ -24,6 +24,7 @@
 #include "fls_rng.hpp"
 #include "fls_rows.hpp"
 #include "fls_runtime.hpp"
+#include "fls_scan.hpp"
 #include "fls_select.hpp"
 
 namespace fls {
@@ -130,32 +131,43 @@ __global__ __launch_bounds__(kBlock) void exhaustive_kernel(const uint32_t* __re
 // reads 1/8 of the vector's lines and includes its first and last rows (a
 // sorted vector's sample spans its whole range); lane l takes rows
 // 32*((l/8)*31/3) + 4*(l%8) + 0..3
-// the 16 features of one vector from its sample (4 rows per lane)
-__device__ __forceinline__ void vector_features(const uint32_t (&s)[4], float* __restrict f) {
+// What the features are computed from: this lane's part of the sample's
+// statistics.  Differences are taken inside groups of four rows, `first` is a
+// group's first row.
+struct SampleStats {
     uint32_t orv = 0, mn = 0xffffffffu, mx = 0, dor = 0, zero = 0, nondec = 0, absmax = 0, dsum = 0, big = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        orv |= s[j];
-        mn = min(mn, s[j]);
-        mx = max(mx, s[j]);
-        if (j) {
-            const uint32_t d = s[j] - s[j - 1];
-            const uint32_t a = (int32_t)d < 0 ? 0u - d : d;
-            dor |= d;
-            zero += d == 0;
-            nondec += s[j] >= s[j - 1];
-            absmax = max(absmax, a);
-            dsum += min(a, 0xffffu);
-            big += a >= 256u;
-        }
+    uint32_t all_eq = 0, first_min = 0xffffffffu, first_max = 0, wsum = 0;
+    __device__ __forceinline__ void value(uint32_t y) {
+        orv |= y;
+        mn = min(mn, y);
+        mx = max(mx, y);
+        wsum += wid(y);
     }
-    const uint32_t all_eq = (s[0] == s[1]) & (s[1] == s[2]) & (s[2] == s[3]);
-    const uint32_t g_or = h_or(orv), g_min = h_min(mn), g_max = h_max(mx), g_dor = h_or(dor);
-    const uint32_t g_zero = h_sum(zero), g_nondec = h_sum(nondec), g_abs = h_max(absmax), g_dsum = h_sum(dsum);
-    const uint32_t g_big = h_sum(big), g_eq = h_sum(all_eq);
-    const uint32_t first_min = h_min(s[0]), first_max = h_max(s[0]);
+    __device__ __forceinline__ void step(uint32_t prev, uint32_t y) {
+        const uint32_t d = y - prev;
+        const uint32_t a = (int32_t)d < 0 ? 0u - d : d;
+        dor |= d;
+        zero += d == 0;
+        nondec += y >= prev;
+        absmax = max(absmax, a);
+        dsum += min(a, 0xffffu);
+        big += a >= 256u;
+    }
+    __device__ __forceinline__ void first(uint32_t y) {
+        first_min = min(first_min, y);
+        first_max = max(first_max, y);
+    }
+};
+
+// the 16 features of one vector from its lanes' statistics; s: the lane's four
+// rows of the sample
+__device__ __forceinline__ void vector_features(const SampleStats& t, const uint32_t (&s)[4], float* __restrict f) {
+    const uint32_t g_or = h_or(t.orv), g_min = h_min(t.mn), g_max = h_max(t.mx), g_dor = h_or(t.dor);
+    const uint32_t g_zero = h_sum(t.zero), g_nondec = h_sum(t.nondec), g_abs = h_max(t.absmax);
+    const uint32_t g_dsum = h_sum(t.dsum), g_big = h_sum(t.big), g_eq = h_sum(t.all_eq);
+    const uint32_t first_min = h_min(t.first_min), first_max = h_max(t.first_max);
     const uint32_t at_min = h_sum((uint32_t)(s[0] == g_min) + (s[1] == g_min) + (s[2] == g_min) + (s[3] == g_min));
-    const uint32_t wsum = h_sum(wid(s[0]) + wid(s[1]) + wid(s[2]) + wid(s[3]));
+    const uint32_t wsum = h_sum(t.wsum);
     if (dev::lane32() == 0) {
         f[0] = wid(g_or) / 32.f;
         f[1] = wid(g_max - g_min) / 32.f;
@@ -174,6 +186,43 @@ __device__ __forceinline__ void vector_features(const uint32_t (&s)[4], float* _
         f[14] = (float)(wid(g_max - g_min) > wid(g_dor));
         f[15] = 1.0f;
     }
+}
+
+// The sample as features_kernel reads it: four consecutive rows per lane.
+__device__ __forceinline__ void sample_features(const uint32_t (&s)[4], float* __restrict f) {
+    SampleStats t;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        t.value(s[j]);
+        if (j) t.step(s[j - 1], s[j]);
+    }
+    t.first(s[0]);
+    t.all_eq = (s[0] == s[1]) & (s[1] == s[2]) & (s[2] == s[3]);
+    vector_features(t, s, f);
+}
+
+// The same from the coalesced layout: the sampled lines are rows 0, 10, 20 and
+// 31 of the layout, a group of four rows is a lane quad.
+__device__ __forceinline__ void line_features(const uint32_t (&x)[32], float* __restrict f) {
+    const uint32_t s[4] = {x[0], x[10], x[20], x[31]};
+    const bool head = (threadIdx.x & 3u) == 0;
+    SampleStats t;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t up = dpp<kWaveShr1>(s[j]);
+        t.value(s[j]);
+        uint32_t same = 1;
+        if (head) {
+            t.first(s[j]);
+        } else {
+            t.step(up, s[j]);
+            same = s[j] == up;
+        }
+        same &= dpp<kQuadXor1>(same);
+        same &= dpp<kQuadXor2>(same);
+        t.all_eq += head ? same : 0u;
+    }
+    vector_features(t, s, f);
 }
 
 // A half-wave takes kFeatVec consecutive vectors and issues all their sample
@@ -196,7 +245,7 @@ __global__ __launch_bounds__(kBlock) void features_kernel(const uint32_t* __rest
     }
 #pragma unroll
     for (int k = 0; k < kFeatVec; ++k)
-        if (v0 + k < n_vec) vector_features(s[k], feat + 16 * (v0 + k));
+        if (v0 + k < n_vec) sample_features(s[k], feat + 16 * (v0 + k));
 }
 
 // plan the chosen encoding of every vector: words and metadata.  With a
@@ -231,6 +280,57 @@ __global__ __launch_bounds__(kBlock) void mixed_plan_kernel(const uint32_t* __re
         aux[v] = enc_aux(enc, st);
         if (fallback) cls[v] = (uint8_t)mix_class(enc, w);
     }
+}
+
+// One pass over the input for everything that is decided before packing: the
+// statistics of all four encodings and, with feat, the features.  They wait in
+// the outputs of the plan: vmeta[v] = w_bp | w_for << 8 | w_delta << 16, aux[v]
+// in its RLE form (smallest value, run count, index width).  Bound by the
+// read: 85 us for 120M values with the features, where features, then the chosen
+// encoding's statistics read them one and an eighth times (35 + 72 us); 39 us
+// for 60M without, where the exhaustive search, then the plan read them twice
+// (40 + 38).
+template <bool FEAT>
+__global__ __launch_bounds__(kBlock) void stats_kernel(const uint32_t* __restrict in, uint64_t n, uint64_t n_vec,
+                                                       float* __restrict feat, uint64_t* __restrict widths,
+                                                       uint64_t* __restrict aux, ScanState state) {
+    scan_clear(state);
+    const uint64_t v = (uint64_t)blockIdx.x * kVecPerBlock + (threadIdx.x >> 5);
+    if (v >= n_vec) return;
+    uint32_t x[32];
+    load_rows(in, n, v, x);
+    const VecStats st = analyze_rows<true>(x, 0);
+    if (dev::lane32() == 0) {
+        widths[v] = st.w_bp | st.w_for << 8 | st.w_delta << 16;
+        aux[v] = enc_aux(MIX_RLE, st);
+    }
+    if constexpr (FEAT) line_features(x, feat + 16 * v);
+}
+
+// Statistics to plan: each vector's class (cls) or, with exhaustive or below
+// conf_min, its smallest encoding, whose class is written back; then offsets.
+__global__ __launch_bounds__(kScanBlock) void resolve_kernel(uint64_t n_vec, uint8_t* __restrict cls,
+                                                             const float* __restrict conf, float conf_min,
+                                                             uint32_t exhaustive, fls_vmeta* vmeta, uint64_t* aux,
+                                                             uint64_t* __restrict total,
+                                                             uint32_t* __restrict fallbacks,
+                                                             unsigned long long* __restrict state) {
+    scan_vectors(
+        [&](uint64_t v, uint32_t& words, uint32_t& encw) {
+            const uint64_t ax = aux[v];
+            const uint32_t wd = (uint32_t)vmeta[v];
+            const VecStats st{wd & 255u, (uint32_t)ax, (wd >> 8) & 255u, (wd >> 16) & 255u,
+                              (uint32_t)(ax >> 32) & 0xffffu, (uint32_t)(ax >> 48)};
+            const bool fallback = conf && conf[v] < conf_min;
+            const bool best = exhaustive || fallback;
+            const uint32_t enc = best ? best_encoding(st) : mix_class_enc(cls[v]);
+            const uint32_t w = enc_width(enc, st);
+            words = (mix_bytes(enc, st) - 16u) / 4u;
+            encw = (enc << 6) | w | (fallback ? kScanFlag : 0u);
+            aux[v] = enc_aux(enc, st);
+            if (best) cls[v] = (uint8_t)mix_class(enc, w);
+        },
+        n_vec, state, vmeta, total, fallbacks);
 }
 
 // pack every vector with its planned encoding.  The vector is loaded
@@ -649,6 +749,34 @@ int fls_mixed_plan_device(const uint32_t* d_in, uint64_t n, uint8_t* d_class, co
                        n_vec, d_class, d_conf, conf_min, e.words, e.bws, d_aux, e.state);
     if (const int rc = check_launch()) return rc;
     return scan_offsets(e, n_vec, d_vmeta, d_total_words, s, d_fallbacks);
+}
+
+int fls_mixed_stats_device(const uint32_t* d_in, uint64_t n, float* d_feat, fls_vmeta* d_vmeta, uint64_t* d_aux,
+                           void* d_scratch, void* stream) {
+    using namespace fls;
+    if (n == 0) return FLS_OK;
+    FLS_RETURN_IF(!d_in || !d_vmeta || !d_aux || !d_scratch, FLS_ERR_NULL);
+    const uint64_t n_vec = ceil_div(n, 1024), blocks = ceil_div(n_vec, kVecPerBlock);
+    FLS_RETURN_IF(blocks > 0x7fffffffu, FLS_ERR_SIZE);
+    const EncodeScratch e = encode_scratch(d_scratch, n_vec);
+    auto k = d_feat ? stats_kernel<true> : stats_kernel<false>;
+    hipLaunchKernelGGL(k, dim3((uint32_t)blocks), dim3(kBlock), 0, as_stream(stream), d_in, n, n_vec, d_feat, d_vmeta,
+                       d_aux, e.state);
+    return check_launch();
+}
+
+int fls_mixed_resolve_device(uint64_t n, uint8_t* d_class, const float* d_conf, float conf_min, uint32_t exhaustive,
+                             fls_vmeta* d_vmeta, uint64_t* d_aux, uint64_t* d_total_words, uint32_t* d_fallbacks,
+                             void* d_scratch, void* stream) {
+    using namespace fls;
+    if (n == 0) return zero_u64(d_total_words, 1, as_stream(stream));
+    FLS_RETURN_IF(!d_class || !d_vmeta || !d_aux || !d_total_words || !d_scratch, FLS_ERR_NULL);
+    const uint64_t n_vec = ceil_div(n, 1024);
+    const EncodeScratch e = encode_scratch(d_scratch, n_vec);
+    hipLaunchKernelGGL(resolve_kernel, dim3(e.state.n - 1u), dim3(kScanBlock), 0, as_stream(stream), n_vec, d_class,
+                       exhaustive ? nullptr : d_conf, conf_min, exhaustive, d_vmeta, d_aux, d_total_words, d_fallbacks,
+                       e.state.p);
+    return check_launch();
 }
 
 int fls_mixed_encode_device(const uint32_t* d_in, uint64_t n, uint8_t* d_class, const float* d_conf, float conf_min,

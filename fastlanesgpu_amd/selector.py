@@ -237,6 +237,22 @@ def mixed_plan(d_in, n, ws, conf=None, conf_min=0.0, stream=None):
          dptr(ws.vmeta), dptr(ws.aux), dptr(ws.total), dptr(ws.fallbacks), dptr(ws.scratch), _stream(stream))
 
 
+def mixed_stats(d_in, n, ws, features=False, stream=None):
+    """One pass over the input: every vector's statistics (kept in ws.vmeta and
+    ws.aux for mixed_resolve) and, if asked for, its features (ws.feat)."""
+    call("fls_mixed_stats_device", dptr(d_in), n, dptr(ws.feat) if features else None, dptr(ws.vmeta), dptr(ws.aux),
+         dptr(ws.scratch), _stream(stream))
+
+
+def mixed_resolve(n, ws, conf=None, conf_min=0.0, exhaustive=False, stream=None):
+    """mixed_stats' results to the plan of the classes in ws.cls (with the
+    confidence fallback when conf is given) or of every vector's smallest
+    encoding."""
+    call("fls_mixed_resolve_device", n, dptr(ws.cls), dptr(conf), ctypes.c_float(conf_min), int(exhaustive),
+         dptr(ws.vmeta), dptr(ws.aux), dptr(ws.total), None if exhaustive else dptr(ws.fallbacks), dptr(ws.scratch),
+         _stream(stream))
+
+
 def mixed_pack(d_in, n, ws, stream=None):
     call("fls_mixed_pack_device", dptr(d_in), n, dptr(ws.vmeta), dptr(ws.aux), dptr(ws.words), _stream(stream))
 
@@ -260,9 +276,11 @@ def mixed_encode_classes(d_in, n, ws, stream=None):
 
 
 def mixed_encode_exhaustive(d_in, n, ws, stream=None):
-    """Statistics-only exhaustive choice, then plan + pack."""
-    call("fls_exhaustive_select", dptr(d_in), n, dptr(ws.cls), None, _stream(stream))
-    mixed_encode_classes(d_in, n, ws, stream)
+    """Statistics-only exhaustive choice: one pass for every encoding's
+    statistics, the smallest of each vector, pack."""
+    mixed_stats(d_in, n, ws, stream=stream)
+    mixed_resolve(n, ws, exhaustive=True, stream=stream)
+    mixed_pack(d_in, n, ws, stream)
 
 
 def trial_buffer(n):
@@ -310,14 +328,19 @@ class LearnedSelector:
 
     def choose(self, d_in, n, ws, stream=None):
         """features -> MLP -> ws.cls / ws.conf."""
-        nv = n_vectors(n)
         call("fls_vector_features", dptr(d_in), n, dptr(ws.feat), _stream(stream))
-        call("fls_mlp_forward", dptr(self.mlp.wb), dptr(ws.feat), nv, dptr(ws.cls), dptr(ws.conf), None,
+        self.classify(n, ws, stream)
+
+    def classify(self, n, ws, stream=None):
+        """The network on ws.feat -> ws.cls / ws.conf."""
+        call("fls_mlp_forward", dptr(self.mlp.wb), dptr(ws.feat), n_vectors(n), dptr(ws.cls), dptr(ws.conf), None,
              _stream(stream))
 
     def encode(self, d_in, n, ws, stream=None):
-        """The learned encode: choose, then plan (with the confidence fallback)
-        and pack.  Asynchronous; ws.column(n) reads the result."""
-        self.choose(d_in, n, ws, stream)
-        mixed_plan(d_in, n, ws, conf=ws.conf, conf_min=self.conf_min, stream=stream)
+        """The learned encode: statistics and features in one pass, the
+        network's choice (ws.cls, ws.conf), the plan with the confidence
+        fallback, and the pack.  Asynchronous; ws.column(n) reads the result."""
+        mixed_stats(d_in, n, ws, features=True, stream=stream)
+        self.classify(n, ws, stream)
+        mixed_resolve(n, ws, conf=ws.conf, conf_min=self.conf_min, stream=stream)
         mixed_pack(d_in, n, ws, stream)

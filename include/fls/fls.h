@@ -513,6 +513,18 @@ int fls_mixed_plan_device(const uint32_t* d_in, uint64_t n, uint8_t* d_class, co
                           void* d_scratch, void* stream);
 int fls_mixed_pack_device(const uint32_t* d_in, uint64_t n, const fls_vmeta* d_vmeta, const uint64_t* d_aux,
                           uint32_t* d_out, void* stream);
+/* The same plan in two steps around the choice, reading the input once for
+ * everything that precedes the pack.  stats: every vector's statistics, left in
+ * d_vmeta and d_aux for resolve, and with d_feat (else NULL) the features of
+ * fls_vector_features.  resolve: from d_class and d_conf / conf_min /
+ * d_fallbacks as above, or with exhaustive != 0 every vector's smallest
+ * encoding (d_class is written, d_conf not read), to the d_vmeta, d_aux and
+ * *d_total_words of the plan.  Both take the same scratch, unused in between. */
+int fls_mixed_stats_device(const uint32_t* d_in, uint64_t n, float* d_feat, fls_vmeta* d_vmeta, uint64_t* d_aux,
+                           void* d_scratch, void* stream);
+int fls_mixed_resolve_device(uint64_t n, uint8_t* d_class, const float* d_conf, float conf_min, uint32_t exhaustive,
+                             fls_vmeta* d_vmeta, uint64_t* d_aux, uint64_t* d_total_words, uint32_t* d_fallbacks,
+                             void* d_scratch, void* stream);
 /* The same mixed column in one pass over the input: plan, offsets (a
  * decoupled look-back over the blocks, in the scratch of
  * fls_encode_scratch_bytes(n), cleared by a small fill launch first) and pack

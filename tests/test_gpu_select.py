@@ -201,6 +201,40 @@ def test_trial_equals_exhaustive(k):
     check_against_oracle(b, x, pb[4])
 
 
+def test_stats_and_resolve_equal_features_and_plan():
+    """One pass for statistics and features, then resolve: the features of
+    fls_vector_features bit for bit and the plan of fls_mixed_plan_device, for
+    given classes with a fallback and for the exhaustive choice."""
+    torch = torch_cuda()
+    rng = np.random.default_rng(31)
+    extra = [("wrap", rng.integers(0, 1 << 32, 3 * 1024 + 5, dtype=np.uint64).astype(np.uint32)),
+             ("quads", np.repeat(rng.integers(0, 1 << 32, 600, dtype=np.uint64), 4).astype(np.uint32)),
+             ("one", np.array([7], np.uint32))]
+    for name, x in mixed_inputs() + extra:
+        n, nv, d = x.size, sel.n_vectors(x.size), to_dev(x)
+        classes = torch.from_numpy(rng.integers(0, 40, nv).astype(np.uint8)).cuda()
+        conf = torch.from_numpy(rng.random(nv).astype(np.float32)).cuda()
+        a, b = sel.MixedWorkspace(n), sel.MixedWorkspace(n)
+        for ws in (a, b):
+            ws.cls[:nv] = classes
+        sel.mixed_plan(d, n, a, conf=conf, conf_min=0.4)
+        sel.mixed_stats(d, n, b, features=True)
+        assert torch.equal(b.feat[:nv], sel.vector_features(d, n)[:nv]), name
+        sel.mixed_resolve(n, b, conf=conf, conf_min=0.4)
+        assert int(a.fallbacks.item()) == int(b.fallbacks.item()) == int((conf < 0.4).sum()), name
+        for k in ("vmeta", "aux", "cls"):
+            assert torch.equal(getattr(a, k)[:nv], getattr(b, k)[:nv]), (name, k)
+        assert int(a.total.item()) == int(b.total.item()), name
+        best, _ = sel.exhaustive_select(d, n)
+        a.cls[:nv] = best[:nv]
+        sel.mixed_plan(d, n, a)
+        sel.mixed_stats(d, n, b)
+        sel.mixed_resolve(n, b, exhaustive=True)
+        for k in ("vmeta", "aux", "cls"):
+            assert torch.equal(getattr(a, k)[:nv], getattr(b, k)[:nv]), (name, k)
+        assert int(a.total.item()) == int(b.total.item()), name
+
+
 def test_confidence_fallback():
     torch = torch_cuda()
     _, x = cases()[0]
