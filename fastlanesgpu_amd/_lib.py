@@ -102,16 +102,12 @@ def load(path=None):
     return lib
 
 
-def check(lib, name, status):
-    if status != 0:
-        raise FlsError(name, status, lib)
-
-
 def call(name, *args):
     """Call a status-returning C-ABI function and raise FlsError on failure."""
-    lib = load()
+    lib = _lib or load()
     st = getattr(lib, name)(*args)
-    check(lib, name, st)
+    if st != 0:
+        raise FlsError(name, st, lib)
     return st
 
 

@@ -490,13 +490,9 @@ __global__ __launch_bounds__(1024) void q21_any_kernel(const Q21Dev a) {
 
 template <typename Kernel>
 int launch_resident_q21(Kernel k, int block, size_t lds, const Q21Dev& a, hipStream_t s) {
-    int per_cu = 0;
-    FLS_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, block, lds));
-    if (per_cu < 1) per_cu = 1;
-    uint32_t cus = 0;
-    int st = device_cus(&cus);
+    uint32_t grid = 0;
+    const int st = resident_grid_of(reinterpret_cast<const void*>(k), block, lds, a.n_groups, &grid);
     if (st) return st;
-    const uint32_t grid = balanced_grid((uint64_t)cus * per_cu, a.n_groups);
     hipLaunchKernelGGL(k, dim3(grid), dim3(block), lds, s, a);
     return check_launch();
 }
