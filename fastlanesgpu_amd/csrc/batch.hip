@@ -494,8 +494,11 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) v
     }
 }
 
-__global__ void zero_u32_kernel(uint32_t* __restrict p, uint32_t n) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0u;
+// The counters and the tile queue of a run, in one launch.
+__global__ void zero_batch_kernel(uint64_t* __restrict counts, uint32_t n, uint32_t* __restrict queue) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) counts[i] = 0u;
+    if (i == 0) *queue = 0u;
 }
 
 // ------------------------------------------------------------ generation
@@ -707,8 +710,9 @@ int run_batch(fls_batch* b, const fls_tune* t, uint64_t* d_counts, hipStream_t s
     int st;
     if ((st = check_tune(t)) != FLS_OK) return st;
     if ((st = set_tiles(b, *t, only)) != FLS_OK) return st;
-    if ((st = zero_u64(d_counts, b->segs.size(), s)) != FLS_OK) return st;
-    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, s, b->d_queue, 1u);
+    const uint32_t n_seg = (uint32_t)b->segs.size();
+    hipLaunchKernelGGL(zero_batch_kernel, dim3(n_seg / 256u + 1u), dim3(256), 0, s, d_counts, n_seg, b->d_queue);
+    if ((st = check_launch()) != FLS_OK) return st;
     const bool dynamic = t->schedule == FLS_SCHED_DYNAMIC;
     uint32_t grid = 0;
     if (t->block_threads == 512) {

@@ -32,6 +32,7 @@
 #include "fls_fastdiv.hpp"
 #include "fls_group_hash.hpp"
 #include "fls_runtime.hpp"
+#include "fls_stage.hpp"
 
 namespace fls {
 namespace {
@@ -296,10 +297,10 @@ __global__ __launch_bounds__(1024) void q21_compact_kernel(const Q21Dev a) {
         uint32_t* s = stage;
         uint32_t* p = stage + a.supp_words + 1u;
         uint16_t* y = reinterpret_cast<uint16_t*>(p + a.part_words + 1u);
-        for (uint32_t i = threadIdx.x; i <= a.supp_words; i += blockDim.x) s[i] = i < a.supp_words ? supp_bm[i] : 0u;
-        for (uint32_t i = threadIdx.x; i <= a.part_words; i += blockDim.x) p[i] = i < a.part_words ? part_bm[i] : 0u;
-        if constexpr (!PHT)
-            for (uint32_t i = threadIdx.x; i < a.n_date; i += blockDim.x) y[i] = a.year[i];
+        stage_words(s, supp_bm, a.supp_words);
+        stage_words(p, part_bm, a.part_words);
+        if (threadIdx.x == 0) s[a.supp_words] = p[a.part_words] = 0u;
+        if constexpr (!PHT) stage_bytes(reinterpret_cast<uint8_t*>(y), reinterpret_cast<const uint8_t*>(a.year), 2u * a.n_date);
         supp_bm = s;
         part_bm = p;
         year_tab = y;
@@ -437,9 +438,9 @@ __global__ __launch_bounds__(1024) void q21_any_kernel(const Q21Dev a) {
         uint32_t* s = lds;
         uint32_t* p = lds + a.supp_words;
         uint16_t* y = reinterpret_cast<uint16_t*>(p + a.part_words);
-        for (uint32_t i = threadIdx.x; i < a.supp_words; i += blockDim.x) s[i] = a.supp_bm[i];
-        for (uint32_t i = threadIdx.x; i < a.part_words; i += blockDim.x) p[i] = a.part_bm[i];
-        for (uint32_t i = threadIdx.x; i < a.n_date; i += blockDim.x) y[i] = a.year[i];
+        stage_words(s, a.supp_bm, a.supp_words);
+        stage_words(p, a.part_bm, a.part_words);
+        stage_bytes(reinterpret_cast<uint8_t*>(y), reinterpret_cast<const uint8_t*>(a.year), 2u * a.n_date);
         __syncthreads();
         supp_bm = s;
         part_bm = p;
@@ -501,8 +502,7 @@ int launch_resident_q21(Kernel k, int block, size_t lds, const Q21Dev& a, hipStr
 // caller accumulates.
 int zero_groups(const Q21Dev& a, uint32_t flags, hipStream_t s) {
     if (flags & FLS_Q_ACCUMULATE) return FLS_OK;
-    const int st = zero_u64(reinterpret_cast<uint64_t*>(a.sums), a.n_slots, s);
-    return st ? st : zero_u64(a.counts, a.n_slots, s);
+    return zero_u64_pair(reinterpret_cast<uint64_t*>(a.sums), a.counts, a.n_slots, s);
 }
 
 // This call's set of partial tables: the device address of q21_copies (looked

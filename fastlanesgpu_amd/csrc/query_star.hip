@@ -14,6 +14,7 @@
 #include "fls_fastdiv.hpp"
 #include "fls_group_hash.hpp"
 #include "fls_runtime.hpp"
+#include "fls_stage.hpp"
 
 namespace fls {
 namespace {
@@ -148,14 +149,14 @@ __device__ __forceinline__ StarLds star_stage(const StarDev& a, uint8_t* lds) {
         uint8_t* q = lds + 12ull * a.n_slots;
         uint32_t* pb = reinterpret_cast<uint32_t*>(q);  // part bits first: 4-byte aligned
         if constexpr (PARTS) {
-            for (uint32_t i = threadIdx.x; i < a.p_words; i += blockDim.x) pb[i] = a.p_bits[i];
+            stage_words(pb, a.p_bits, a.p_words);
             q += 4ull * a.p_words;
             t.p_bits = pb;
         }
         uint8_t* s = q;
         uint8_t* y = q + a.n_supp;
-        for (uint32_t i = threadIdx.x; i < a.n_supp; i += blockDim.x) s[i] = a.s_code[i];
-        for (uint32_t i = threadIdx.x; i < a.n_date; i += blockDim.x) y[i] = a.y_code[i];
+        stage_bytes(s, a.s_code, a.n_supp);
+        stage_bytes(y, a.y_code, a.n_date);
         t.s_code = s;
         t.y_code = y;
     }
@@ -491,10 +492,13 @@ __global__ __launch_bounds__(kStarBlock) void q31_bitmap_kernel(const StarDev a)
         reinterpret_cast<uint32_t*>(lds + ((kQ31SupplierLds + a.n_supp + 1u + a.n_date + 3u) & ~(size_t)3u));
     // supplier codes staged as nation + 1 (0: not qualifying, and the
     // sentinel), so a lookup's hit bit is min(code, 1)
-    for (uint32_t i = threadIdx.x; i <= a.n_supp; i += blockDim.x)
-        s_tab[i] = i < a.n_supp ? (uint8_t)(a.s_code[i] + 1u) : (uint8_t)0;
-    for (uint32_t i = threadIdx.x; i < a.n_date; i += blockDim.x) y_tab[i] = a.y_code[i];
-    for (uint32_t i = threadIdx.x; i <= a.c_words; i += blockDim.x) c_tab[i] = i < a.c_words ? a.c_bits[i] : 0u;
+    stage_bytes(s_tab, a.s_code, a.n_supp, 1u);
+    stage_bytes(y_tab, a.y_code, a.n_date);
+    stage_words(c_tab, a.c_bits, a.c_words);
+    if (threadIdx.x == 0) {
+        s_tab[a.n_supp] = 0;
+        c_tab[a.c_words] = 0u;
+    }
     __syncthreads();
     const uint32_t tail = live_row_mask((uint32_t)(a.n_rows - (a.n_vec - 1) * 1024u), a.rev.transposed != 0);
     const uint32_t km = a.keys_min;
@@ -701,9 +705,9 @@ __global__ __launch_bounds__(kStarBlock) void q41_kernel(const StarDev a) {
         uint32_t* pb = reinterpret_cast<uint32_t*>(base + 12ull * a.n_slots);  // 4-byte aligned
         uint32_t* sb = pb + a.p_words;
         uint8_t* y = reinterpret_cast<uint8_t*>(sb + a.s_words);
-        for (uint32_t i = threadIdx.x; i < a.p_words; i += blockDim.x) pb[i] = a.p_bits[i];
-        for (uint32_t i = threadIdx.x; i < a.s_words; i += blockDim.x) sb[i] = a.s_bits[i];
-        for (uint32_t i = threadIdx.x; i < a.n_date; i += blockDim.x) y[i] = a.y_code[i];
+        stage_words(pb, a.p_bits, a.p_words);
+        stage_words(sb, a.s_bits, a.s_words);
+        stage_bytes(y, a.y_code, a.n_date);
         t.p_bits = pb;
         t.y_code = y;
         s_bits = sb;
@@ -835,9 +839,10 @@ __global__ __launch_bounds__(kStarBlock) void q41_bitmap_kernel(const StarDev a)
                          ~(size_t)7u;
     unsigned long long* sum = reinterpret_cast<unsigned long long*>(lds + g_off);
     uint32_t* cnt = reinterpret_cast<uint32_t*>(sum + a.n_slots);
-    for (uint32_t i = threadIdx.x; i <= a.s_words; i += blockDim.x) sb[i] = i < a.s_words ? a.s_bits[i] : 0u;
-    for (uint32_t i = threadIdx.x; i <= a.p_words; i += blockDim.x) pb[i] = i < a.p_words ? a.p_bits[i] : 0u;
-    for (uint32_t i = threadIdx.x; i < a.n_date; i += blockDim.x) y_tab[i] = a.y_code[i];
+    stage_words(sb, a.s_bits, a.s_words);
+    stage_words(pb, a.p_bits, a.p_words);
+    if (threadIdx.x == 0) sb[a.s_words] = pb[a.p_words] = 0u;
+    stage_bytes(y_tab, a.y_code, a.n_date);
     for (uint32_t i = threadIdx.x; i < a.n_slots; i += blockDim.x) {
         sum[i] = 0ull;
         cnt[i] = 0u;
@@ -1038,11 +1043,8 @@ int star_outputs(StarDev& a, uint32_t n_slots, int64_t* d_sums, uint64_t* d_coun
     a.slot_div = make_fastdiv(n_slots);
     a.sums = d_sums;
     a.counts = d_counts;
-    if (!(flags & FLS_Q_ACCUMULATE)) {
-        if (const int st = zero_u64(reinterpret_cast<uint64_t*>(d_sums), n_slots, s)) return st;
-        return zero_u64(d_counts, n_slots, s);
-    }
-    return FLS_OK;
+    if (flags & FLS_Q_ACCUMULATE) return FLS_OK;
+    return zero_u64_pair(reinterpret_cast<uint64_t*>(d_sums), d_counts, n_slots, s);
 }
 
 constexpr size_t kLdsBudget = 150u * 1024u;

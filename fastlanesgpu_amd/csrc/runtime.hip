@@ -24,6 +24,17 @@ int zero_u64(uint64_t* d, uint64_t n, hipStream_t stream) {
     return check_launch();
 }
 
+__global__ void zero_u64_pair_kernel(uint64_t* __restrict a, uint64_t* __restrict b, uint64_t n) {
+    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) a[i] = b[i] = 0;
+}
+
+int zero_u64_pair(uint64_t* a, uint64_t* b, uint64_t n, hipStream_t stream) {
+    if (n == 0) return FLS_OK;
+    zero_u64_pair_kernel<<<(uint32_t)ceil_div(n, 256), 256, 0, stream>>>(a, b, n);
+    return check_launch();
+}
+
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // 16-byte-per-lane streaming copy, one element per work-item over a grid of
