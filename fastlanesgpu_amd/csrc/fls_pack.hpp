@@ -6,7 +6,12 @@
 
 namespace fls {
 
-// rows (row order) -> the lane's BW words at vec_out + lane + 32*k
+// rows (row order) -> the lane's BW words at vec_out + lane + 32*k.  Stores are
+// non-temporal: an encoded column is larger than the caches, and left dirty in
+// them it is written back under the next kernel's reads (120M prices, learned:
+// 283 -> 250 us a pass; the first Q2.1 over columns just packed 222 -> 173 us,
+// Q4.1 190 -> 176, Q1.1 120 -> 111; only a 24-bit transposed pack by itself is
+// slower, 63.5 -> 67.4 us at 60M values).
 template <int BW>
 __device__ __forceinline__ void pack_lane(const uint32_t (&x)[32], uint32_t* __restrict vec_out) {
     if constexpr (BW == 0) {
@@ -24,7 +29,7 @@ __device__ __forceinline__ void pack_lane(const uint32_t (&x)[32], uint32_t* __r
         }
         uint32_t* o = vec_out + dev::lane32();
 #pragma unroll
-        for (int k = 0; k < BW; ++k) o[32 * k] = w[k];
+        for (int k = 0; k < BW; ++k) __builtin_nontemporal_store(w[k], o + 32 * k);
     }
 }
 

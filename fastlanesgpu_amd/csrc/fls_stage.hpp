@@ -4,7 +4,9 @@
 // Every block of a star probe copies 80-110 KB before its first row, so the
 // copy's latency is the kernel's: a loop of one word (or byte) per work-item
 // waits for a round trip per 4 KB (or 1 KB), while four 16-byte loads in
-// flight per work-item take two round trips in all.  XX
+// flight per work-item take two round trips in all.  At 1M rows, where little
+// else is left: Q3.1 24.2 -> 17.0 us, Q4.1 23.4 -> 20.3, Q2.1 17.3 -> 16.0 (a
+// zeroing launch less among them in the first two).
 #pragma once
 
 #include <hip/hip_runtime.h>
