@@ -45,7 +45,7 @@ struct SegDev {
 };
 
 struct TileDev {
-    uint32_t seg, v0, nv, pad;
+    uint32_t seg, v0, nv, cost;
 };
 
 // ------------------------------------------------------------ range counts
@@ -110,6 +110,50 @@ struct SwarRange {
     }
 };
 
+// Other widths are compared where they lie: with the field moved to the top of
+// a word the bits below it cannot change an order against a bound whose low
+// bits are 0 (or a closed upper bound's are 1), so a row is one shift-add (or,
+// across a word boundary, a funnel shift and an add), a compare and a carry,
+// with no mask.
+//
+// The fields x with (x - lo_adj) mod 2^32 <= span as one interval [a, b] of
+// [0, 2^BW), or as everything outside one.
+template <int BW>
+struct TopRange {
+    uint32_t minus_a, len;  // x in [a, b]: (x << (32 - BW) | junk) - (a << (32 - BW)) <= len
+    bool outside, none;
+    __device__ __forceinline__ TopRange(uint32_t lo_adj, uint32_t span) : outside(false), none(false) {
+        constexpr uint32_t m = BW >= 32 ? 0xffffffffu : (1u << (BW & 31)) - 1u;
+        const uint64_t end = (uint64_t)lo_adj + span, e2 = end - (1ull << 32);
+        const bool first = lo_adj <= m, wraps = (end >> 32) != 0;  // wrapping adds [0, end - 2^32]
+        uint32_t a = first ? lo_adj : 0u;
+        uint32_t b = first ? (end < m ? (uint32_t)end : m) : (e2 < m ? (uint32_t)e2 : m);
+        none = !first && !wraps;
+        if (first && wraps) {  // all but (e2, lo_adj), which may be empty
+            if (e2 + 1u >= lo_adj) {
+                a = 0u;
+                b = m;
+            } else {
+                outside = true;
+                a = (uint32_t)e2 + 1u;
+                b = lo_adj - 1u;
+            }
+        }
+        constexpr int sh = 32 - BW;
+        minus_a = 0u - (a << sh);
+        asm("" : "+s"(minus_a));  // an added constant to the compiler, which would turn it back into a subtraction
+        len = ((b - a) << sh) | ((1u << sh) - 1u);
+    }
+};
+
+// Field r of the lane at the top of a word, plus add.
+template <int BW>
+__device__ __forceinline__ uint32_t top_field(const uint32_t (&w)[BW], int r, uint32_t add) {
+    const int end = r * BW + BW, k = (end - 1) >> 5, e = ((end - 1) & 31) + 1;  // bits below e of word k end the field
+    if (e >= BW) return (w[k] << (32 - e)) + add;
+    return __builtin_amdgcn_alignbit(w[k], w[k > 0 ? k - 1 : 0], e) + add;
+}
+
 // BITPACK (+ FOR): vectors [0, nfull) of the segment's tile range starting at
 // v0; `lo_adj` = lo - base.  Returns this work-item's count.
 template <int BW, int VPB>
@@ -148,6 +192,7 @@ __device__ __forceinline__ uint32_t count_fixed_full(const uint32_t* __restrict 
         }
         return cnt;
     } else {
+        const TopRange<BW> rg(lo_adj, span);
         uint32_t cnt = 0;
         for (uint32_t vb = 0; vb < nfull; vb += VPB * K) {
             uint32_t w[K][BW];
@@ -163,11 +208,11 @@ __device__ __forceinline__ uint32_t count_fixed_full(const uint32_t* __restrict 
             for (int k = 0; k < K; ++k) {
                 uint32_t ck = 0;
 #pragma unroll
-                for (int r = 0; r < 32; ++r) ck += (uint32_t)(dev::extract_at<BW>(w[k], r) - lo_adj <= span);
-                cnt += live[k] ? ck : 0u;
+                for (int r = 0; r < 32; ++r) ck += (uint32_t)(top_field<BW>(w[k], r, rg.minus_a) <= rg.len);
+                cnt += live[k] ? (rg.outside ? 32u - ck : ck) : 0u;
             }
         }
-        return cnt;
+        return rg.none ? 0u : cnt;
     }
 }
 
@@ -192,6 +237,7 @@ __device__ __forceinline__ uint32_t count_delta_full(const uint32_t* __restrict 
             live[k] = idx < nfull;
             const uint64_t v = v0 + (live[k] ? idx : nfull - 1u);
             acc[k] = ldg(bases + v * 32u + l) - lo;
+            asm("" : "+v"(acc[k]));  // or the compiler subtracts lo from every row's sum instead
             if constexpr (BW > 0) load_lane_g<BW>(words + FLS_VMETA_OFFSET(ldg(vmeta + v)) + l, w[k]);
         }
 #pragma unroll
@@ -245,7 +291,7 @@ __device__ __forceinline__ uint32_t count_rle_full(const SegDev& sg, uint64_t v0
             first[k] = ldg(sg.bases + v * 32u + l);
             ibw[k] = FLS_VMETA_BW(m) ? 1u : 0u;
             const uint32_t* p = sg.words + FLS_VMETA_OFFSET(m);
-            starts[k] = ibw[k] ? ldg_nt(p + l) : 0u;
+            starts[k] = ibw[k] ? ldg(p + l) : 0u;
             vals[k] = p + 32u * ibw[k];
             nr[k] = min((uint32_t)rm.n_runs, 1024u);
             vlo[k] = lo - rm.vbase;  // run value - vbase compared against lo - vbase
@@ -289,12 +335,16 @@ __device__ __forceinline__ uint32_t count_rle_full(const SegDev& sg, uint64_t v0
             if (ibw[k] == 0) {
                 c += 32u * (F & 1u);
             } else {
-                uint32_t off = 0;
+                // the flags shifted past each run start leave the row's own
+                // flag lowest: bit extract, shift and a funnel shift that
+                // collects it, then one bit count
+                uint32_t f = F, rows = 0;
 #pragma unroll
                 for (int j = 0; j < 32; ++j) {
-                    off += (starts[k] >> dev::rsum_row(j)) & 1u;
-                    c += (F >> off) & 1u;
+                    f >>= (starts[k] >> dev::rsum_row(j)) & 1u;
+                    rows = __builtin_amdgcn_alignbit(f, rows, 1u);
                 }
+                c += __builtin_popcount(rows);
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -379,9 +429,15 @@ __device__ __forceinline__ uint32_t count_vector_slow(const SegDev& sg, uint64_t
 }
 
 // ---------------------------------------------------------------- kernel
+// Tile counters, a 128-byte line each.
+constexpr uint32_t kQueues = 8, kQueueStride = 32;
+
 // Eight waves per SIMD (64 VGPRs): the fast paths are latency-bound, and
 // measured 2.32 ms at five waves against 1.99 ms at eight over the
 // 4096-segment batch (a few loop-invariant values spill; no spill in a row loop).
+// That batch (9.3 GB) takes 1,770 us now, 5.25 TB/s, against 1,930 with one
+// queue, non-temporal loads and an instruction more per delta and RLE row;
+// 1,024 segments of up to 2^18 values in 64-vector tiles 49 against 61.
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) void batch_kernel(const SegDev* __restrict segs, const TileDev* __restrict tiles,
                                                       uint32_t n_tiles, uint64_t* __restrict counts,
@@ -393,18 +449,15 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) v
     __shared__ uint32_t s_mm[2 * WAVES];
     __shared__ uint32_t s_tile;
     const uint32_t hw = threadIdx.x >> 5, wave = threadIdx.x >> 6;
-    uint32_t iter = 0;
-    for (;;) {
-        uint32_t t;
-        if (dynamic) {
-            if (threadIdx.x == 0) s_tile = atomicAdd(queue, 1u);
-            __syncthreads();
-            t = s_tile;
-        } else {
-            t = blockIdx.x + iter * gridDim.x;
-            ++iter;
-        }
-        if (t >= n_tiles) break;  // uniform over the block
+    // Tiles past the first round come from kQueues counters (the tile numbers
+    // that are q mod kQueues from counter q), a block's own first and the others
+    // once that has run out: atomics on one address complete 5 ns apart, which
+    // for the thousands of blocks that start together is the length of a tile.
+    // (Drawn before the tile in hand is counted, the next ticket came no sooner
+    // and left blocks holding work at the end: 1,947 against 1,925 us.)
+    uint32_t t = blockIdx.x, own = blockIdx.x % kQueues;
+    auto draw = [&] { return gridDim.x + own + kQueues * atomicAdd(queue + kQueueStride * own, 1u); };
+    while (t < n_tiles) {  // uniform over the block
         const TileDev tile = tiles[t];
         const SegDev sg = segs[tile.seg];
         const uint32_t lo = sg.lo, span = sg.hi - sg.lo;
@@ -489,16 +542,26 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) v
 #pragma unroll
             for (int w = 0; w < WAVES; ++w) total += s_part[w];
             if (total) atomicAdd((unsigned long long*)&counts[tile.seg], (unsigned long long)total);
+            uint32_t next = t + gridDim.x;
+            if (dynamic) {
+                next = draw();
+                for (uint32_t k = 1; next >= n_tiles && k < kQueues; ++k) {
+                    own = (own + 1u) % kQueues;
+                    next = draw();
+                }
+            }
+            s_tile = next;
         }
-        __syncthreads();  // s_part / s_mm / s_tile / flags are rewritten next iteration
+        __syncthreads();  // s_part / s_mm / flags are rewritten next iteration
+        t = __builtin_amdgcn_readfirstlane(s_tile);
     }
 }
 
-// The counters and the tile queue of a run, in one launch.
+// The counters and the tile queues of a run, in one launch.
 __global__ void zero_batch_kernel(uint64_t* __restrict counts, uint32_t n, uint32_t* __restrict queue) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) counts[i] = 0u;
-    if (i == 0) *queue = 0u;
+    if (i < kQueues) queue[kQueueStride * i] = 0u;
 }
 
 // ------------------------------------------------------------ generation
@@ -611,6 +674,9 @@ struct fls_batch {
     int tile_filter = -2;
     fls::TileDev* d_tiles = nullptr;
     uint32_t n_tiles = 0;
+    // and, for launches of one segment each, in segment order
+    uint32_t seg_tile_vectors = 0, seg_class_tiles = 0;
+    fls::TileDev* d_seg_tiles = nullptr;
     std::vector<uint32_t> seg_tile_off, seg_tile_cnt;
     uint32_t* d_queue = nullptr;
     // graph
@@ -640,34 +706,105 @@ uint32_t class_tile(const fls_tune& t, uint32_t cls) {
     return nib ? (1u << nib) : t.tile_vectors;
 }
 
-// Cut the segments into tiles (only those of class `only`, when >= 0) and
-// upload the tile list, unless the current one already is that tiling.
+// Cost of one vector of segment s in a run, in nanoseconds of a block: about 60
+// and 10 per encoded bit, RLE 150.
+uint32_t vector_cost(const fls_batch* b, uint32_t s) {
+    const fls_segment_info& i = b->info[s];
+    if (i.encoding != FLS_ENC_BITPACK && i.encoding != FLS_ENC_DELTA) return 150u;
+    const uint64_t bits = i.n_values ? 32ull * i.n_words / i.n_values : 0u;
+    return 60u + 10u * (uint32_t)(bits < 64u ? bits : 64u);
+}
+
+// Cut the segments into tiles (only those of class `only`, when >= 0), segment
+// by segment; per segment its tiles' place, if asked for.
+std::vector<TileDev> cut_tiles(const fls_batch* b, const fls_tune& t, int only, std::vector<uint32_t>* off,
+                               std::vector<uint32_t>* cnt) {
+    std::vector<TileDev> tiles;
+    size_t most = 0;
+    for (uint32_t s = 0; s < b->segs.size(); ++s)
+        most += ceil_div(ceil_div(b->segs[s].n_values, 1024), class_tile(t, seg_class(b, s)));
+    tiles.reserve(most);
+    for (uint32_t s = 0; s < b->segs.size(); ++s) {
+        const uint32_t cls = seg_class(b, s);
+        const size_t first = tiles.size();
+        if (only < 0 || (int)cls == only) {
+            const uint32_t tv = class_tile(t, cls), cost = vector_cost(b, s);
+            const uint64_t nv = ceil_div(b->segs[s].n_values, 1024);
+            for (uint64_t v0 = 0; v0 < nv; v0 += tv) {
+                const uint32_t n = (uint32_t)(nv - v0 < tv ? nv - v0 : tv);
+                const uint64_t c = (uint64_t)n * cost;
+                tiles.push_back(TileDev{s, (uint32_t)v0, n, c < 0xffffffffu ? (uint32_t)c : 0xffffffffu});
+            }
+        }
+        if (off) off->push_back((uint32_t)first);
+        if (cnt) cnt->push_back((uint32_t)(tiles.size() - first));
+    }
+    return tiles;
+}
+
+// The order in which a run takes the tiles: as they lie, but with the cheapest
+// quarter last, dearest first, so that the blocks run out of work together.
+// (4,096 segments in 256-vector tiles: 2,009 us as they lie, 1,975 with a
+// quarter or a half held back, 2,040 all sorted, which parts the tiles bound by
+// memory from those XX
+std::vector<TileDev> run_order(const std::vector<TileDev>& tiles) {
+    const size_t n = tiles.size(), hold = n / 4;
+    uint32_t top = 0, shift = 0;
+    for (const TileDev& t : tiles) top |= t.cost;
+    while ((top >> shift) > 255u) ++shift;
+    auto level = [shift](const TileDev& t) { return t.cost >> shift; };
+    size_t count[256] = {0};
+    for (const TileDev& t : tiles) ++count[level(t)];
+    uint32_t held = 0;  // levels below this are held back
+    size_t cheap = 0;
+    while (held < 256 && cheap + count[held] <= hold) cheap += count[held++];
+    size_t place[256], at = n - cheap;
+    for (uint32_t k = held; k-- > 0;) {
+        place[k] = at;
+        at += count[k];
+    }
+    std::vector<TileDev> out(n);
+    size_t next = 0;
+    for (const TileDev& t : tiles) {
+        const uint32_t k = level(t);
+        out[k < held ? place[k]++ : next++] = t;
+    }
+    return out;
+}
+
+int upload_tiles(TileDev** d, const std::vector<TileDev>& tiles) {
+    if (*d) FLS_HIP_CHECK(hipFree(*d));
+    *d = nullptr;
+    FLS_HIP_CHECK(hipMalloc((void**)d, sizeof(TileDev) * (tiles.size() ? tiles.size() : 1)));
+    if (!tiles.empty())
+        FLS_HIP_CHECK(hipMemcpy(*d, tiles.data(), sizeof(TileDev) * tiles.size(), hipMemcpyHostToDevice));
+    return FLS_OK;
+}
+
+// Upload the tile list of a run, unless the current one already is that tiling.
 int set_tiles(fls_batch* b, const fls_tune& t, int only = -1) {
     if (t.tile_vectors == 0) return FLS_ERR_ARG;
     if (b->d_tiles && b->tile_vectors == t.tile_vectors && b->class_tiles == t.class_tiles && b->tile_filter == only)
         return FLS_OK;
-    std::vector<TileDev> tiles;
-    b->seg_tile_off.assign(b->segs.size(), 0);
-    b->seg_tile_cnt.assign(b->segs.size(), 0);
-    for (uint32_t s = 0; s < b->segs.size(); ++s) {
-        const uint32_t cls = seg_class(b, s);
-        b->seg_tile_off[s] = (uint32_t)tiles.size();
-        if (only >= 0 && (int)cls != only) continue;
-        const uint32_t tv = class_tile(t, cls);
-        const uint64_t nv = ceil_div(b->segs[s].n_values, 1024);
-        for (uint64_t v0 = 0; v0 < nv; v0 += tv)
-            tiles.push_back(TileDev{s, (uint32_t)v0, (uint32_t)(nv - v0 < tv ? nv - v0 : tv), 0});
-        b->seg_tile_cnt[s] = (uint32_t)tiles.size() - b->seg_tile_off[s];
-    }
-    if (b->d_tiles) FLS_HIP_CHECK(hipFree(b->d_tiles));
-    b->d_tiles = nullptr;
-    FLS_HIP_CHECK(hipMalloc((void**)&b->d_tiles, sizeof(TileDev) * (tiles.size() ? tiles.size() : 1)));
-    if (!tiles.empty())
-        FLS_HIP_CHECK(hipMemcpy(b->d_tiles, tiles.data(), sizeof(TileDev) * tiles.size(), hipMemcpyHostToDevice));
+    const std::vector<TileDev> tiles = run_order(cut_tiles(b, t, only, nullptr, nullptr));
+    if (const int st = upload_tiles(&b->d_tiles, tiles)) return st;
     b->n_tiles = (uint32_t)tiles.size();
     b->tile_vectors = t.tile_vectors;
     b->class_tiles = t.class_tiles;
     b->tile_filter = only;
+    return FLS_OK;
+}
+
+// The same for launches of one segment each: the tiles as they lie.
+int set_seg_tiles(fls_batch* b, const fls_tune& t) {
+    if (t.tile_vectors == 0) return FLS_ERR_ARG;
+    if (b->d_seg_tiles && b->seg_tile_vectors == t.tile_vectors && b->seg_class_tiles == t.class_tiles) return FLS_OK;
+    b->seg_tile_off.clear();
+    b->seg_tile_cnt.clear();
+    const std::vector<TileDev> tiles = cut_tiles(b, t, -1, &b->seg_tile_off, &b->seg_tile_cnt);
+    if (const int st = upload_tiles(&b->d_seg_tiles, tiles)) return st;
+    b->seg_tile_vectors = t.tile_vectors;
+    b->seg_class_tiles = t.class_tiles;
     return FLS_OK;
 }
 
@@ -677,7 +814,7 @@ int upload_segs(fls_batch* b) {
     FLS_HIP_CHECK(hipMalloc((void**)&b->d_segs, sizeof(SegDev) * (b->segs.size() ? b->segs.size() : 1)));
     if (!b->segs.empty())
         FLS_HIP_CHECK(hipMemcpy(b->d_segs, b->segs.data(), sizeof(SegDev) * b->segs.size(), hipMemcpyHostToDevice));
-    if (!b->d_queue) FLS_HIP_CHECK(hipMalloc((void**)&b->d_queue, 256));
+    if (!b->d_queue) FLS_HIP_CHECK(hipMalloc((void**)&b->d_queue, 4u * kQueues * kQueueStride));
     b->n_values = 0;
     b->n_vectors = 0;
     for (const auto& s : b->segs) {
@@ -688,10 +825,10 @@ int upload_segs(fls_batch* b) {
 }
 
 template <int BLOCK>
-int launch_batch(fls_batch* b, uint64_t* d_counts, bool dynamic, uint32_t tile_off, uint32_t n_tiles, uint32_t grid,
-                 hipStream_t s) {
+int launch_batch(fls_batch* b, uint64_t* d_counts, bool dynamic, const TileDev* d_tiles, uint32_t n_tiles,
+                 uint32_t grid, hipStream_t s) {
     if (n_tiles == 0) return FLS_OK;
-    hipLaunchKernelGGL(batch_kernel<BLOCK>, dim3(grid), dim3(BLOCK), 0, s, b->d_segs, b->d_tiles + tile_off, n_tiles,
+    hipLaunchKernelGGL(batch_kernel<BLOCK>, dim3(grid), dim3(BLOCK), 0, s, b->d_segs, d_tiles, n_tiles,
                        d_counts, b->d_queue, (uint32_t)dynamic);
     return check_launch();
 }
@@ -717,10 +854,10 @@ int run_batch(fls_batch* b, const fls_tune* t, uint64_t* d_counts, hipStream_t s
     uint32_t grid = 0;
     if (t->block_threads == 512) {
         if ((st = resident_grid_of((const void*)batch_kernel<512>, 512, 0, b->n_tiles, &grid)) != FLS_OK) return st;
-        return launch_batch<512>(b, d_counts, dynamic, 0, b->n_tiles, grid, s);
+        return launch_batch<512>(b, d_counts, dynamic, b->d_tiles, b->n_tiles, grid, s);
     }
     if ((st = resident_grid_of((const void*)batch_kernel<256>, 256, 0, b->n_tiles, &grid)) != FLS_OK) return st;
-    return launch_batch<256>(b, d_counts, dynamic, 0, b->n_tiles, grid, s);
+    return launch_batch<256>(b, d_counts, dynamic, b->d_tiles, b->n_tiles, grid, s);
 }
 
 // ---------------------------------------------------------------- autotune
@@ -1004,14 +1141,15 @@ int fls_batch_run_per_segment(fls_batch* b, const fls_tune* tune, uint64_t* d_co
     if (!b || !d_counts) return FLS_ERR_NULL;
     int st;
     if ((st = check_tune(tune)) != FLS_OK) return st;
-    if ((st = set_tiles(b, *tune)) != FLS_OK) return st;
+    if ((st = set_seg_tiles(b, *tune)) != FLS_OK) return st;
     hipStream_t s = as_stream(stream);
     if ((st = zero_u64(d_counts, b->segs.size(), s)) != FLS_OK) return st;
     for (uint32_t i = 0; i < b->segs.size(); ++i) {
         // one launch per segment: one block per tile of the segment
         const uint32_t nt = b->seg_tile_cnt[i];
-        st = tune->block_threads == 512 ? launch_batch<512>(b, d_counts, false, b->seg_tile_off[i], nt, nt, s)
-                                        : launch_batch<256>(b, d_counts, false, b->seg_tile_off[i], nt, nt, s);
+        const TileDev* tiles = b->d_seg_tiles + b->seg_tile_off[i];
+        st = tune->block_threads == 512 ? launch_batch<512>(b, d_counts, false, tiles, nt, nt, s)
+                                        : launch_batch<256>(b, d_counts, false, tiles, nt, nt, s);
         if (st) return st;
     }
     return FLS_OK;
@@ -1138,6 +1276,7 @@ void fls_batch_destroy(fls_batch* b) {
     if (b->graph) (void)hipGraphDestroy(b->graph);
     if (b->cap_stream) (void)hipStreamDestroy(b->cap_stream);
     if (b->d_tiles) (void)hipFree(b->d_tiles);
+    if (b->d_seg_tiles) (void)hipFree(b->d_seg_tiles);
     if (b->d_segs) (void)hipFree(b->d_segs);
     if (b->d_queue) (void)hipFree(b->d_queue);
     if (b->d_words) (void)hipFree(b->d_words);

@@ -31,10 +31,14 @@ __device__ __forceinline__ T ldg(const T* p) {
 __device__ __forceinline__ uint32_t ldg_nt(const uint32_t* p) {
     return __builtin_nontemporal_load((const __attribute__((address_space(1))) uint32_t*)p);
 }
+// Cached loads, for vectors whose words may start anywhere in a line (after an
+// RLE vector or segment): two vectors then share most lines, and a
+// non-temporal load drops a line before its other half is read (the
+// 4,096-segment batch: 1,914 us with non-temporal loads, 1,770 with these).
 template <int BW>
 __device__ __forceinline__ void load_lane_g(const uint32_t* lane_in, uint32_t (&w)[BW > 0 ? BW : 1]) {
 #pragma unroll
-    for (int k = 0; k < BW; ++k) w[k] = ldg_nt(lane_in + 32 * k);
+    for (int k = 0; k < BW; ++k) w[k] = ldg(lane_in + 32 * k);
 }
 
 struct ColDev {

@@ -240,3 +240,44 @@ def test_empty_ranges_every_encoding():
         d.fill_(-1)
         b.run_per_segment(fls.tune(tile, 256, fls.SCHED_STATIC), d)
         np.testing.assert_array_equal(counts_of(d), np.array(want, np.uint64), err_msg=f"per segment, tile {tile}")
+
+
+@pytest.mark.parametrize("bw", [3, 5, 13, 16, 17, 31, 32])
+def test_bitpack_ranges_that_wrap(bw):
+    """Frame-of-reference bases whose values wrap past 2^32 and ranges that
+    then hold a field interval, two of them, or all but one: the batched counts
+    equal numpy's lo <= x <= hi on the wrapped values."""
+    torch = T.torch_cuda()
+    rng = np.random.default_rng(bw)
+    n = 9 * 1024 + 5
+    segs, want = [], []
+    for base in (0, 1000, 2**31 + 10, 2**32 - 50):
+        field = rng.integers(0, 2**bw, n, dtype=np.uint64)
+        x = ((field + base) % 2**32).astype(np.uint32)
+        col = fls.Column(fls.ENC_BITPACK, n, fls.pack_column_device(T.to_dev(x), n, bw, base=base), bw=bw, base=base)
+        edges = [0, 1, 5, base, (base - 1) % 2**32, (base + 2**bw - 1) % 2**32, (base + 2**bw // 2) % 2**32, 2**31 + 20,
+                 2**32 - 1] + [int(v) for v in rng.integers(0, 2**32, 3, dtype=np.uint64)]
+        for lo in edges:
+            for hi in edges:
+                segs.append({"col": col, "rmeta": None, "n_values": n, "lo": lo, "hi": hi})
+                want.append(int(((x >= lo) & (x <= hi)).sum()))
+    b = fls.batch_from_segments(segs)
+    d = torch.full((len(segs),), -1, dtype=torch.int64, device="cuda")
+    b.run(fls.tune(8, 256, fls.SCHED_DYNAMIC), d)
+    np.testing.assert_array_equal(counts_of(d), np.array(want, np.uint64))
+
+
+@pytest.mark.parametrize("n_tiles", [1, 7, 2049, 9001])
+@pytest.mark.parametrize("schedule", [fls.SCHED_STATIC, fls.SCHED_DYNAMIC])
+def test_every_tile_is_taken_once(n_tiles, schedule):
+    """Fewer tiles than blocks or queues, one more than a round, and many
+    rounds: every tile counts once, run after run, in both schedules."""
+    torch = T.torch_cuda()
+    n = n_tiles * 2048
+    x = torch.arange(n, device="cuda", dtype=torch.int32) & 31
+    col = fls.Column(fls.ENC_BITPACK, n, fls.pack_column_device(x, n, 5), bw=5)
+    b = fls.batch_from_segments([{"col": col, "rmeta": None, "n_values": n, "lo": 4, "hi": 11}])
+    d = torch.full((1,), -1, dtype=torch.int64, device="cuda")
+    for _ in range(3):
+        b.run(fls.tune(2, 256, schedule), d)
+        assert int(d.item()) == n // 4
