@@ -674,6 +674,7 @@ struct fls_batch {
     int tile_filter = -2;
     fls::TileDev* d_tiles = nullptr;
     uint32_t n_tiles = 0;
+    uint64_t tile_lists = 0;  // tile lists uploaded so far: a captured graph holds the address of one
     // and, for launches of one segment each, in segment order
     uint32_t seg_tile_vectors = 0, seg_class_tiles = 0;
     fls::TileDev* d_seg_tiles = nullptr;
@@ -684,6 +685,7 @@ struct fls_batch {
     hipGraphExec_t exec = nullptr;
     hipGraph_t graph = nullptr;
     fls_tune graph_tune{};
+    uint64_t graph_tiles = 0;  // the tile list it was captured with
     uint64_t* graph_counts = nullptr;
     uint64_t n_values = 0, n_vectors = 0, encoded_bytes = 0;
     uint32_t count_by_enc[3] = {0, 0, 0};
@@ -788,6 +790,7 @@ int set_tiles(fls_batch* b, const fls_tune& t, int only = -1) {
         return FLS_OK;
     const std::vector<TileDev> tiles = run_order(cut_tiles(b, t, only, nullptr, nullptr));
     if (const int st = upload_tiles(&b->d_tiles, tiles)) return st;
+    ++b->tile_lists;
     b->n_tiles = (uint32_t)tiles.size();
     b->tile_vectors = t.tile_vectors;
     b->class_tiles = t.class_tiles;
@@ -1160,7 +1163,7 @@ int fls_batch_graph_launch(fls_batch* b, const fls_tune* tune, uint64_t* d_count
     if (!b || !d_counts) return FLS_ERR_NULL;
     int st;
     if ((st = check_tune(tune)) != FLS_OK) return st;
-    const bool same = b->exec && b->graph_counts == d_counts && b->graph_tune.tile_vectors == tune->tile_vectors &&
+    const bool same = b->exec && b->graph_tiles == b->tile_lists && b->graph_counts == d_counts && b->graph_tune.tile_vectors == tune->tile_vectors &&
                       b->graph_tune.block_threads == tune->block_threads && b->graph_tune.schedule == tune->schedule &&
                       b->graph_tune.class_tiles == tune->class_tiles;
     if (!same) {
@@ -1183,6 +1186,7 @@ int fls_batch_graph_launch(fls_batch* b, const fls_tune* tune, uint64_t* d_count
         FLS_HIP_CHECK(hipGraphInstantiate(&b->exec, g, nullptr, nullptr, 0));
         b->graph_counts = d_counts;
         b->graph_tune = *tune;
+        b->graph_tiles = b->tile_lists;
     }
     FLS_HIP_CHECK(hipGraphLaunch(b->exec, as_stream(stream)));
     return FLS_OK;

@@ -281,3 +281,23 @@ def test_every_tile_is_taken_once(n_tiles, schedule):
     for _ in range(3):
         b.run(fls.tune(2, 256, schedule), d)
         assert int(d.item()) == n // 4
+
+
+def test_graph_after_a_run_with_another_tiling():
+    """A captured graph holds its tile list's address: a plain run with another
+    tile size replaces the list, and the next launch captures anew."""
+    torch = T.torch_cuda()
+    b = fls.batch_c4(5, 24, 10, 16)
+    want, d = (torch.zeros(24, dtype=torch.int64, device="cuda") for _ in range(2))
+    small, large = (fls.tune(k, 256, fls.SCHED_DYNAMIC) for k in (4, 64))
+    b.run(small, want)
+    for _ in range(3):
+        d.fill_(-1)
+        b.graph_launch(small, d)
+        assert torch.equal(d, want)
+        d.fill_(-1)
+        b.run(large, d)
+        assert torch.equal(d, want)
+    d.fill_(-1)
+    b.graph_launch(large, d)
+    assert torch.equal(d, want)
