@@ -85,6 +85,7 @@ int to_dev_column(const fls_column& c, uint64_t n_rows, ColDev* out, bool allow_
     out->vmeta = c.vmeta;
     out->bases = c.bases;
     out->aux = c.aux;
+    out->cached = keep_cached(4u * (c.encoding == FLS_ENC_BITPACK ? n_vec * 32u * c.bw : c.n_words));
     switch (c.encoding) {
         case FLS_ENC_BITPACK:
             if (c.bw > 32) return FLS_ERR_BW;

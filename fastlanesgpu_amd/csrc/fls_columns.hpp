@@ -28,9 +28,6 @@ __device__ __forceinline__ T ldg(const T* p) {
         return t;
     }
 }
-__device__ __forceinline__ uint32_t ldg_nt(const uint32_t* p) {
-    return __builtin_nontemporal_load((const __attribute__((address_space(1))) uint32_t*)p);
-}
 // Cached loads, for vectors whose words may start anywhere in a line (after an
 // RLE vector or segment): two vectors then share most lines, and a
 // non-temporal load drops a line before its other half is read (the
@@ -47,7 +44,17 @@ struct ColDev {
     const fls_vmeta* vmeta;
     const uint32_t* bases;
     const uint64_t* aux;  // RLE: fls_rle_meta per vector; MIXED: aux per vector
+    uint32_t cached;      // decode kernels: keep the packed words in the caches (keep_cached)
 };
+
+// Whether a decode reads its packed words through the caches, by their bytes.
+// Columns that fit the 256 MB memory-side cache beside others are worth
+// keeping there (they were written or read before, and will be read again);
+// larger ones only evict each other.  Two columns unpacked in turn, not kept
+// and kept: 60M values of 11 bits (82 MB) 54.3 and 47.0 us, 18 bits (135 MB)
+// 61.2 and 56.4, 24 bits (180 MB) 68.7 and 69.8, 120M of 28 bits 144 and 152.
+// Full scans (queries) read more than that and were faster not keeping.
+inline bool keep_cached(uint64_t packed_bytes) { return packed_bytes <= 128ull << 20; }
 
 // Validate a host-side column descriptor for n_rows rows and build its device
 // view.  Fixed-width columns are bounds-checked against n_words.
@@ -226,8 +233,9 @@ __device__ __forceinline__ void decode_parts(const VecParts& q, uint32_t* __rest
 // of the run values straight from the column (a vector's run values are at
 // most 1024 packed values, so the gathers hit the cache after the first).
 // Row order: normal for BITPACK unless c.transposed, transposed otherwise.
-// RLE = false leaves the gather out, for callers that take RLE vectors apart.
-template <bool RLE = true>
+// RLE = false leaves the gather out, for callers that take RLE vectors apart;
+// CACHED keeps the packed words in the caches.
+template <bool RLE = true, bool CACHED = false>
 __device__ __forceinline__ void decode_regs(const ColDev& c, uint64_t v, uint32_t (&x)[32]) {
     const uint32_t l = dev::lane32();
     const uint32_t* p;
@@ -274,7 +282,7 @@ __device__ __forceinline__ void decode_regs(const ColDev& c, uint64_t v, uint32_
             nr = rm.n_runs < 1024u ? rm.n_runs : 1024u;
         }
     }
-    dev::unpack_device(p, x, w);
+    dev::unpack_device(p, x, w, CACHED);
     if (rsum) dev::rsum_lane(x, seed);
     if (RLE && vals) {
         const uint32_t last = nr ? nr - 1u : 0u;

@@ -102,7 +102,7 @@ constexpr uint32_t kRowPad = 33u;       // words per 32 staged rows
 // and 67.5; an all-bit-packed mixed column 71.6 against 70.2).  Half of every
 // chain at a time (64-byte pieces) took 88 us: lines have to be filled by one
 // instruction.
-template <bool ROWS, bool VEC, bool MIXED>
+template <bool ROWS, bool VEC, bool MIXED, bool CACHED>
 __global__ __launch_bounds__(kMatBlock) void materialize_kernel(const ColDev c, uint64_t n_rows, uint64_t n_vec,
                                                                 uint32_t* __restrict out) {
     constexpr bool kStage = ROWS || VEC;
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(kMatBlock) void materialize_kernel(const ColDev c, 
                             ROWS ? (uint32_t)min<uint64_t>(1024u, n_rows - v * 1024u) : 1024u, dst);
         live = false;  // done
     }
-    if (live) decode_regs<false>(c, v, x);
+    if (live) decode_regs<false, CACHED>(c, v, x);
     if constexpr (!kStage) {
         if (live) {
 #pragma unroll
@@ -253,16 +253,22 @@ __global__ __launch_bounds__(kMatBlock) void rle_kernel(const ColDev c, uint64_t
                         out + v * 1024u);
 }
 
+template <bool ROWS, bool VEC, bool MIXED>
+auto pick(const ColDev& c) {
+    return c.cached ? materialize_kernel<ROWS, VEC, MIXED, true> : materialize_kernel<ROWS, VEC, MIXED, false>;
+}
+
 template <bool ROWS>
 int launch_order(const ColDev& c, uint64_t n_rows, uint32_t* d_out, hipStream_t s) {
     const uint64_t n_vec = ceil_div(n_rows, 1024);
     const uint64_t work = ceil_div(n_vec, kMatVecs);  // a grid of every group: the grid-stride loop runs once
     FLS_RETURN_IF(work > 0x7fffffffu, FLS_ERR_SIZE);
-    // 16-byte stores where the output allows them
-    const bool vec = reinterpret_cast<uintptr_t>(d_out) % 16u == 0;
-    auto k = vec ? materialize_kernel<ROWS, true, false> : materialize_kernel<ROWS, false, false>;
-    if (c.enc == FLS_ENC_RLE) k = vec ? rle_kernel<ROWS, true> : rle_kernel<ROWS, false>;
-    if (c.enc == FLS_ENC_MIXED) k = vec ? materialize_kernel<ROWS, true, true> : materialize_kernel<ROWS, false, true>;
+    const bool vec = reinterpret_cast<uintptr_t>(d_out) % 16u == 0;  // 16-byte stores where the output allows them
+    auto k = vec ? rle_kernel<ROWS, true> : rle_kernel<ROWS, false>;
+    if (c.enc == FLS_ENC_MIXED)
+        k = vec ? pick<ROWS, true, true>(c) : pick<ROWS, false, true>(c);
+    else if (c.enc != FLS_ENC_RLE)
+        k = vec ? pick<ROWS, true, false>(c) : pick<ROWS, false, false>(c);
     hipLaunchKernelGGL(k, dim3((uint32_t)work), dim3(kMatBlock), 0, s, c, n_rows, n_vec, d_out);
     return check_launch();
 }

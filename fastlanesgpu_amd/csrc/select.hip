@@ -699,7 +699,8 @@ int fls_mixed_decode_u32(const uint32_t* d_words, const fls_vmeta* d_vmeta, cons
     using namespace fls;
     if (n_vec == 0) return FLS_OK;
     FLS_RETURN_IF(!d_words || !d_vmeta || !d_aux || !d_out, FLS_ERR_NULL);
-    const ColDev c{FLS_ENC_MIXED, 0, 0, 1, d_words, d_vmeta, nullptr, d_aux};
+    // the words' number is not known here: a quarter of the values' bytes is assumed
+    const ColDev c{FLS_ENC_MIXED, 0, 0, 1, d_words, d_vmeta, nullptr, d_aux, keep_cached(n_vec * 1024u)};
     return materialize(c, n_vec * 1024u, false, d_out, as_stream(stream));
 }
 

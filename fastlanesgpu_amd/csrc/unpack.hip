@@ -61,7 +61,7 @@ __device__ __forceinline__ void checksum_finish(unsigned long long t, uint64_t* 
 // checksum is reduced before its stores are issued: the reduction's atomics
 // return a value, and on gfx950 waiting for one also waits for the wave's
 // outstanding stores.
-template <int BW, bool WRITE, bool CHECKSUM>
+template <int BW, bool WRITE, bool CHECKSUM, bool CACHED>
 __global__ __launch_bounds__(kBlock) void unpack_global_kernel(const uint32_t* __restrict in,
                                                                uint32_t* __restrict out, uint64_t n_vec,
                                                                uint64_t n_values, uint64_t* __restrict checksum) {
@@ -69,7 +69,7 @@ __global__ __launch_bounds__(kBlock) void unpack_global_kernel(const uint32_t* _
     const uint64_t v = (uint64_t)blockIdx.x * kVecPerBlock + (threadIdx.x >> 5);
     const bool live = v < n_vec;
     uint32_t vals[32];
-    if (live) dev::unpack_lane<BW>(in + v * (32u * BW), vals);
+    if (live) dev::unpack_lane<BW>(in + v * (32u * BW), vals, CACHED);
     if constexpr (CHECKSUM) {
         // sum_r (first + 32r) * v_r with first = v*1024 + l + 1
         //   = first * S0 + 32 * S1,  S0 = sum v_r,  S1 = sum r*v_r   (mod 2^64);
@@ -146,6 +146,7 @@ __global__ __launch_bounds__(kBlock) void unpack_global_kernel(const uint32_t* _
 }
 
 // FastLanes delta decode: per-vector (offset, bw), 32 bases per vector.
+template <bool CACHED>
 __global__ __launch_bounds__(kBlock) void delta_decode_kernel(const uint32_t* __restrict words,
                                                               const fls_vmeta* __restrict vmeta,
                                                               const uint32_t* __restrict bases, uint64_t n_vec,
@@ -155,19 +156,19 @@ __global__ __launch_bounds__(kBlock) void delta_decode_kernel(const uint32_t* __
     if (v >= n_vec) return;
     const fls_vmeta m = vmeta[v];
     uint32_t vals[32];
-    dev::unpack_device(words + FLS_VMETA_OFFSET(m), vals, FLS_VMETA_BW(m));
+    dev::unpack_device(words + FLS_VMETA_OFFSET(m), vals, FLS_VMETA_BW(m), CACHED);
     dev::rsum_lane(vals, bases[v * 32u + l]);
     uint32_t* o = out + v * 1024u + l;
 #pragma unroll
     for (int r = 0; r < 32; ++r) __builtin_nontemporal_store(vals[r], o + 32 * r);
 }
 
-template <bool WRITE, bool CHECKSUM>
+template <bool WRITE, bool CHECKSUM, bool CACHED>
 struct UnpackTable {
     using Fn = void (*)(const uint32_t*, uint32_t*, uint64_t, uint64_t, uint64_t*);
     template <int... B>
     static constexpr auto make(std::integer_sequence<int, B...>) {
-        return std::array<Fn, sizeof...(B)>{&unpack_global_kernel<B, WRITE, CHECKSUM>...};
+        return std::array<Fn, sizeof...(B)>{&unpack_global_kernel<B, WRITE, CHECKSUM, CACHED>...};
     }
     static constexpr auto table = make(std::make_integer_sequence<int, 33>{});
 };
@@ -178,7 +179,8 @@ int launch_unpack(const uint32_t* in, uint32_t* out, uint64_t n_vec, uint64_t n_
     if (n_vec == 0) return FLS_OK;
     const uint64_t blocks = ceil_div(n_vec, kVecPerBlock);
     FLS_RETURN_IF(blocks > 0x7fffffffu, FLS_ERR_SIZE);
-    auto fn = UnpackTable<WRITE, CHECKSUM>::table[bw];
+    auto fn = keep_cached(n_vec * 128u * bw) ? UnpackTable<WRITE, CHECKSUM, true>::table[bw]
+                                              : UnpackTable<WRITE, CHECKSUM, false>::table[bw];
     hipLaunchKernelGGL(fn, dim3((uint32_t)blocks), dim3(kBlock), 0, stream, in, out, n_vec, n_values, checksum);
     return check_launch();
 }
@@ -212,8 +214,10 @@ int fls_delta_decode_u32(const uint32_t* d_words, const fls_vmeta* d_vmeta, cons
     FLS_RETURN_IF(!d_words || !d_vmeta || !d_bases || !d_out, FLS_ERR_NULL);
     const uint64_t blocks = fls::ceil_div(n_vec, fls::kVecPerBlock);
     FLS_RETURN_IF(blocks > 0x7fffffffu, FLS_ERR_SIZE);
-    hipLaunchKernelGGL(fls::delta_decode_kernel, dim3((uint32_t)blocks), dim3(fls::kBlock), 0,
-                       fls::as_stream(stream), d_words, d_vmeta, d_bases, n_vec, d_out);
+    // the words' number is not known here: a quarter of the values' bytes is assumed
+    auto k = fls::keep_cached(n_vec * 1024u) ? fls::delta_decode_kernel<true> : fls::delta_decode_kernel<false>;
+    hipLaunchKernelGGL(k, dim3((uint32_t)blocks), dim3(fls::kBlock), 0, fls::as_stream(stream), d_words, d_vmeta,
+                       d_bases, n_vec, d_out);
     return fls::check_launch();
 }
 

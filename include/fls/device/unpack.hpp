@@ -75,11 +75,16 @@ __device__ __forceinline__ void extract_rows(const uint32_t (&w)[BW > 0 ? BW : 1
 }
 
 // Load the BW words of one lane: `lane_in` points at word 0 of the lane
-// (vector base + lane).  Word k sits 32*k words further.
+// (vector base + lane).  Word k sits 32*k words further.  The words are read
+// past the caches, or with `cached` through them.
 template <int BW>
-__device__ __forceinline__ void load_lane(const uint32_t* __restrict lane_in, uint32_t (&w)[BW > 0 ? BW : 1]) {
+__device__ __forceinline__ void load_lane(const uint32_t* __restrict lane_in, uint32_t (&w)[BW > 0 ? BW : 1],
+                                          bool cached = false) {
     if constexpr (BW == 0) {
         w[0] = 0u;
+    } else if (cached) {
+#pragma unroll
+        for (int k = 0; k < BW; ++k) w[k] = lane_in[32 * k];
     } else {
 #pragma unroll
         for (int k = 0; k < BW; ++k) w[k] = __builtin_nontemporal_load(lane_in + 32 * k);
@@ -91,9 +96,10 @@ __device__ __forceinline__ void load_lane(const uint32_t* __restrict lane_in, ui
 // Counterpart of generated::unpack::cuda::fused::unpack_<bw>bw_32ow_32crw_1uf
 // (fastlanes/src/include/fls_gen/unpack/unpack_fused.cuh:7-3328).
 template <int BW>
-__device__ __forceinline__ void unpack_lane(const uint32_t* __restrict vec_in, uint32_t (&out)[32]) {
+__device__ __forceinline__ void unpack_lane(const uint32_t* __restrict vec_in, uint32_t (&out)[32],
+                                            bool cached = false) {
     uint32_t w[BW > 0 ? BW : 1];
-    load_lane<BW>(vec_in + lane32(), w);
+    load_lane<BW>(vec_in + lane32(), w, cached);
     extract_rows<BW>(w, out);
 }
 
@@ -101,12 +107,13 @@ __device__ __forceinline__ void unpack_lane(const uint32_t* __restrict vec_in, u
 // (unpack_fused.cuh:3455-3462).  Work-items of one half-wave must share bw for
 // best speed; divergent widths are correct but serialise.
 template <typename T>
-__device__ __forceinline__ void unpack_device(const T* __restrict vec_in, T (&out_t)[32], uint32_t bw) {
+__device__ __forceinline__ void unpack_device(const T* __restrict vec_in, T (&out_t)[32], uint32_t bw,
+                                              bool cached = false) {
     const uint32_t* in = reinterpret_cast<const uint32_t*>(vec_in);
     uint32_t(&out)[32] = reinterpret_cast<uint32_t(&)[32]>(out_t);
     switch (bw) {
 #define FLS_UNPACK_CASE(B) \
-    case B: unpack_lane<B>(in, out); break;
+    case B: unpack_lane<B>(in, out, cached); break;
         FLS_UNPACK_CASE(0) FLS_UNPACK_CASE(1) FLS_UNPACK_CASE(2) FLS_UNPACK_CASE(3) FLS_UNPACK_CASE(4)
         FLS_UNPACK_CASE(5) FLS_UNPACK_CASE(6) FLS_UNPACK_CASE(7) FLS_UNPACK_CASE(8) FLS_UNPACK_CASE(9)
         FLS_UNPACK_CASE(10) FLS_UNPACK_CASE(11) FLS_UNPACK_CASE(12) FLS_UNPACK_CASE(13) FLS_UNPACK_CASE(14)
