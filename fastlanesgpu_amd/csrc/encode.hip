@@ -267,7 +267,7 @@ struct PackTable {
 
 uint64_t scratch_words(uint64_t n_vec) {
     // bws[n_vec] + words[n_vec] (u32), then 8 bytes per 1,024 vectors, 256-byte
-    // aligned; the slack covers the scan's state (a ticket and a sum per 4,096)
+    // aligned: the scan's state (a sum per 1,024 vectors; its ticket is in the slack)
     const uint64_t nb = ceil_div(n_vec ? n_vec : 1, 1024);
     return ((2 * n_vec * 4 + 255) / 256 * 256 + nb * 8 + 255) / 4;
 }

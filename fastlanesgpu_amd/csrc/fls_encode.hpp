@@ -9,7 +9,7 @@ namespace fls {
 uint64_t scratch_words(uint64_t n_vec);
 
 // Vectors per block of the offset scan.
-constexpr uint32_t kScanChunk = 4096;
+constexpr uint32_t kScanChunk = 1024;
 
 // State of the offset scan (a ticket, then a published sum per block): n words
 // that the planner clears with scan_clear before the scan is launched.

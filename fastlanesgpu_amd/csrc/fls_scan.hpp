@@ -8,21 +8,23 @@
 namespace fls {
 
 // offsets[i] = sum_{k<i} words[i]; vmeta[i] = offsets[i] << 8 | bw[i];
-// *total = sum of all, in one launch.  A block takes a ticket, scans its 4,096
+// *total = sum of all, in one launch.  A block takes a ticket, scans its 1,024
 // entries and publishes their sum, then adds up the sums of the blocks before
 // it (a work-item per block, so one round trip up to 1,024 blocks).  A block
 // waits only on blocks that drew their ticket before it, and every block
 // publishes before it waits, so each wait ends.  The planner that fills words
-// clears the state (scan_clear).  Bound by those round trips: 7 us for 58,581
+// clears the state (scan_clear).  Bound by those round trips: 6 us for 58,581
 // vectors against 15 us (and two more launch gaps) as a reduction, a
-// one-block scan of the sums and an apply pass.
+// one-block scan of the sums and an apply pass.  (With 4,096 entries per block,
+// too few to keep the loads moving, 7 us; mixed columns, which resolve their
+// plan in it, 6.6 against 9.6 for 117,188 vectors.)
 constexpr int kScanBlock = 1024, kScanPer = (int)kScanChunk / kScanBlock;
 constexpr int kScanWaves = kScanBlock / 64;
 constexpr unsigned long long kScanReady = 1ull << 63;  // a published sum
 
 // Exclusive scan of one 32-bit value per work-item over the block: a DPP
 // prefix sum per wave, then the 16 wave totals read by every work-item (a
-// block's values here are vector word counts, at most 2^23 in total).
+// block's values here are vector word counts, at most 2^21 in total).
 // sh: kScanWaves words of LDS.
 __device__ __forceinline__ uint32_t block_exclusive_scan32(uint32_t x, uint32_t* sh, uint32_t& total) {
     const uint32_t incl = dev::wave_inclusive_sum(x);

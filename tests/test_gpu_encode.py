@@ -123,10 +123,10 @@ def test_encoders_at_vector_and_block_edges(n):
     np.testing.assert_array_equal(u32(out), T.transpose_vectors(padded))
 
 
-@pytest.mark.parametrize("n_vec", [4095, 4096, 4097, 2 * 4096 + 3])
+@pytest.mark.parametrize("n_vec", [1023, 1024, 1025, 2 * 4096 + 3])
 def test_offsets_over_several_scan_blocks(n_vec):
     """Offsets, total and fallback count where the scan runs in one block, in
-    exactly one, and in several (4,096 vectors each)."""
+    exactly one, and in several (1,024 vectors each)."""
     import fastlanesgpu_amd.selector as sel
     torch = T.torch_cuda()
     n = n_vec * 1024 - 5
