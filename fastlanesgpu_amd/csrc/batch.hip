@@ -748,7 +748,7 @@ std::vector<TileDev> cut_tiles(const fls_batch* b, const fls_tune& t, int only, 
 // quarter last, dearest first, so that the blocks run out of work together.
 // (4,096 segments in 256-vector tiles: 2,009 us as they lie, 1,975 with a
 // quarter or a half held back, 2,040 all sorted, which parts the tiles bound by
-// memory from those XX
+// memory from those bound by their instructions.)
 std::vector<TileDev> run_order(const std::vector<TileDev>& tiles) {
     const size_t n = tiles.size(), hold = n / 4;
     uint32_t top = 0, shift = 0;

@@ -99,7 +99,8 @@ constexpr uint32_t kRowPad = 33u;       // words per 32 staged rows
 // rle_emit, whose latency wants the waves, so the rest go half the chains, or
 // eight stored rows, at a time through a stage of that size (60M rows of mixed
 // families: 64.4 us in row order and 63.1 stored, with the whole stage 71.0
-// and 67.5; an all-bit-packed mixed column 71.6 against 70.2).  Half of every
+// and 67.5; an all-bit-packed mixed column 71.6 against 70.2; with the packed
+// words through the caches 50.7 and 49.1).  Half of every
 // chain at a time (64-byte pieces) took 88 us: lines have to be filled by one
 // instruction.
 template <bool ROWS, bool VEC, bool MIXED, bool CACHED>
@@ -234,10 +235,13 @@ __global__ __launch_bounds__(kMatBlock) void materialize_kernel(const ColDev c, 
 }
 
 // An RLE column: see fls_rle.hpp.  Bound by two dependent round trips per
-// vector, then the writes: seven to eight waves per SIMD (18.4 KB of LDS; at
-// four, 63.8 us).  60M rows of mean run 8 in row order: 55.8 us (4.8 TB/s), and
-// 89.2 through the general kernel with a gather from memory per row; stored
-// order 55.2 against 60.3 with 1,024-run stages and one word per store.
+// vector, then the writes: seven to eight waves per SIMD (18.4 KB of LDS; 60M
+// rows of mean run 8 55.8 us, and 63.8 with four waves).  67,109,641 such rows
+// in row order: 97.7 us through the general kernel with a gather from memory
+// per row, 61.3 here, and 48.3 with the index words through the caches, whose
+// lines neighbouring vectors share (6.3 TB/s).  Stored order, 60M rows: 60.3
+// with 1,024-run stages and one word per store, 55.2 here, 44.0 through the
+// caches.
 template <bool ROWS, bool VEC>
 __global__ __launch_bounds__(kMatBlock) void rle_kernel(const ColDev c, uint64_t n_rows, uint64_t n_vec,
                                                         uint32_t* __restrict out) {

@@ -470,7 +470,7 @@ __global__ __launch_bounds__(256) void mlp_grad_kernel(const uint16_t* __restric
 // block serves 16 parameters with 16 slices each: slice s adds rows
 // s, s+16, s+32, ... in order, then slice sums are added in slice order --
 // a fixed order, so the result is bit-reproducible.  Sixteen rows' loads are in
-// flight at a time (one after another: 7.3 us for 256 rows, XX this way).
+// flight at a time (one after another: 7.3 us for 256 rows, 4.5 this way).
 __global__ __launch_bounds__(256) void grad_reduce_kernel(const float* __restrict part, uint32_t n_rows,
                                                           float* __restrict grad, float* __restrict loss) {
     __shared__ float red[16][17];

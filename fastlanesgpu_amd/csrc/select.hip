@@ -476,7 +476,7 @@ __device__ __forceinline__ VecPlan plan_vector(const uint32_t (&x)[32], uint8_t 
 
 // Single-pass mixed encode: plan, offsets and pack in one launch (after a
 // fill of its look-back state).  At 120M rows it measured slower than plan +
-// scan + pack (0.20-0.24 ms against 0.15-0.20 ms per column): the plan's
+// scan + pack (0.21-0.26 ms against 0.15-0.21 ms per column): the plan's
 // work joins the pack's in blocks held to the pack's LDS occupancy, and
 // without the look-back at all (offsets at fixed slots, a timing variant) it
 // was still slower, so the encoders default to plan + pack.  Blocks take
