@@ -57,13 +57,20 @@ uint32_t balanced_grid(uint64_t max_blocks, uint64_t work) {
     return (uint32_t)ceil_div(work, rounds);
 }
 
-int resident_grid_of(const void* kernel, int block, size_t lds, uint64_t work, uint32_t* grid) {
+int resident_blocks(const void* kernel, int block, size_t lds, uint64_t* blocks) {
     int per_cu = 0;
     int st = blocks_per_cu(kernel, block, lds, &per_cu);
     if (st) return st;
     uint32_t cus = 0;
     if ((st = device_cus(&cus)) != FLS_OK) return st;
-    *grid = balanced_grid((uint64_t)cus * (uint64_t)per_cu, work);
+    *blocks = (uint64_t)cus * (uint64_t)(per_cu < 1 ? 1 : per_cu);
+    return FLS_OK;
+}
+
+int resident_grid_of(const void* kernel, int block, size_t lds, uint64_t work, uint32_t* grid) {
+    uint64_t blocks = 0;
+    if (const int st = resident_blocks(kernel, block, lds, &blocks)) return st;
+    *grid = balanced_grid(blocks, work);
     return FLS_OK;
 }
 

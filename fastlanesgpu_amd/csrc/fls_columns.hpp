@@ -77,6 +77,9 @@ int device_cus(uint32_t* cus);
 // dynamic LDS, queried once per (kernel, block, lds) and cached.
 int blocks_per_cu(const void* kernel, int block, size_t lds, int* per_cu);
 
+// Blocks of `kernel` that are resident at once on the device (at least one).
+int resident_blocks(const void* kernel, int block, size_t lds, uint64_t* blocks);
+
 // Grid of a persistent kernel: every block resident at once (CUs x the
 // kernel's occupancy), capped by the work.  A larger grid would leave the
 // excess blocks to run as a tail after the first ones retire.

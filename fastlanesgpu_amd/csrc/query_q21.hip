@@ -110,7 +110,7 @@ __global__ void q21_build_compact(const uint32_t* __restrict s_region, uint32_t 
 // ------------------------------------------------------------ probe kernels
 struct Q21Dev {
     ColDev date, supp, part, rev;
-    uint64_t n_rows, n_vec, n_groups;
+    uint64_t n_rows, n_vec, n_groups;  // n_groups: vector pairs (compact probe) or a block's vectors at a time
     // PHT path
     const uint32_t *ht_s, *ht_p, *ht_d;
     uint32_t s_len, p_len, d_len, s_min, p_min, d_min;
@@ -310,13 +310,12 @@ __global__ __launch_bounds__(1024) void q21_compact_kernel(const Q21Dev a) {
     const uint32_t tail =
         live_row_mask((uint32_t)(a.n_rows - (a.n_vec - 1) * 1024u), a.rev.transposed != 0);
     uint32_t qn = 0;  // wave-uniform; the queue carries over from step to step
-    for (uint64_t g = blockIdx.x; g < a.n_groups; g += gridDim.x) {
-        const uint64_t v = g * 32u + (threadIdx.x >> 5);
+    for (uint64_t g = first_pair(); g < a.n_groups; g += pair_step()) {
+        const uint64_t v = 2u * g + ((threadIdx.x >> 5) & 1u);
         // the whole wave stays in step (the queue flush needs every lane): a
         // half-wave past the last vector reads the last vector again (in
         // bounds, loads unconditional) and keeps no rows
         const bool vlive = v < a.n_vec;
-        if (!__any(vlive)) continue;
         const uint64_t vl = vlive ? v : a.n_vec - 1;
         LaneCol<SBW> sc;
         LaneCol<PBW> pc;
@@ -539,7 +538,12 @@ int launch_compact(Q21Dev a, bool in_lds, size_t lds, uint32_t flags, hipStream_
     const bool spread = a.n_slots <= kQ21MaxSlots;
     int st = spread ? q21_set(&a.copies) : zero_groups(a, flags, s);
     if (st) return st;
-    if ((st = launch_resident_q21(k, 1024, bytes, a, s)) != FLS_OK || !spread) return st;
+    a.n_groups = ceil_div(a.n_vec, 2);
+    uint32_t grid = 0;
+    if ((st = pair_grid(reinterpret_cast<const void*>(k), 1024, bytes, a.n_groups, kFixedPairs, &grid)) != FLS_OK)
+        return st;
+    hipLaunchKernelGGL(k, dim3(grid), dim3(1024), bytes, s, a);
+    if ((st = check_launch()) != FLS_OK || !spread) return st;
     hipLaunchKernelGGL(q21_collect_kernel, dim3((a.n_slots + 255u) / 256u), dim3(256), 0, s, a.copies, a.n_slots,
                        a.sums, a.counts, (flags & FLS_Q_ACCUMULATE) ? 1u : 0u);
     return check_launch();

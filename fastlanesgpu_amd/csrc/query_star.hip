@@ -108,7 +108,7 @@ __global__ void q41_build_kernel(fls_star_dims d, fls_q41_params p, uint8_t* __r
 
 struct StarDev {
     ColDev date, cust, supp, part, rev, cost;
-    uint64_t n_rows, n_vec, n_groups;
+    uint64_t n_rows, n_vec, n_groups;  // n_groups: vector pairs, one a wave and step
     const uint8_t *s_code, *c_code, *y_code;
     const uint32_t *p_bits, *c_bits, *s_bits;
     const uint32_t* masks;  // Q3.1: qualifying supplier nations (words 0-7) and customer nations (8-15)
@@ -302,13 +302,12 @@ __global__ __launch_bounds__(kStarBlock) void q31_kernel(const StarDev a) {
     const uint32_t tail = live_row_mask((uint32_t)(a.n_rows - (a.n_vec - 1) * 1024u), a.rev.transposed != 0);
     const uint32_t km = a.keys_min;
     uint32_t qn = 0;  // wave-uniform; the queue carries over from step to step
-    for (uint64_t g = blockIdx.x; g < a.n_groups; g += gridDim.x) {
-        const uint64_t v = g * kStarVecs + (threadIdx.x >> 5);
+    for (uint64_t g = first_pair(); g < a.n_groups; g += pair_step()) {
+        const uint64_t v = 2u * g + ((threadIdx.x >> 5) & 1u);
         // the whole wave stays in step (the queue flush needs every lane): a
         // half-wave past the last vector reads the last vector again (in
         // bounds) and keeps no rows
         const bool vlive = v < a.n_vec;
-        if (!__any(vlive)) continue;
         const uint64_t vl = vlive ? v : a.n_vec - 1;
         LaneCol<SBW> sc;
         LaneCol<CBW> cc;
@@ -504,15 +503,14 @@ __global__ __launch_bounds__(kStarBlock) void q31_bitmap_kernel(const StarDev a)
     const uint32_t km = a.keys_min;
     const uint32_t d_s = a.supp.base - km, d_c = a.cust.base - km;
     uint32_t qn = 0;  // wave-uniform; the queue carries over from step to step
-    for (uint64_t g = blockIdx.x; g < a.n_groups; g += gridDim.x) {
-        const uint64_t v = g * kStarVecs + (threadIdx.x >> 5);
+    for (uint64_t g = first_pair(); g < a.n_groups; g += pair_step()) {
+        const uint64_t v = 2u * g + ((threadIdx.x >> 5) & 1u);
         // the whole wave stays in step (the queue flush needs every lane): a
-        // half-wave past the last vector reads the group's first vector (in
-        // bounds: the group has a live vector) and keeps no rows
+        // half-wave past the last vector reads the pair's first vector (always
+        // live) and keeps no rows
         const bool vlive = v < a.n_vec;
-        if (!__any(vlive)) continue;
-        const uint64_t g0 = g * kStarVecs;
-        const uint32_t slot = vlive ? (threadIdx.x >> 5) : 0u;
+        const uint64_t g0 = 2u * g;
+        const uint32_t slot = vlive ? (threadIdx.x >> 5) & 1u : 0u;
         LaneCol<SBW> sc;
         LaneCol<CBW> cc;
         LaneCol<DBW> dc;
@@ -617,8 +615,9 @@ __global__ __launch_bounds__(kStarBlock) void q31_any_kernel(const StarDev a) {
     const StarLds t = star_stage<USE_LDS, false>(a, lds);
     const uint32_t tail = live_row_mask((uint32_t)(a.n_rows - (a.n_vec - 1) * 1024u), a.rev.transposed != 0);
     const uint32_t km = a.keys_min;
-    for (uint64_t g = blockIdx.x; g < a.n_groups; g += gridDim.x) {
-        const uint64_t v = g * kStarVecs + (threadIdx.x >> 5);
+    const PairRange mine = block_pairs(a.n_groups);
+    for (uint64_t g = mine.first; g < mine.end; g += mine.step) {
+        const uint64_t v = 2u * g + ((threadIdx.x >> 5) & 1u);
         if (v >= a.n_vec) continue;
         RegCol col;
         uint32_t m = (v == a.n_vec - 1) ? tail : 0xFFFFFFFFu;
@@ -716,13 +715,12 @@ __global__ __launch_bounds__(kStarBlock) void q41_kernel(const StarDev a) {
     const uint32_t tail = live_row_mask((uint32_t)(a.n_rows - (a.n_vec - 1) * 1024u), a.rev.transposed != 0);
     const uint32_t km = a.keys_min;
     uint32_t qn = 0;  // wave-uniform; the queue carries over from step to step
-    for (uint64_t g = blockIdx.x; g < a.n_groups; g += gridDim.x) {
-        const uint64_t v = g * kStarVecs + (threadIdx.x >> 5);
+    for (uint64_t g = first_pair(); g < a.n_groups; g += pair_step()) {
+        const uint64_t v = 2u * g + ((threadIdx.x >> 5) & 1u);
         // the whole wave stays in step (the queue flush needs every lane): a
         // half-wave past the last vector reads the last vector again (in
         // bounds) and keeps no rows
         const bool vlive = v < a.n_vec;
-        if (!__any(vlive)) continue;
         const uint64_t vl = vlive ? v : a.n_vec - 1;
         uint32_t m = 0;
         {
@@ -852,15 +850,14 @@ __global__ __launch_bounds__(kStarBlock) void q41_bitmap_kernel(const StarDev a)
     const uint32_t km = a.keys_min;
     const uint32_t d_s = a.supp.base - km, d_p = a.part.base - km;
     uint32_t qn = 0;  // wave-uniform; the queue carries over from step to step
-    for (uint64_t g = blockIdx.x; g < a.n_groups; g += gridDim.x) {
-        const uint64_t v = g * kStarVecs + (threadIdx.x >> 5);
+    for (uint64_t g = first_pair(); g < a.n_groups; g += pair_step()) {
+        const uint64_t v = 2u * g + ((threadIdx.x >> 5) & 1u);
         // the whole wave stays in step (the queue flush needs every lane): a
-        // half-wave past the last vector reads the group's first vector (in
-        // bounds: the group has a live vector) and keeps no rows
+        // half-wave past the last vector reads the pair's first vector (always
+        // live) and keeps no rows
         const bool vlive = v < a.n_vec;
-        if (!__any(vlive)) continue;
-        const uint64_t g0 = g * kStarVecs;
-        const uint32_t slot = vlive ? (threadIdx.x >> 5) : 0u;
+        const uint64_t g0 = 2u * g;
+        const uint32_t slot = vlive ? (threadIdx.x >> 5) & 1u : 0u;
         uint32_t m = 0;
         {
             LaneCol<SBW> sc;
@@ -944,8 +941,9 @@ __global__ __launch_bounds__(kStarBlock) void q41_any_kernel(const StarDev a) {
     const StarLds t = star_stage<USE_LDS, true>(a, lds);
     const uint32_t tail = live_row_mask((uint32_t)(a.n_rows - (a.n_vec - 1) * 1024u), a.rev.transposed != 0);
     const uint32_t km = a.keys_min;
-    for (uint64_t g = blockIdx.x; g < a.n_groups; g += gridDim.x) {
-        const uint64_t v = g * kStarVecs + (threadIdx.x >> 5);
+    const PairRange mine = block_pairs(a.n_groups);
+    for (uint64_t g = mine.first; g < mine.end; g += mine.step) {
+        const uint64_t v = 2u * g + ((threadIdx.x >> 5) & 1u);
         if (v >= a.n_vec) continue;
         RegCol col;
         uint32_t m = (v == a.n_vec - 1) ? tail : 0xFFFFFFFFu;
@@ -985,11 +983,11 @@ __global__ __launch_bounds__(kStarBlock) void q41_any_kernel(const StarDev a) {
 }
 
 template <typename Kernel>
-int launch_star(Kernel k, size_t lds, const StarDev& a, hipStream_t s) {
+int launch_star(Kernel k, size_t lds, const StarDev& a, hipStream_t s, uint64_t per_block = kFixedPairs) {
     FLS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
                                       (int)lds));
     uint32_t grid = 0;
-    if (const int st = resident_grid_of(reinterpret_cast<const void*>(k), kStarBlock, lds, a.n_groups, &grid))
+    if (const int st = pair_grid(reinterpret_cast<const void*>(k), kStarBlock, lds, a.n_groups, per_block, &grid))
         return st;
     hipLaunchKernelGGL(k, dim3(grid), dim3(kStarBlock), lds, s, a);
     return check_launch();
@@ -1005,7 +1003,7 @@ int star_columns(StarDev& a, const fls_column* const* cols, ColDev* const* outs,
     }
     a.n_rows = n_rows;
     a.n_vec = ceil_div(n_rows, 1024);
-    a.n_groups = ceil_div(a.n_vec, kStarVecs);
+    a.n_groups = ceil_div(a.n_vec, 2);
     return FLS_OK;
 }
 
@@ -1112,7 +1110,7 @@ int fls_query_q31(const fls_column* datekey, const fls_column* custkey, const fl
     }
     const bool in_lds = staged <= kLdsBudget;
     const size_t lds = in_lds ? staged : table;
-    return in_lds ? launch_star(q31_any_kernel<true>, lds, a, s) : launch_star(q31_any_kernel<false>, lds, a, s);
+    return launch_star(in_lds ? q31_any_kernel<true> : q31_any_kernel<false>, lds, a, s, kAnyPairs);
 }
 
 int fls_q41_build(const fls_star_dims* dims, const fls_q41_params* params, void* d_workspace, uint64_t ws_bytes,
@@ -1168,7 +1166,7 @@ int fls_query_q41(const fls_column* datekey, const fls_column* custkey, const fl
     }
     const bool in_lds = staged <= kLdsBudget;
     const size_t lds = in_lds ? staged : table;
-    return in_lds ? launch_star(q41_any_kernel<true>, lds, a, s) : launch_star(q41_any_kernel<false>, lds, a, s);
+    return launch_star(in_lds ? q41_any_kernel<true> : q41_any_kernel<false>, lds, a, s, kAnyPairs);
 }
 
 }  // extern "C"

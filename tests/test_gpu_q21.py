@@ -66,6 +66,18 @@ def test_generators_match_oracle():
         np.testing.assert_array_equal(dims_d[k].cpu().numpy().view(np.uint32)[: want.size], want)
 
 
+@pytest.mark.parametrize("n_vec", [2, 3, 17, 513, 8195])
+def test_vector_pairs_shared_among_blocks(n_vec):
+    # an odd last vector, and a second step that a few waves of every block take
+    n = n_vec * 1024 - 5
+    fact, dims = T.o_gen_c3(13, n, **SMALL)
+    fact[1] %= SMALL["n_supp"]
+    fact[2] %= SMALL["n_part"]
+    want = T.o_q21(fact, dims, n)
+    for out in run_both(fact, dims, SMALL, n, fls.encode_c3_table(*fact)):  # 12/16/20-bit keys
+        check(out, want)
+
+
 @pytest.mark.parametrize("n", [1, 700, 1024, 50_000 + 17])
 def test_q21_small(n):
     fact, dims = T.o_gen_c3(11, n, **SMALL)

@@ -88,6 +88,18 @@ def test_q41_small(n):
     check(run_q41(f, d, SMALL, n, encode(f, SMALL, FAST)), T.o_q41(f, d, n))
 
 
+@pytest.mark.parametrize("widths", [FAST, None])
+@pytest.mark.parametrize("n_vec", [2, 3, 9, 17, 513, 2049, 8195])
+def test_vector_pairs_shared_among_blocks(n_vec, widths):
+    # an odd last vector, blocks of fewer pairs than waves, a second step that a few
+    # waves of every block take (8,192 vectors are one step of 256 blocks)
+    n = n_vec * 1024 - 5
+    f, d = small_table(47, n)
+    enc = encode(f, SMALL, widths)
+    check(run_q31(f, d, SMALL, n, enc), T.o_q31(f, d, n))
+    check(run_q41(f, d, SMALL, n, enc), T.o_q41(f, d, n))
+
+
 @pytest.mark.parametrize("transposed", [False, True])
 def test_runtime_widths_and_row_order(transposed):
     # minimal key widths (9-13 bits here) take the run-time-width kernels
