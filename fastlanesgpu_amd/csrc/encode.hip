@@ -278,6 +278,7 @@ EncodeScratch encode_scratch(void* d_scratch, uint64_t n_vec) {
     e.words = e.bws + n_vec;
     e.state.p = reinterpret_cast<unsigned long long*>(static_cast<char*>(d_scratch) + (2 * n_vec * 4 + 255) / 256 * 256);
     e.state.n = (uint32_t)(ceil_div(n_vec, kScanChunk) + 1);
+    e.state.ticket = scan_ticket_word(n_vec);
     return e;
 }
 

@@ -2,6 +2,7 @@
 #pragma once
 
 #include "fls_runtime.hpp"
+#include "fls_scan_ticket.hpp"
 
 namespace fls {
 
@@ -11,18 +12,20 @@ uint64_t scratch_words(uint64_t n_vec);
 // Vectors per block of the offset scan.
 constexpr uint32_t kScanChunk = 1024;
 
-// State of the offset scan (a ticket, then a published sum per block): n words
-// that the planner clears with scan_clear before the scan is launched.
+// State of the offset scan (a ticket word, then a published sum per block): n
+// words that the planner prepares with scan_clear before the scan is launched,
+// and that one scan uses up.
 struct ScanState {
     unsigned long long* p;
     uint32_t n;
+    unsigned long long ticket;  // scan_ticket_word of the vectors
 };
 
 // Called by every work-item of a planner whose grid has at least a work-item
 // per 8 vectors and 256 in all.
 __device__ __forceinline__ void scan_clear(const ScanState& st) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < st.n) st.p[i] = 0ull;
+    if (i < st.n) st.p[i] = i ? 0ull : st.ticket;
 }
 
 // The caller's scratch, cut up: per vector its width word and word count,

@@ -13,7 +13,8 @@ namespace fls {
 // it (a work-item per block, so one round trip up to 1,024 blocks).  A block
 // waits only on blocks that drew their ticket before it, and every block
 // publishes before it waits, so each wait ends.  The planner that fills words
-// clears the state (scan_clear).  Bound by those round trips: 6 us for 58,581
+// prepares the state (scan_clear); blocks that draw no valid ticket from it
+// (scan_ticket) leave everything as it is.  Bound by those round trips: 6 us for 58,581
 // vectors against 15 us (and two more launch gaps) as a reduction, a
 // one-block scan of the sums and an apply pass.  (With 4,096 entries per block,
 // too few to keep the loads moving, 7 us; mixed columns, which resolve their
@@ -54,9 +55,10 @@ __device__ __forceinline__ void scan_vectors(Load load, uint64_t n, unsigned lon
     __shared__ uint32_t sh[kScanWaves], s_flags[kScanWaves], s_ticket;
     __shared__ uint64_t sh64[kScanWaves];
     const uint32_t t = threadIdx.x;
-    if (t == 0) s_ticket = atomicAdd(reinterpret_cast<unsigned int*>(state), 1u);
+    if (t == 0) s_ticket = scan_ticket(atomicAdd(state, 1ull), n, gridDim.x);
     __syncthreads();
     const uint32_t b = s_ticket;
+    if (b == kNoTicket) return;  // the whole block
     unsigned long long* sums = state + 1;
     const uint64_t i0 = (uint64_t)b * kScanChunk + (uint64_t)kScanPer * t;
     uint32_t w[kScanPer], bw[kScanPer], mine = 0, flags = 0;

@@ -223,6 +223,7 @@ class MixedWorkspace:
         self.feat = torch.empty((nv, N_FEATURES), dtype=torch.float32, device="cuda")
         self.conf = torch.empty(nv, dtype=torch.float32, device="cuda")
         self.trial = trial_buffer(n) if trial else None
+        self.stats_n = None  # values whose statistics mixed_stats left for mixed_resolve
 
     def column(self, n):
         """The encoded MIXED column (views of this workspace)."""
@@ -233,6 +234,7 @@ class MixedWorkspace:
 
 
 def mixed_plan(d_in, n, ws, conf=None, conf_min=0.0, stream=None):
+    ws.stats_n = None
     call("fls_mixed_plan_device", dptr(d_in), n, dptr(ws.cls), dptr(conf), ctypes.c_float(conf_min),
          dptr(ws.vmeta), dptr(ws.aux), dptr(ws.total), dptr(ws.fallbacks), dptr(ws.scratch), _stream(stream))
 
@@ -242,12 +244,17 @@ def mixed_stats(d_in, n, ws, features=False, stream=None):
     ws.aux for mixed_resolve) and, if asked for, its features (ws.feat)."""
     call("fls_mixed_stats_device", dptr(d_in), n, dptr(ws.feat) if features else None, dptr(ws.vmeta), dptr(ws.aux),
          dptr(ws.scratch), _stream(stream))
+    ws.stats_n = n
 
 
 def mixed_resolve(n, ws, conf=None, conf_min=0.0, exhaustive=False, stream=None):
     """mixed_stats' results to the plan of the classes in ws.cls (with the
     confidence fallback when conf is given) or of every vector's smallest
-    encoding."""
+    encoding.  The plan takes the statistics' place: every resolve needs a
+    mixed_stats of the same n before it."""
+    if ws.stats_n != n:
+        raise ValueError(f"no statistics of {n} values in this workspace: run mixed_stats before every mixed_resolve")
+    ws.stats_n = None
     call("fls_mixed_resolve_device", n, dptr(ws.cls), dptr(conf), ctypes.c_float(conf_min), int(exhaustive),
          dptr(ws.vmeta), dptr(ws.aux), dptr(ws.total), None if exhaustive else dptr(ws.fallbacks), dptr(ws.scratch),
          _stream(stream))
@@ -263,6 +270,7 @@ def mixed_encode(d_in, n, ws, conf=None, conf_min=0.0, stream=None):
     launch after a small fill.  The same column as plan + pack; slower at
     120M rows (see mixed_encode_classes), kept for callers that want one
     launch."""
+    ws.stats_n = None
     call("fls_mixed_encode_device", dptr(d_in), n, dptr(ws.cls), dptr(conf), ctypes.c_float(conf_min),
          dptr(ws.vmeta), dptr(ws.aux), dptr(ws.words), dptr(ws.total), dptr(ws.fallbacks), dptr(ws.scratch),
          _stream(stream))
@@ -296,6 +304,7 @@ def mixed_encode_trial(d_in, n, ws, stream=None, buf=None):
     buf = ws.trial if buf is None else buf
     if buf is None:
         raise ValueError("no trial workspace: build with trial=True or pass buf=trial_buffer(n)")
+    ws.stats_n = None
     call("fls_mixed_encode_trial", dptr(d_in), n, dptr(ws.cls), dptr(ws.vmeta), dptr(ws.aux), dptr(ws.words),
          dptr(ws.total), dptr(buf), _stream(stream))
 

@@ -519,7 +519,9 @@ int fls_mixed_pack_device(const uint32_t* d_in, uint64_t n, const fls_vmeta* d_v
  * fls_vector_features.  resolve: from d_class and d_conf / conf_min /
  * d_fallbacks as above, or with exhaustive != 0 every vector's smallest
  * encoding (d_class is written, d_conf not read), to the d_vmeta, d_aux and
- * *d_total_words of the plan.  Both take the same scratch, unused in between. */
+ * *d_total_words of the plan.  Both take the same n and scratch, unused in
+ * between.  A resolve uses the statistics up: another one takes another stats
+ * call first, and without one (or after one with another n) it changes nothing. */
 int fls_mixed_stats_device(const uint32_t* d_in, uint64_t n, float* d_feat, fls_vmeta* d_vmeta, uint64_t* d_aux,
                            void* d_scratch, void* stream);
 int fls_mixed_resolve_device(uint64_t n, uint8_t* d_class, const float* d_conf, float conf_min, uint32_t exhaustive,

@@ -235,6 +235,47 @@ def test_stats_and_resolve_equal_features_and_plan():
         assert int(a.total.item()) == int(b.total.item()), name
 
 
+@pytest.mark.parametrize("n_vec", [7, 2051])
+def test_resolve_without_statistics_changes_nothing(n_vec):
+    """A second fls_mixed_resolve_device after one stats call, one over scratch
+    that no stats call prepared, and one with another n leave the plan, the
+    classes, the counters and every byte around the scan's state as they are."""
+    torch = torch_cuda()
+    n = n_vec * 1024 - 3
+    d = sel.gen_train_vectors(41, 0, n_vec)
+    ws = sel.MixedWorkspace(n)
+    ws.fallbacks.zero_()
+    need = int(fl.load().fls_encode_scratch_bytes(n))
+    state = (8 * n_vec + 255) // 256 * 256
+    blocks = (n_vec + 1023) // 1024
+    ws.scratch = torch.full((need + 65536,), 0xA5, dtype=torch.uint8, device="cuda")
+    conf = torch.rand(n_vec, device="cuda")
+    sel.mixed_stats(d, n, ws)
+    ws.cls.zero_()
+
+    def resolve(k, scratch):
+        fl.call("fls_mixed_resolve_device", k, fl.dptr(ws.cls), fl.dptr(conf), 0.7, 0, fl.dptr(ws.vmeta),
+                fl.dptr(ws.aux), fl.dptr(ws.total), fl.dptr(ws.fallbacks), fl.dptr(scratch), fl.current_stream())
+
+    resolve(n, ws.scratch)
+    assert int(ws.fallbacks.item()) == int((conf < 0.7).sum())
+    plan = [t.clone() for t in (ws.vmeta, ws.aux, ws.cls, ws.total, ws.fallbacks)]
+    sums = ws.scratch[state + 8:state + 8 + 8 * blocks].clone()
+    assert bool((ws.scratch[state + 8 + 8 * blocks:] == 0xA5).all())
+    other = [torch.zeros_like(ws.scratch), torch.full_like(ws.scratch, 0xFF), torch.full_like(ws.scratch, 3)]
+    for k, scratch in [(n, ws.scratch), (n - 1024, ws.scratch)] + [(n, o) for o in other]:
+        before = scratch.clone()
+        resolve(k, scratch)
+        after = scratch.clone()
+        for t in (before, after):  # the ticket word counts what was drawn
+            t[state:state + 8] = 0
+            t[(8 * (n_vec - 1) + 255) // 256 * 256:][:8] = 0
+        assert torch.equal(before, after)
+    assert torch.equal(ws.scratch[state + 8:state + 8 + 8 * blocks], sums)
+    for t, want in zip((ws.vmeta, ws.aux, ws.cls, ws.total, ws.fallbacks), plan):
+        assert torch.equal(t, want)
+
+
 def test_confidence_fallback():
     torch = torch_cuda()
     _, x = cases()[0]
