@@ -64,6 +64,38 @@ def _stream(s):
     return current_stream() if s is None else s
 
 
+def _side_stream(stream):
+    """The torch stream of an explicit `stream` argument (an address or a torch
+    stream) that is not torch's current one, else None."""
+    if stream is None:
+        return None
+    raw = getattr(stream, "cuda_stream", getattr(stream, "value", stream)) or 0
+    if raw == (current_stream() or 0):
+        return None
+    import torch
+
+    return torch.cuda.ExternalStream(raw) if raw else torch.cuda.default_stream()
+
+
+def _on_stream(stream, work):
+    """work(stream), a function that allocates device tensors, puts kernels on
+    `stream` and reads a result of theirs back, with `stream` as torch's current
+    one: then the allocator's reuse of memory, the read and the kernels are in
+    one order.  The tensors it returns are also kept for the stream that was
+    current, whose work the caller is about to give them to."""
+    side = _side_stream(stream)
+    if side is None:
+        return work(_stream(stream))
+    import torch
+
+    caller = torch.cuda.current_stream()
+    with torch.cuda.stream(side):
+        out = work(side.cuda_stream)
+    for t in out:
+        t.record_stream(caller)
+    return out
+
+
 # ----------------------------------------------------------- host encoders
 def pack(values, bw):
     """generated::pack::fallback::scalar::pack for one 1024-value vector."""
@@ -657,14 +689,17 @@ def delta_encode_device(d_in, n, stream=None):
     import torch
 
     n_vec = (n + VECTOR_SIZE - 1) // VECTOR_SIZE
-    vmeta, bases = _dev_u64(n_vec), _dev_u32(32 * n_vec)
-    total = _dev_u64(1)  # the plan writes it
-    scratch = torch.empty(max(16, int(load().fls_encode_scratch_bytes(n))), dtype=torch.uint8, device="cuda")
-    stream = _stream(stream)
-    call("fls_delta_plan_device", dptr(d_in), n, dptr(vmeta), dptr(bases), dptr(total), dptr(scratch), stream)
-    words = _dev_u32(int(total.item()))
-    call("fls_delta_pack_device", dptr(d_in), n, dptr(vmeta), dptr(words), stream)
-    return words, vmeta, bases
+
+    def encode(stream):
+        vmeta, bases = _dev_u64(n_vec), _dev_u32(32 * n_vec)
+        total = _dev_u64(1)  # the plan writes it
+        scratch = torch.empty(max(16, int(load().fls_encode_scratch_bytes(n))), dtype=torch.uint8, device="cuda")
+        call("fls_delta_plan_device", dptr(d_in), n, dptr(vmeta), dptr(bases), dptr(total), dptr(scratch), stream)
+        words = _dev_u32(int(total.item()))
+        call("fls_delta_pack_device", dptr(d_in), n, dptr(vmeta), dptr(words), stream)
+        return words, vmeta, bases
+
+    return _on_stream(stream, encode)
 
 
 def rle_encode_device(d_in, n, stream=None):
@@ -673,15 +708,18 @@ def rle_encode_device(d_in, n, stream=None):
     import torch
 
     n_vec = (n + VECTOR_SIZE - 1) // VECTOR_SIZE
-    vmeta, rmeta, bases = _dev_u64(n_vec), _dev_u64(n_vec), _dev_u32(32 * n_vec)
-    total = _dev_u64(1)  # the plan writes it
-    scratch = torch.empty(max(16, int(load().fls_encode_scratch_bytes(n))), dtype=torch.uint8, device="cuda")
-    stream = _stream(stream)
-    call("fls_rle_plan_device", dptr(d_in), n, dptr(vmeta), dptr(rmeta), dptr(bases), dptr(total), dptr(scratch),
-         stream)
-    words = _dev_u32(int(total.item()))
-    call("fls_rle_pack_device", dptr(d_in), n, dptr(vmeta), dptr(rmeta), dptr(words), stream)
-    return words, vmeta, rmeta, bases
+
+    def encode(stream):
+        vmeta, rmeta, bases = _dev_u64(n_vec), _dev_u64(n_vec), _dev_u32(32 * n_vec)
+        total = _dev_u64(1)  # the plan writes it
+        scratch = torch.empty(max(16, int(load().fls_encode_scratch_bytes(n))), dtype=torch.uint8, device="cuda")
+        call("fls_rle_plan_device", dptr(d_in), n, dptr(vmeta), dptr(rmeta), dptr(bases), dptr(total), dptr(scratch),
+             stream)
+        words = _dev_u32(int(total.item()))
+        call("fls_rle_pack_device", dptr(d_in), n, dptr(vmeta), dptr(rmeta), dptr(words), stream)
+        return words, vmeta, rmeta, bases
+
+    return _on_stream(stream, encode)
 
 
 def rle_decode(d_words, d_vmeta, d_rmeta, d_bases, n_vec, d_out, stream=None):

@@ -21,7 +21,7 @@ import ctypes
 
 import numpy as np
 
-from . import ENC_MIXED, VECTOR_SIZE, Column, _dev_u32, _dev_u64, _stream, call, dptr, load
+from . import ENC_MIXED, VECTOR_SIZE, Column, _dev_u32, _dev_u64, _side_stream, _stream, call, dptr, load
 
 MIX_BITPACK, MIX_FOR, MIX_DELTA, MIX_RLE = 0, 1, 2, 3
 ENCODING_NAMES = ("bitpack", "for", "delta", "rle")
@@ -224,19 +224,48 @@ class MixedWorkspace:
         self.conf = torch.empty(nv, dtype=torch.float32, device="cuda")
         self.trial = trial_buffer(n) if trial else None
         self.stats_n = None  # values whose statistics mixed_stats left for mixed_resolve
+        self.ready = None  # where the latest encode step is waited for: see _written
 
     def column(self, n):
-        """The encoded MIXED column (views of this workspace)."""
+        """The encoded MIXED column (views of this workspace).  torch's current
+        stream waits for the encode first where that ran on another one."""
+        import torch
+
+        if isinstance(self.ready, torch.cuda.Event):
+            torch.cuda.current_stream().wait_event(self.ready)
+        else:
+            side = _side_stream(self.ready)
+            if side is not None:
+                torch.cuda.current_stream().wait_stream(side)
         total = int(self.total.item())
         nv = n_vectors(n)
         return Column(ENC_MIXED, n, self.words[:max(1, total)], vmeta=self.vmeta[:max(1, nv)],
                       aux=self.aux[:max(1, nv)], n_words=total)
 
 
+def _written(ws, stream):
+    """Note for ws.column where an encode step has just been put: an event on an
+    explicit stream, which its owner may destroy before the column is read, or
+    the address of the stream that was torch's current one."""
+    side = _side_stream(stream)
+    if side is None:
+        ws.ready = _stream(None)
+        return
+    import torch
+
+    with torch.cuda.stream(side):
+        if torch.cuda.is_current_stream_capturing():  # an event of a graph cannot be waited for outside it
+            ws.ready = None
+        else:
+            ws.ready = torch.cuda.Event()
+            ws.ready.record(side)
+
+
 def mixed_plan(d_in, n, ws, conf=None, conf_min=0.0, stream=None):
     ws.stats_n = None
     call("fls_mixed_plan_device", dptr(d_in), n, dptr(ws.cls), dptr(conf), ctypes.c_float(conf_min),
          dptr(ws.vmeta), dptr(ws.aux), dptr(ws.total), dptr(ws.fallbacks), dptr(ws.scratch), _stream(stream))
+    _written(ws, stream)
 
 
 def mixed_stats(d_in, n, ws, features=False, stream=None):
@@ -258,10 +287,12 @@ def mixed_resolve(n, ws, conf=None, conf_min=0.0, exhaustive=False, stream=None)
     call("fls_mixed_resolve_device", n, dptr(ws.cls), dptr(conf), ctypes.c_float(conf_min), int(exhaustive),
          dptr(ws.vmeta), dptr(ws.aux), dptr(ws.total), None if exhaustive else dptr(ws.fallbacks), dptr(ws.scratch),
          _stream(stream))
+    _written(ws, stream)
 
 
 def mixed_pack(d_in, n, ws, stream=None):
     call("fls_mixed_pack_device", dptr(d_in), n, dptr(ws.vmeta), dptr(ws.aux), dptr(ws.words), _stream(stream))
+    _written(ws, stream)
 
 
 def mixed_encode(d_in, n, ws, conf=None, conf_min=0.0, stream=None):
@@ -274,6 +305,7 @@ def mixed_encode(d_in, n, ws, conf=None, conf_min=0.0, stream=None):
     call("fls_mixed_encode_device", dptr(d_in), n, dptr(ws.cls), dptr(conf), ctypes.c_float(conf_min),
          dptr(ws.vmeta), dptr(ws.aux), dptr(ws.words), dptr(ws.total), dptr(ws.fallbacks), dptr(ws.scratch),
          _stream(stream))
+    _written(ws, stream)
 
 
 def mixed_encode_classes(d_in, n, ws, stream=None):
@@ -307,6 +339,7 @@ def mixed_encode_trial(d_in, n, ws, stream=None, buf=None):
     ws.stats_n = None
     call("fls_mixed_encode_trial", dptr(d_in), n, dptr(ws.cls), dptr(ws.vmeta), dptr(ws.aux), dptr(ws.words),
          dptr(ws.total), dptr(buf), _stream(stream))
+    _written(ws, stream)
 
 
 def mixed_decode(col, out=None, stream=None):

@@ -149,3 +149,53 @@ def test_offsets_over_several_scan_blocks(n_vec):
     assert int(ws.fallbacks.item()) == int((conf < 0.3).sum())
     sel.mixed_plan(d, n, ws, conf=conf, conf_min=0.3)  # the counter is added to
     assert int(ws.fallbacks.item()) == 2 * int((conf < 0.3).sum())
+
+
+@pytest.mark.parametrize("how", ["explicit", "current"])
+def test_encodes_on_another_stream(how):
+    """Encodes on a stream that has other work queued first: the size is read in
+    that stream's order (delta, RLE), the column of a workspace is not read
+    before its encode, and all equal the encodes on the default stream."""
+    import contextlib
+
+    import fastlanesgpu_amd.selector as sel
+    torch = T.torch_cuda()
+    n = 300 * 1024 + 5
+    x = sel.gen_train_vectors(17, 0, 301)[:n]
+    ws, want_ws = sel.MixedWorkspace(n, trial=True), sel.MixedWorkspace(n)
+    sel.mixed_encode_exhaustive(x, n, want_ws)
+    want = [fls.delta_encode_device(x, n), fls.rle_encode_device(x, n), want_ws.column(n)]
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    arg = {"explicit": {"stream": side.cuda_stream}, "current": {}}[how]
+    inside = contextlib.nullcontext if how == "explicit" else lambda: torch.cuda.stream(side)
+
+    def busy():  # about 30 ms of other work on the side stream
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(60_000_000)
+
+    with inside():
+        busy()
+        got = [fls.delta_encode_device(x, n, **arg)]
+        busy()
+        got.append(fls.rle_encode_device(x, n, **arg))
+    torch.cuda.synchronize()
+    for g, w in zip(got, want):
+        for a, b in zip(g, w):
+            assert torch.equal(a, b)
+    encoders = [sel.mixed_encode_exhaustive, sel.mixed_encode_classes, sel.mixed_encode, sel.mixed_encode_trial]
+    for encode in encoders:
+        ws.total.fill_(1)
+        ws.words.zero_()
+        torch.cuda.synchronize()
+        with inside():
+            busy()
+            encode(x, n, ws, **arg)
+        col = ws.column(n)
+        assert col.n_words == want[2].n_words, encode.__name__
+        for k in ("words", "vmeta", "aux"):
+            assert torch.equal(getattr(col, k), getattr(want[2], k)), (encode.__name__, k)
+    fresh = [fls.delta_encode_device(x, n, stream=0), fls.rle_encode_device(x, n, stream=torch.cuda.default_stream())]
+    for g, w in zip(fresh, want):
+        for a, b in zip(g, w):
+            assert torch.equal(a, b)
