@@ -774,12 +774,20 @@ std::vector<TileDev> run_order(const std::vector<TileDev>& tiles) {
     return out;
 }
 
+// The new list takes the old one's place when it is complete: after a failure
+// the old one is still what its key and a captured graph say it is.
 int upload_tiles(TileDev** d, const std::vector<TileDev>& tiles) {
-    if (*d) FLS_HIP_CHECK(hipFree(*d));
-    *d = nullptr;
-    FLS_HIP_CHECK(hipMalloc((void**)d, sizeof(TileDev) * (tiles.size() ? tiles.size() : 1)));
-    if (!tiles.empty())
-        FLS_HIP_CHECK(hipMemcpy(*d, tiles.data(), sizeof(TileDev) * tiles.size(), hipMemcpyHostToDevice));
+    TileDev* list = nullptr;
+    FLS_HIP_CHECK(hipMalloc((void**)&list, sizeof(TileDev) * (tiles.size() ? tiles.size() : 1)));
+    if (!tiles.empty()) {
+        const hipError_t e = hipMemcpy(list, tiles.data(), sizeof(TileDev) * tiles.size(), hipMemcpyHostToDevice);
+        if (e != hipSuccess) {
+            (void)hipFree(list);
+            return record_hip_error(e);
+        }
+    }
+    if (*d) (void)hipFree(*d);
+    *d = list;
     return FLS_OK;
 }
 
@@ -802,10 +810,11 @@ int set_tiles(fls_batch* b, const fls_tune& t, int only = -1) {
 int set_seg_tiles(fls_batch* b, const fls_tune& t) {
     if (t.tile_vectors == 0) return FLS_ERR_ARG;
     if (b->d_seg_tiles && b->seg_tile_vectors == t.tile_vectors && b->seg_class_tiles == t.class_tiles) return FLS_OK;
-    b->seg_tile_off.clear();
-    b->seg_tile_cnt.clear();
-    const std::vector<TileDev> tiles = cut_tiles(b, t, -1, &b->seg_tile_off, &b->seg_tile_cnt);
+    std::vector<uint32_t> off, cnt;
+    const std::vector<TileDev> tiles = cut_tiles(b, t, -1, &off, &cnt);
     if (const int st = upload_tiles(&b->d_seg_tiles, tiles)) return st;
+    b->seg_tile_off.swap(off);
+    b->seg_tile_cnt.swap(cnt);
     b->seg_tile_vectors = t.tile_vectors;
     b->seg_class_tiles = t.class_tiles;
     return FLS_OK;
