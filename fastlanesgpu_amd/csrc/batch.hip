@@ -429,6 +429,104 @@ __device__ __forceinline__ uint32_t count_vector_slow(const SegDev& sg, uint64_t
 }
 
 // ---------------------------------------------------------------- kernel
+template <int BLOCK>
+struct BatchLds {
+    uint32_t flags[BLOCK / 32 * kRleK * kFlagWords];
+    uint32_t part[BLOCK / 64];
+    uint32_t mm[2 * BLOCK / 64];
+};
+
+// The values in range of vectors v0 .. v0 + nv - 1 of segment sg, counted by the
+// whole block; the count is work-item 0's.
+template <int BLOCK>
+__device__ __forceinline__ uint64_t count_tile(const SegDev& sg, uint32_t v0, uint32_t nv, BatchLds<BLOCK>& s) {
+    constexpr int VPB = BLOCK / 32;
+    constexpr int WAVES = BLOCK / 64;
+    const uint32_t hw = threadIdx.x >> 5, wave = threadIdx.x >> 6;
+    const uint32_t lo = sg.lo, span = sg.hi - sg.lo;
+    const uint64_t seg_vecs = ceil_div(sg.n_values, 1024);
+    const bool has_partial = (sg.n_values & 1023u) != 0 && v0 + nv == seg_vecs;
+    const uint32_t nfull = nv - (has_partial ? 1u : 0u);
+    uint32_t lane_cnt = 0;  // per work-item
+    const bool none = sg.hi < sg.lo;  // lo <= value <= hi holds for no value (block-uniform)
+    if (none) {
+    } else if (sg.enc == FLS_ENC_BITPACK) {
+        const uint32_t lo_adj = lo - sg.base;
+        switch (sg.bw) {
+#define FLS_BK_CASE(B) \
+    case B: lane_cnt = count_fixed_full<B, VPB>(sg.words, v0, nfull, lo_adj, span); break;
+            FLS_WIDTH_CASES(FLS_BK_CASE)
+#undef FLS_BK_CASE
+            default: break;
+        }
+        if (sg.bw == 0 && (0u - lo_adj) <= span && threadIdx.x == 0) lane_cnt = 1024u * nfull;
+    } else if (sg.enc == FLS_ENC_DELTA) {
+        // one width for the whole tile range takes the batched walk
+        uint32_t mn = 0xffffffffu, mx = 0u;
+        for (uint32_t i = threadIdx.x; i < nfull; i += BLOCK) {
+            const uint32_t b = FLS_VMETA_BW(ldg(sg.vmeta + v0 + i));
+            mn = min(mn, b);
+            mx = max(mx, b);
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            mn = min(mn, (uint32_t)__shfl_xor(mn, off, 64));
+            mx = max(mx, (uint32_t)__shfl_xor(mx, off, 64));
+        }
+        if (dev::is_wave_leader()) {
+            s.mm[2 * wave] = mn;
+            s.mm[2 * wave + 1] = mx;
+        }
+        __syncthreads();
+        mn = s.mm[0];
+        mx = s.mm[1];
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) {
+            mn = min(mn, s.mm[2 * w]);
+            mx = max(mx, s.mm[2 * w + 1]);
+        }
+        if (nfull && mn == mx) {
+            switch (mn) {
+#define FLS_DK_CASE(B)                                                                                  \
+    case B: lane_cnt = count_delta_full<B, VPB>(sg.words, sg.vmeta, sg.bases, v0, nfull, lo, span); break;
+                FLS_WIDTH_CASES(FLS_DK_CASE)
+#undef FLS_DK_CASE
+                default: break;
+            }
+        } else {
+            // widths differ inside the tile: one vector per half-wave at its own width
+            for (uint32_t vb = hw; vb < nfull; vb += VPB) {
+                const uint64_t v = v0 + vb;
+                const fls_vmeta m = ldg(sg.vmeta + v);
+                uint32_t c = 0;
+                auto f = [&](int, uint32_t x) { c += (uint32_t)(x - lo <= span); };
+                walk_delta(sg.words + FLS_VMETA_OFFSET(m) + dev::lane32(), FLS_VMETA_BW(m),
+                           ldg(sg.bases + v * 32u + dev::lane32()), f);
+                lane_cnt += c;
+            }
+        }
+    } else if (sg.enc == FLS_ENC_RLE) {
+        lane_cnt = count_rle_full<VPB, kRleK>(sg, v0, nfull, lo, span, s.flags);
+    } else {  // MIXED: every vector through the slow path
+        for (uint32_t vb = hw; vb < nfull; vb += VPB)
+            lane_cnt += count_vector_slow(sg, v0 + vb, 0xffffffffu, lo, span);
+    }
+    if (has_partial && hw == 0 && !none) {
+        const uint64_t v = seg_vecs - 1u;
+        lane_cnt += count_vector_slow(sg, v, live_row_mask((uint32_t)(sg.n_values - v * 1024u), sg.transposed != 0),
+                                      lo, span);
+    }
+    const uint32_t total_wave = dev::wave_sum(lane_cnt);
+    if (dev::is_wave_leader()) s.part[wave] = total_wave;
+    __syncthreads();
+    uint64_t total = 0;
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) total += s.part[w];
+    }
+    return total;
+}
+
 // Tile counters, a 128-byte line each.
 constexpr uint32_t kQueues = 8, kQueueStride = 32;
 
@@ -442,13 +540,8 @@ template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) void batch_kernel(const SegDev* __restrict segs, const TileDev* __restrict tiles,
                                                       uint32_t n_tiles, uint64_t* __restrict counts,
                                                       uint32_t* __restrict queue, uint32_t dynamic) {
-    constexpr int VPB = BLOCK / 32;
-    constexpr int WAVES = BLOCK / 64;
-    __shared__ uint32_t flags_lds[VPB * kRleK * kFlagWords];
-    __shared__ uint32_t s_part[WAVES];
-    __shared__ uint32_t s_mm[2 * WAVES];
+    __shared__ BatchLds<BLOCK> s;
     __shared__ uint32_t s_tile;
-    const uint32_t hw = threadIdx.x >> 5, wave = threadIdx.x >> 6;
     // Tiles past the first round come from kQueues counters (the tile numbers
     // that are q mod kQueues from counter q), a block's own first and the others
     // once that has run out: atomics on one address complete 5 ns apart, which
@@ -460,87 +553,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) v
     while (t < n_tiles) {  // uniform over the block
         const TileDev tile = tiles[t];
         const SegDev sg = segs[tile.seg];
-        const uint32_t lo = sg.lo, span = sg.hi - sg.lo;
-        const uint64_t seg_vecs = ceil_div(sg.n_values, 1024);
-        const bool has_partial = (sg.n_values & 1023u) != 0 && tile.v0 + tile.nv == seg_vecs;
-        const uint32_t nfull = tile.nv - (has_partial ? 1u : 0u);
-        uint32_t lane_cnt = 0;  // per work-item
-        const bool none = sg.hi < sg.lo;  // lo <= value <= hi holds for no value (block-uniform)
-        if (none) {
-        } else if (sg.enc == FLS_ENC_BITPACK) {
-            const uint32_t lo_adj = lo - sg.base;
-            switch (sg.bw) {
-#define FLS_BK_CASE(B) \
-    case B: lane_cnt = count_fixed_full<B, VPB>(sg.words, tile.v0, nfull, lo_adj, span); break;
-                FLS_WIDTH_CASES(FLS_BK_CASE)
-#undef FLS_BK_CASE
-                default: break;
-            }
-            if (sg.bw == 0 && (0u - lo_adj) <= span && threadIdx.x == 0) lane_cnt = 1024u * nfull;
-        } else if (sg.enc == FLS_ENC_DELTA) {
-            // one width for the whole tile range takes the batched walk
-            uint32_t mn = 0xffffffffu, mx = 0u;
-            for (uint32_t i = threadIdx.x; i < nfull; i += BLOCK) {
-                const uint32_t b = FLS_VMETA_BW(ldg(sg.vmeta + tile.v0 + i));
-                mn = min(mn, b);
-                mx = max(mx, b);
-            }
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                mn = min(mn, (uint32_t)__shfl_xor(mn, off, 64));
-                mx = max(mx, (uint32_t)__shfl_xor(mx, off, 64));
-            }
-            if (dev::is_wave_leader()) {
-                s_mm[2 * wave] = mn;
-                s_mm[2 * wave + 1] = mx;
-            }
-            __syncthreads();
-            mn = s_mm[0];
-            mx = s_mm[1];
-#pragma unroll
-            for (int w = 1; w < WAVES; ++w) {
-                mn = min(mn, s_mm[2 * w]);
-                mx = max(mx, s_mm[2 * w + 1]);
-            }
-            if (nfull && mn == mx) {
-                switch (mn) {
-#define FLS_DK_CASE(B)                                                                                       \
-    case B: lane_cnt = count_delta_full<B, VPB>(sg.words, sg.vmeta, sg.bases, tile.v0, nfull, lo, span); \
-        break;
-                    FLS_WIDTH_CASES(FLS_DK_CASE)
-#undef FLS_DK_CASE
-                    default: break;
-                }
-            } else {
-                // widths differ inside the tile: one vector per half-wave at its own width
-                for (uint32_t vb = hw; vb < nfull; vb += VPB) {
-                    const uint64_t v = tile.v0 + vb;
-                    const fls_vmeta m = ldg(sg.vmeta + v);
-                    uint32_t c = 0;
-                    auto f = [&](int, uint32_t x) { c += (uint32_t)(x - lo <= span); };
-                    walk_delta(sg.words + FLS_VMETA_OFFSET(m) + dev::lane32(), FLS_VMETA_BW(m),
-                               ldg(sg.bases + v * 32u + dev::lane32()), f);
-                    lane_cnt += c;
-                }
-            }
-        } else if (sg.enc == FLS_ENC_RLE) {
-            lane_cnt = count_rle_full<VPB, kRleK>(sg, tile.v0, nfull, lo, span, flags_lds);
-        } else {  // MIXED: every vector through the slow path
-            for (uint32_t vb = hw; vb < nfull; vb += VPB)
-                lane_cnt += count_vector_slow(sg, tile.v0 + vb, 0xffffffffu, lo, span);
-        }
-        if (has_partial && hw == 0 && !none) {
-            const uint64_t v = seg_vecs - 1u;
-            lane_cnt += count_vector_slow(sg, v, live_row_mask((uint32_t)(sg.n_values - v * 1024u), sg.transposed != 0),
-                                          lo, span);
-        }
-        const uint32_t total_wave = dev::wave_sum(lane_cnt);
-        if (dev::is_wave_leader()) s_part[wave] = total_wave;
-        __syncthreads();
+        const uint64_t total = count_tile(sg, tile.v0, tile.nv, s);
         if (threadIdx.x == 0) {
-            uint64_t total = 0;
-#pragma unroll
-            for (int w = 0; w < WAVES; ++w) total += s_part[w];
             if (total) atomicAdd((unsigned long long*)&counts[tile.seg], (unsigned long long)total);
             uint32_t next = t + gridDim.x;
             if (dynamic) {
@@ -552,9 +566,21 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) v
             }
             s_tile = next;
         }
-        __syncthreads();  // s_part / s_mm / flags are rewritten next iteration
+        __syncthreads();  // the counting's LDS is rewritten next iteration
         t = __builtin_amdgcn_readfirstlane(s_tile);
     }
+}
+
+// One segment, a block per tile of it: no list, so such a launch needs nothing
+// uploaded before it.
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) void segment_kernel(
+    const SegDev* __restrict seg, uint32_t tile_vectors, uint64_t* __restrict count) {
+    __shared__ BatchLds<BLOCK> s;
+    const SegDev sg = *seg;
+    const uint32_t v0 = blockIdx.x * tile_vectors, nv = (uint32_t)ceil_div(sg.n_values, 1024) - v0;
+    const uint64_t total = count_tile(sg, v0, min(nv, tile_vectors), s);
+    if (threadIdx.x == 0 && total) atomicAdd((unsigned long long*)count, (unsigned long long)total);
 }
 
 // The counters and the tile queues of a run, in one launch.
@@ -675,10 +701,6 @@ struct fls_batch {
     fls::TileDev* d_tiles = nullptr;
     uint32_t n_tiles = 0;
     uint64_t tile_lists = 0;  // tile lists uploaded so far: a captured graph holds the address of one
-    // and, for launches of one segment each, in segment order
-    uint32_t seg_tile_vectors = 0, seg_class_tiles = 0;
-    fls::TileDev* d_seg_tiles = nullptr;
-    std::vector<uint32_t> seg_tile_off, seg_tile_cnt;
     uint32_t* d_queue = nullptr;
     // graph
     hipStream_t cap_stream = nullptr;
@@ -718,9 +740,8 @@ uint32_t vector_cost(const fls_batch* b, uint32_t s) {
 }
 
 // Cut the segments into tiles (only those of class `only`, when >= 0), segment
-// by segment; per segment its tiles' place, if asked for.
-std::vector<TileDev> cut_tiles(const fls_batch* b, const fls_tune& t, int only, std::vector<uint32_t>* off,
-                               std::vector<uint32_t>* cnt) {
+// by segment.
+std::vector<TileDev> cut_tiles(const fls_batch* b, const fls_tune& t, int only) {
     std::vector<TileDev> tiles;
     size_t most = 0;
     for (uint32_t s = 0; s < b->segs.size(); ++s)
@@ -728,7 +749,6 @@ std::vector<TileDev> cut_tiles(const fls_batch* b, const fls_tune& t, int only, 
     tiles.reserve(most);
     for (uint32_t s = 0; s < b->segs.size(); ++s) {
         const uint32_t cls = seg_class(b, s);
-        const size_t first = tiles.size();
         if (only < 0 || (int)cls == only) {
             const uint32_t tv = class_tile(t, cls), cost = vector_cost(b, s);
             const uint64_t nv = ceil_div(b->segs[s].n_values, 1024);
@@ -738,8 +758,6 @@ std::vector<TileDev> cut_tiles(const fls_batch* b, const fls_tune& t, int only, 
                 tiles.push_back(TileDev{s, (uint32_t)v0, n, c < 0xffffffffu ? (uint32_t)c : 0xffffffffu});
             }
         }
-        if (off) off->push_back((uint32_t)first);
-        if (cnt) cnt->push_back((uint32_t)(tiles.size() - first));
     }
     return tiles;
 }
@@ -796,27 +814,13 @@ int set_tiles(fls_batch* b, const fls_tune& t, int only = -1) {
     if (t.tile_vectors == 0) return FLS_ERR_ARG;
     if (b->d_tiles && b->tile_vectors == t.tile_vectors && b->class_tiles == t.class_tiles && b->tile_filter == only)
         return FLS_OK;
-    const std::vector<TileDev> tiles = run_order(cut_tiles(b, t, only, nullptr, nullptr));
+    const std::vector<TileDev> tiles = run_order(cut_tiles(b, t, only));
     if (const int st = upload_tiles(&b->d_tiles, tiles)) return st;
     ++b->tile_lists;
     b->n_tiles = (uint32_t)tiles.size();
     b->tile_vectors = t.tile_vectors;
     b->class_tiles = t.class_tiles;
     b->tile_filter = only;
-    return FLS_OK;
-}
-
-// The same for launches of one segment each: the tiles as they lie.
-int set_seg_tiles(fls_batch* b, const fls_tune& t) {
-    if (t.tile_vectors == 0) return FLS_ERR_ARG;
-    if (b->d_seg_tiles && b->seg_tile_vectors == t.tile_vectors && b->seg_class_tiles == t.class_tiles) return FLS_OK;
-    std::vector<uint32_t> off, cnt;
-    const std::vector<TileDev> tiles = cut_tiles(b, t, -1, &off, &cnt);
-    if (const int st = upload_tiles(&b->d_seg_tiles, tiles)) return st;
-    b->seg_tile_off.swap(off);
-    b->seg_tile_cnt.swap(cnt);
-    b->seg_tile_vectors = t.tile_vectors;
-    b->seg_class_tiles = t.class_tiles;
     return FLS_OK;
 }
 
@@ -1153,16 +1157,19 @@ int fls_batch_run_per_segment(fls_batch* b, const fls_tune* tune, uint64_t* d_co
     if (!b || !d_counts) return FLS_ERR_NULL;
     int st;
     if ((st = check_tune(tune)) != FLS_OK) return st;
-    if ((st = set_seg_tiles(b, *tune)) != FLS_OK) return st;
     hipStream_t s = as_stream(stream);
     if ((st = zero_u64(d_counts, b->segs.size(), s)) != FLS_OK) return st;
     for (uint32_t i = 0; i < b->segs.size(); ++i) {
         // one launch per segment: one block per tile of the segment
-        const uint32_t nt = b->seg_tile_cnt[i];
-        const TileDev* tiles = b->d_seg_tiles + b->seg_tile_off[i];
-        st = tune->block_threads == 512 ? launch_batch<512>(b, d_counts, false, tiles, nt, nt, s)
-                                        : launch_batch<256>(b, d_counts, false, tiles, nt, nt, s);
-        if (st) return st;
+        const uint32_t tv = class_tile(*tune, seg_class(b, i));
+        const uint64_t tiles = ceil_div(ceil_div(b->segs[i].n_values, 1024), tv);
+        if (tiles == 0) continue;
+        FLS_RETURN_IF(tiles > 0x7fffffffu, FLS_ERR_SIZE);
+        if (tune->block_threads == 512)
+            hipLaunchKernelGGL(segment_kernel<512>, dim3((uint32_t)tiles), dim3(512), 0, s, b->d_segs + i, tv, d_counts + i);
+        else
+            hipLaunchKernelGGL(segment_kernel<256>, dim3((uint32_t)tiles), dim3(256), 0, s, b->d_segs + i, tv, d_counts + i);
+        if ((st = check_launch()) != FLS_OK) return st;
     }
     return FLS_OK;
 }
@@ -1289,7 +1296,6 @@ void fls_batch_destroy(fls_batch* b) {
     if (b->graph) (void)hipGraphDestroy(b->graph);
     if (b->cap_stream) (void)hipStreamDestroy(b->cap_stream);
     if (b->d_tiles) (void)hipFree(b->d_tiles);
-    if (b->d_seg_tiles) (void)hipFree(b->d_seg_tiles);
     if (b->d_segs) (void)hipFree(b->d_segs);
     if (b->d_queue) (void)hipFree(b->d_queue);
     if (b->d_words) (void)hipFree(b->d_words);

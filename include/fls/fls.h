@@ -647,9 +647,10 @@ int fls_batch_segment(const fls_batch* b, uint32_t s, fls_segment_info* info);
 /* Segment s as fls_batch_create takes it: device pointers borrowed from the
  * batch (valid until fls_batch_destroy), e.g. to copy a segment out.        */
 int fls_batch_segment_column(const fls_batch* b, uint32_t s, fls_segment* seg);
-/* one persistent launch (after two tiny zero-fill kernels) */
+/* one persistent launch (after a tiny zero-fill kernel); the first run of a
+ * tiling uploads its tile list, so a capture takes runs of the current one  */
 int fls_batch_run(fls_batch* b, const fls_tune* tune, uint64_t* d_counts, void* stream);
-/* baseline: one launch per segment */
+/* baseline: one launch per segment, nothing uploaded                         */
 int fls_batch_run_per_segment(fls_batch* b, const fls_tune* tune, uint64_t* d_counts, void* stream);
 /* fls_batch_run captured once in a hipGraph (re-captured when tune or
  * d_counts change) and replayed on `stream`                                  */

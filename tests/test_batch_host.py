@@ -112,7 +112,6 @@ int main(int argc, char** argv) {
     fls_batch* b = nullptr;
     NEED(create(seg, 3, &b) == FLS_OK);
     const fls_tune small = {16, 256, FLS_SCHED_DYNAMIC, 0}, large = {64, 256, FLS_SCHED_DYNAMIC, 0};
-    (void)per_segment;
     BODY
     NEED(stale == 0);
     destroy(b);
@@ -140,6 +139,19 @@ FAILED_UPLOAD = r"""
     NEED(graph(b, &small, counts, nullptr) == FLS_OK);
 """
 
+# hipMalloc, hipMemcpy and hipFree fail in a capture that forbids them
+CAPTURED = r"""
+    NEED(run(b, &small, counts, nullptr) == FLS_OK);
+    user_capture = true;
+    int before = launches;
+    NEED(run(b, &small, counts, nullptr) == FLS_OK);
+    NEED(launches == before + 2);
+    NEED(per_segment(b, &small, counts, nullptr) == FLS_OK);
+    NEED(launches == before + 2 + 1 + 3);  // one clears the counters
+    NEED(run(b, &small, counts, nullptr) == FLS_OK);
+    user_capture = false;
+"""
+
 
 def run_body(tmp_path, body):
     src, exe = tmp_path / "batch_host.cpp", tmp_path / "batch_host"
@@ -155,4 +167,10 @@ def run_body(tmp_path, body):
 def test_a_failed_tile_upload_leaves_the_batch_as_it_was(tmp_path, fail):
     """No graph replays and no launch reads a list that was freed on the way to a
     list that could not be allocated or filled."""
-    run_body(tmp_path, FAILED_UPLOAD.replace("FAIL", fail))
+    run_body(tmp_path, FAILED_UPLOAD.replace("FAIL", fail) + "    (void)per_segment;")
+
+
+def test_per_segment_launches_are_captured_after_a_run(tmp_path):
+    """After a run, the launches of one segment each need no allocation or copy:
+    a capture takes them, as it takes another run."""
+    run_body(tmp_path, CAPTURED + "    (void)graph, (void)large;")
