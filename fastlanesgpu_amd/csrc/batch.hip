@@ -700,7 +700,7 @@ struct fls_batch {
     int tile_filter = -2;
     fls::TileDev* d_tiles = nullptr;
     uint32_t n_tiles = 0;
-    uint64_t tile_lists = 0;  // tile lists uploaded so far: a captured graph holds the address of one
+    uint64_t tile_lists = 0;  // tile lists there have been: a captured graph holds the address of one
     uint32_t* d_queue = nullptr;
     // graph
     hipStream_t cap_stream = nullptr;
@@ -792,31 +792,22 @@ std::vector<TileDev> run_order(const std::vector<TileDev>& tiles) {
     return out;
 }
 
-// The new list takes the old one's place when it is complete: after a failure
-// the old one is still what its key and a captured graph say it is.
-int upload_tiles(TileDev** d, const std::vector<TileDev>& tiles) {
-    TileDev* list = nullptr;
-    FLS_HIP_CHECK(hipMalloc((void**)&list, sizeof(TileDev) * (tiles.size() ? tiles.size() : 1)));
-    if (!tiles.empty()) {
-        const hipError_t e = hipMemcpy(list, tiles.data(), sizeof(TileDev) * tiles.size(), hipMemcpyHostToDevice);
-        if (e != hipSuccess) {
-            (void)hipFree(list);
-            return record_hip_error(e);
-        }
-    }
-    if (*d) (void)hipFree(*d);
-    *d = list;
-    return FLS_OK;
-}
-
 // Upload the tile list of a run, unless the current one already is that tiling.
+// Before the old list is freed, its key and every graph captured with it become
+// invalid, so that a failure on the way leaves nothing that still names it.
+// (Allocated before the old one is freed, the new list cost 10 us more.)
 int set_tiles(fls_batch* b, const fls_tune& t, int only = -1) {
     if (t.tile_vectors == 0) return FLS_ERR_ARG;
     if (b->d_tiles && b->tile_vectors == t.tile_vectors && b->class_tiles == t.class_tiles && b->tile_filter == only)
         return FLS_OK;
     const std::vector<TileDev> tiles = run_order(cut_tiles(b, t, only));
-    if (const int st = upload_tiles(&b->d_tiles, tiles)) return st;
+    b->tile_vectors = 0;
     ++b->tile_lists;
+    if (b->d_tiles) FLS_HIP_CHECK(hipFree(b->d_tiles));
+    b->d_tiles = nullptr;
+    FLS_HIP_CHECK(hipMalloc((void**)&b->d_tiles, sizeof(TileDev) * (tiles.size() ? tiles.size() : 1)));
+    if (!tiles.empty())
+        FLS_HIP_CHECK(hipMemcpy(b->d_tiles, tiles.data(), sizeof(TileDev) * tiles.size(), hipMemcpyHostToDevice));
     b->n_tiles = (uint32_t)tiles.size();
     b->tile_vectors = t.tile_vectors;
     b->class_tiles = t.class_tiles;
