@@ -381,8 +381,17 @@ class LearnedSelector:
     def encode(self, d_in, n, ws, stream=None):
         """The learned encode: statistics and features in one pass, the
         network's choice (ws.cls, ws.conf), the plan with the confidence
-        fallback, and the pack.  Asynchronous; ws.column(n) reads the result."""
-        mixed_stats(d_in, n, ws, features=True, stream=stream)
-        self.classify(n, ws, stream)
-        mixed_resolve(n, ws, conf=ws.conf, conf_min=self.conf_min, stream=stream)
+        fallback, and the pack.  A choose that is not this class's own is called
+        in the place of the first two, and its choice planned from the input.
+        Asynchronous; ws.column(n) reads the result."""
+        if getattr(self.choose, "__func__", None) is _OWN_CHOOSE:
+            mixed_stats(d_in, n, ws, features=True, stream=stream)
+            self.classify(n, ws, stream)
+            mixed_resolve(n, ws, conf=ws.conf, conf_min=self.conf_min, stream=stream)
+        else:
+            self.choose(d_in, n, ws, stream)
+            mixed_plan(d_in, n, ws, conf=ws.conf, conf_min=self.conf_min, stream=stream)
         mixed_pack(d_in, n, ws, stream)
+
+
+_OWN_CHOOSE = LearnedSelector.choose
