@@ -48,12 +48,17 @@ struct ColDev {
 };
 
 // Whether a decode reads its packed words through the caches, by their bytes.
-// Columns that fit the 256 MB memory-side cache beside others are worth
-// keeping there (they were written or read before, and will be read again);
-// larger ones only evict each other.  Two columns unpacked in turn, not kept
-// and kept: 60M values of 11 bits (82 MB) 54.3 and 47.0 us, 18 bits (135 MB)
-// 61.2 and 56.4, 24 bits (180 MB) 68.7 and 69.8, 120M of 28 bits 144 and 152.
-// Full scans (queries) read more than that and were faster not keeping.
+// It gains what is still in the 256 MB memory-side cache from an earlier read,
+// and pays where another kernel's stores are, which its own lines then push out.
+// Unpack, us not kept and kept:
+//                                       23 MB       82 MB        128 MB       240 MB
+//   the same column again            15.5  12.3  54.3  46.5   60.4  53.2   75.4   68.5
+//   two columns in turn              15.8  13.7  54.2  46.5   60.8  53.2   76.0   80.8
+//   1.2 GB of columns in turn        16.5  16.5  54.6  53.8   61.5  60.6   77.1   81.0
+//   each with a kernel that adds 1
+//   to every value, the two          38.6  38.4 136.1 137.6  142.0 145.8  158.2  171.7
+//   each after a fill of 1 GB        19.1  21.1  55.7  69.0   62.4  83.4   79.1  125.7
+// Queries do not keep theirs.
 inline bool keep_cached(uint64_t packed_bytes) { return packed_bytes <= 128ull << 20; }
 
 // Validate a host-side column descriptor for n_rows rows and build its device
@@ -285,7 +290,7 @@ __device__ __forceinline__ void decode_regs(const ColDev& c, uint64_t v, uint32_
             nr = rm.n_runs < 1024u ? rm.n_runs : 1024u;
         }
     }
-    dev::unpack_device(p, x, w, CACHED);
+    dev::unpack_device<uint32_t, CACHED>(p, x, w);
     if (rsum) dev::rsum_lane(x, seed);
     if (RLE && vals) {
         const uint32_t last = nr ? nr - 1u : 0u;

@@ -69,7 +69,7 @@ __global__ __launch_bounds__(kBlock) void unpack_global_kernel(const uint32_t* _
     const uint64_t v = (uint64_t)blockIdx.x * kVecPerBlock + (threadIdx.x >> 5);
     const bool live = v < n_vec;
     uint32_t vals[32];
-    if (live) dev::unpack_lane<BW>(in + v * (32u * BW), vals, CACHED);
+    if (live) dev::unpack_lane<BW, CACHED>(in + v * (32u * BW), vals);
     if constexpr (CHECKSUM) {
         // sum_r (first + 32r) * v_r with first = v*1024 + l + 1
         //   = first * S0 + 32 * S1,  S0 = sum v_r,  S1 = sum r*v_r   (mod 2^64);
@@ -156,7 +156,7 @@ __global__ __launch_bounds__(kBlock) void delta_decode_kernel(const uint32_t* __
     if (v >= n_vec) return;
     const fls_vmeta m = vmeta[v];
     uint32_t vals[32];
-    dev::unpack_device(words + FLS_VMETA_OFFSET(m), vals, FLS_VMETA_BW(m), CACHED);
+    dev::unpack_device<uint32_t, CACHED>(words + FLS_VMETA_OFFSET(m), vals, FLS_VMETA_BW(m));
     dev::rsum_lane(vals, bases[v * 32u + l]);
     uint32_t* o = out + v * 1024u + l;
 #pragma unroll

@@ -76,13 +76,13 @@ __device__ __forceinline__ void extract_rows(const uint32_t (&w)[BW > 0 ? BW : 1
 
 // Load the BW words of one lane: `lane_in` points at word 0 of the lane
 // (vector base + lane).  Word k sits 32*k words further.  The words are read
-// past the caches, or with `cached` through them.
-template <int BW>
-__device__ __forceinline__ void load_lane(const uint32_t* __restrict lane_in, uint32_t (&w)[BW > 0 ? BW : 1],
-                                          bool cached = false) {
+// past the caches, or with CACHED through them (a template argument: two loads
+// under a run-time condition are merged into one without the hint).
+template <int BW, bool CACHED = false>
+__device__ __forceinline__ void load_lane(const uint32_t* __restrict lane_in, uint32_t (&w)[BW > 0 ? BW : 1]) {
     if constexpr (BW == 0) {
         w[0] = 0u;
-    } else if (cached) {
+    } else if constexpr (CACHED) {
 #pragma unroll
         for (int k = 0; k < BW; ++k) w[k] = lane_in[32 * k];
     } else {
@@ -95,25 +95,23 @@ __device__ __forceinline__ void load_lane(const uint32_t* __restrict lane_in, ui
 // `vec_in` is the vector's first packed word; the lane comes from threadIdx.
 // Counterpart of generated::unpack::cuda::fused::unpack_<bw>bw_32ow_32crw_1uf
 // (fastlanes/src/include/fls_gen/unpack/unpack_fused.cuh:7-3328).
-template <int BW>
-__device__ __forceinline__ void unpack_lane(const uint32_t* __restrict vec_in, uint32_t (&out)[32],
-                                            bool cached = false) {
+template <int BW, bool CACHED = false>
+__device__ __forceinline__ void unpack_lane(const uint32_t* __restrict vec_in, uint32_t (&out)[32]) {
     uint32_t w[BW > 0 ? BW : 1];
-    load_lane<BW>(vec_in + lane32(), w, cached);
+    load_lane<BW, CACHED>(vec_in + lane32(), w);
     extract_rows<BW>(w, out);
 }
 
 // Runtime-width dispatch, the reference's unpack_device(in, out, bw)
 // (unpack_fused.cuh:3455-3462).  Work-items of one half-wave must share bw for
 // best speed; divergent widths are correct but serialise.
-template <typename T>
-__device__ __forceinline__ void unpack_device(const T* __restrict vec_in, T (&out_t)[32], uint32_t bw,
-                                              bool cached = false) {
+template <typename T, bool CACHED = false>
+__device__ __forceinline__ void unpack_device(const T* __restrict vec_in, T (&out_t)[32], uint32_t bw) {
     const uint32_t* in = reinterpret_cast<const uint32_t*>(vec_in);
     uint32_t(&out)[32] = reinterpret_cast<uint32_t(&)[32]>(out_t);
     switch (bw) {
 #define FLS_UNPACK_CASE(B) \
-    case B: unpack_lane<B>(in, out, cached); break;
+    case B: unpack_lane<B, CACHED>(in, out); break;
         FLS_UNPACK_CASE(0) FLS_UNPACK_CASE(1) FLS_UNPACK_CASE(2) FLS_UNPACK_CASE(3) FLS_UNPACK_CASE(4)
         FLS_UNPACK_CASE(5) FLS_UNPACK_CASE(6) FLS_UNPACK_CASE(7) FLS_UNPACK_CASE(8) FLS_UNPACK_CASE(9)
         FLS_UNPACK_CASE(10) FLS_UNPACK_CASE(11) FLS_UNPACK_CASE(12) FLS_UNPACK_CASE(13) FLS_UNPACK_CASE(14)
