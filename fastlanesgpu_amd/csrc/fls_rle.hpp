@@ -69,6 +69,15 @@ __device__ __forceinline__ void rle_emit(const RleVector& r, RleLds& lds, uint32
     const uint32_t l = dev::lane32();
     const uint32_t nr = r.n_runs < 1024u ? r.n_runs : 1024u, last = nr ? nr - 1u : 0u;
     if (r.ibw > 1u) return rle_emit_wide<ROWS>(r, last, rows, dst);
+    if constexpr (VEC) {
+        // Two passes over the stage store only what each holds, so a word per
+        // work-item at consecutive places: the words of a 16-byte store taken
+        // one at a time touched four lines each (60M rows of 1,024 runs a
+        // vector: row order 134 us, stored order 202; this way 94 and 143).  The
+        // wave's two vectors go the same way, or both ways' code runs in turn
+        // (vectors of about 512 runs 69 and 72 us apart, 64 and 70 together).
+        if (__any(last >= kRunStage)) return rle_emit<ROWS, false>(r, lds, rows, dst);
+    }
     // through the cache: RLE vectors end anywhere in a line, which the next one
     // shares (with non-temporal loads here a line was read twice: 62.2 us
     // against 49.2 for 67M rows)
@@ -155,7 +164,7 @@ __device__ __forceinline__ void rle_emit(const RleVector& r, RleLds& lds, uint32
             }
             const uint32_t p = VEC ? 4u * l + 128u * (uint32_t)j : 128u * (uint32_t)j + l;
             constexpr uint32_t step = VEC ? 1u : 32u;  // place of output 4j + i: p + step * i
-            if (last < kRunStage && p + 3u * step < rows) {
+            if ((VEC || last < kRunStage) && p + 3u * step < rows) {
                 if constexpr (VEC) {
                     __builtin_nontemporal_store(u32x4{x[0], x[1], x[2], x[3]}, reinterpret_cast<u32x4*>(dst + p));
                 } else {
@@ -170,7 +179,7 @@ __device__ __forceinline__ void rle_emit(const RleVector& r, RleLds& lds, uint32
             __builtin_amdgcn_sched_barrier(0);  // few outputs in flight: their registers cost more waves than they hide
         }
         from += kRunStage;
-        if (from > last) break;
+        if (VEC || from > last) break;
         fence();
         stage(from, min(last + 1u, from + kRunStage));
         fence();

@@ -180,6 +180,25 @@ def test_decode_rle_run_counts(ibw, vbw):
         assert np.all(got[shift + rows.size:] == 0xFFFFFFFF)
 
 
+@pytest.mark.parametrize("ibw", [1, 3])
+def test_decode_rle_vectors_beside_one_with_more_runs(ibw):
+    """The two vectors of a wave on either side of the stage's 512 runs, and one
+    with index deltas wider than a bit, in both orders, aligned and not; the
+    last vector is partial in row order."""
+    torch = T.torch_cuda()
+    col, rows = rle_vector_column([600, 5, 512, 513, 1, 1024, 1024, 30, 513, 511], ibw, 17)
+    stored = T.transpose_vectors(rows)
+    n = rows.size - 1001
+    for shift in (0, 1, 2):
+        buf = torch.full((rows.size + 8,), -1, dtype=torch.int32, device="cuda")
+        fls.decode_column(col, n, fls.ORDER_ROWS, out=buf[shift:shift + n])
+        got = T.from_dev(buf)
+        np.testing.assert_array_equal(got[shift:shift + n], rows[:n])
+        assert np.all(got[shift + n:] == 0xFFFFFFFF)
+        fls.decode_column(col, rows.size, fls.ORDER_STORED, out=buf[shift:shift + rows.size])
+        np.testing.assert_array_equal(T.from_dev(buf)[shift:shift + rows.size], stored)
+
+
 def test_decode_mixed_column_with_rle_vectors():
     """RLE vectors of every run count beside other encodings in one column."""
     import fastlanesgpu_amd.selector as sel
