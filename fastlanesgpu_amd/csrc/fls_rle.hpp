@@ -62,8 +62,11 @@ __device__ __forceinline__ void rle_emit_wide(const RleVector& r, uint32_t last,
 
 // Decode the half-wave's vector to dst: rows 0..rows-1 in original order
 // (ROWS), or all 1,024 stored positions (rows = 1024).  VEC: dst is 16-byte
-// aligned.  `lds` is this half-wave's; every exchange stays inside it.
-template <bool ROWS, bool VEC>
+// aligned.  ALIGNED: it is whether or not VEC is used; its stores are
+// non-temporal, those to other outputs are not, because they end in the middle
+// of a line (120M rows of mean run 8, unaligned: 199 us non-temporal, 144 this
+// way).  `lds` is this half-wave's; every exchange stays inside it.
+template <bool ROWS, bool VEC, bool ALIGNED = VEC>
 __device__ __forceinline__ void rle_emit(const RleVector& r, RleLds& lds, uint32_t rows, uint32_t* __restrict dst) {
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     const uint32_t l = dev::lane32();
@@ -76,7 +79,7 @@ __device__ __forceinline__ void rle_emit(const RleVector& r, RleLds& lds, uint32
         // vector: row order 134 us, stored order 202; this way 94 and 143).  The
         // wave's two vectors go the same way, or both ways' code runs in turn
         // (vectors of about 512 runs 69 and 72 us apart, 64 and 70 together).
-        if (__any(last >= kRunStage)) return rle_emit<ROWS, false>(r, lds, rows, dst);
+        if (__any(last >= kRunStage)) return rle_emit<ROWS, false, ALIGNED>(r, lds, rows, dst);
     }
     // through the cache: RLE vectors end anywhere in a line, which the next one
     // shares (with non-temporal loads here a line was read twice: 62.2 us
@@ -169,7 +172,10 @@ __device__ __forceinline__ void rle_emit(const RleVector& r, RleLds& lds, uint32
                     __builtin_nontemporal_store(u32x4{x[0], x[1], x[2], x[3]}, reinterpret_cast<u32x4*>(dst + p));
                 } else {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) __builtin_nontemporal_store(x[i], dst + p + step * i);
+                    for (int i = 0; i < 4; ++i) {
+                        if constexpr (ALIGNED) __builtin_nontemporal_store(x[i], dst + p + step * i);
+                        else dst[p + step * i] = x[i];
+                    }
                 }
             } else {
 #pragma unroll

@@ -78,8 +78,12 @@ __global__ __launch_bounds__(kTrBlock) void transpose_kernel(const uint32_t* __r
 // A grid of every vector group (over the resident set with a grid-stride loop
 // the transpose measured 8-10 % slower; in materialize_kernel even a loop that
 // runs once cost 127 VGPRs instead of 54, addresses hoisted out of it: 92.0 us
-// against 88.1 for 120M delta rows).  Materialize's stores are non-temporal
-// (2-3 % faster there, 13 % slower in the transpose).
+// against 88.1 for 120M delta rows).  Materialize's stores to aligned outputs are
+// non-temporal (2-3 % faster there, 13 % slower in the transpose).  To other
+// outputs they are not: every store instruction then ends in the middle of a
+// line, which only the caches can put together again (120M delta rows 205 us
+// non-temporal, 131 this way, stored order 187 and 101; 30M 45.5 and 22.1; 11
+// bits transposed 192 and 117).
 constexpr int kMatBlock = 256;          // 4 waves, two vectors per wave
 constexpr int kMatVecs = kMatBlock / 32;
 constexpr uint32_t kRowPad = 33u;       // words per 32 staged rows
@@ -136,10 +140,14 @@ __global__ __launch_bounds__(kMatBlock) void materialize_kernel(const ColDev c, 
         live = false;  // done
     }
     if (live) decode_regs<false, CACHED>(c, v, x);
+    auto put = [](uint32_t y, uint32_t* p) {  // one word: past the caches where whole lines are stored
+        if constexpr (VEC) __builtin_nontemporal_store(y, p);
+        else *p = y;
+    };
     if constexpr (!kStage) {
         if (live) {
 #pragma unroll
-            for (int r = 0; r < 32; ++r) __builtin_nontemporal_store(x[r], dst + 32u * r + l);
+            for (int r = 0; r < 32; ++r) put(x[r], dst + 32u * r + l);
         }
     } else {
         const uint32_t rows = !live ? 0u : ROWS ? (uint32_t)min<uint64_t>(1024u, n_rows - v * 1024u) : 1024u;
@@ -147,7 +155,7 @@ __global__ __launch_bounds__(kMatBlock) void materialize_kernel(const ColDev c, 
         if (ROWS && !c.transposed) {
 #pragma unroll
             for (int r = 0; r < 32; ++r)
-                if (32u * r + l < rows) __builtin_nontemporal_store(x[r], dst + 32u * r + l);
+                if (32u * r + l < rows) put(x[r], dst + 32u * r + l);
         } else if constexpr (!MIXED) {
             // the whole vector at once: by original row (ROWS) or by place
             if (live) {
@@ -175,7 +183,7 @@ __global__ __launch_bounds__(kMatBlock) void materialize_kernel(const ColDev c, 
             } else {
 #pragma unroll
                 for (int r = 0; r < 32; ++r)
-                    if (32u * r + l < rows) __builtin_nontemporal_store(st[kRowPad * r + l], dst + 32u * r + l);
+                    if (32u * r + l < rows) put(st[kRowPad * r + l], dst + 32u * r + l);
             }
         } else if constexpr (ROWS) {
             // the lane's chain is 32 consecutive rows: half of the chains (512
@@ -206,7 +214,7 @@ __global__ __launch_bounds__(kMatBlock) void materialize_kernel(const ColDev c, 
                 } else {
 #pragma unroll
                     for (int r = 0; r < 16; ++r)
-                        if (32u * r + l < here) __builtin_nontemporal_store(st[kRowPad * r + l], d + 32u * r + l);
+                        if (32u * r + l < here) put(st[kRowPad * r + l], d + 32u * r + l);
                 }
                 fence();
             }
