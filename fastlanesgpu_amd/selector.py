@@ -21,7 +21,8 @@ import ctypes
 
 import numpy as np
 
-from . import ENC_MIXED, VECTOR_SIZE, Column, _dev_u32, _dev_u64, _side_stream, _stream, call, dptr, load
+from . import (ENC_MIXED, VECTOR_SIZE, Column, _dev_u32, _dev_u64, _side_stream, _stream, call, current_stream,
+               dptr, load)
 
 MIX_BITPACK, MIX_FOR, MIX_DELTA, MIX_RLE = 0, 1, 2, 3
 ENCODING_NAMES = ("bitpack", "for", "delta", "rle")
@@ -229,27 +230,27 @@ class MixedWorkspace:
     def column(self, n):
         """The encoded MIXED column (views of this workspace).  torch's current
         stream waits for the encode first where that ran on another one."""
-        import torch
+        if self.ready is not None and self.ready != current_stream():
+            import torch
 
-        if isinstance(self.ready, torch.cuda.Event):
-            torch.cuda.current_stream().wait_event(self.ready)
-        else:
-            side = _side_stream(self.ready)
-            if side is not None:
-                torch.cuda.current_stream().wait_stream(side)
+            if isinstance(self.ready, torch.cuda.Event):
+                torch.cuda.current_stream().wait_event(self.ready)
+            else:
+                torch.cuda.current_stream().wait_stream(_side_stream(self.ready))
         total = int(self.total.item())
         nv = n_vectors(n)
         return Column(ENC_MIXED, n, self.words[:max(1, total)], vmeta=self.vmeta[:max(1, nv)],
                       aux=self.aux[:max(1, nv)], n_words=total)
 
 
-def _written(ws, stream):
-    """Note for ws.column where an encode step has just been put: an event on an
-    explicit stream, which its owner may destroy before the column is read, or
-    the address of the stream that was torch's current one."""
+def _written(ws, stream, raw):
+    """Note for ws.column where an encode step has just been put (`raw`, for the
+    argument `stream`): the address of the stream that was torch's current one,
+    or an event on an explicit one, which its owner may destroy before the column
+    is read."""
     side = _side_stream(stream)
     if side is None:
-        ws.ready = _stream(None)
+        ws.ready = raw if stream is None else current_stream()
         return
     import torch
 
@@ -263,9 +264,10 @@ def _written(ws, stream):
 
 def mixed_plan(d_in, n, ws, conf=None, conf_min=0.0, stream=None):
     ws.stats_n = None
+    raw = _stream(stream)
     call("fls_mixed_plan_device", dptr(d_in), n, dptr(ws.cls), dptr(conf), ctypes.c_float(conf_min),
-         dptr(ws.vmeta), dptr(ws.aux), dptr(ws.total), dptr(ws.fallbacks), dptr(ws.scratch), _stream(stream))
-    _written(ws, stream)
+         dptr(ws.vmeta), dptr(ws.aux), dptr(ws.total), dptr(ws.fallbacks), dptr(ws.scratch), raw)
+    _written(ws, stream, raw)
 
 
 def mixed_stats(d_in, n, ws, features=False, stream=None):
@@ -284,15 +286,17 @@ def mixed_resolve(n, ws, conf=None, conf_min=0.0, exhaustive=False, stream=None)
     if ws.stats_n != n:
         raise ValueError(f"no statistics of {n} values in this workspace: run mixed_stats before every mixed_resolve")
     ws.stats_n = None
+    raw = _stream(stream)
     call("fls_mixed_resolve_device", n, dptr(ws.cls), dptr(conf), ctypes.c_float(conf_min), int(exhaustive),
          dptr(ws.vmeta), dptr(ws.aux), dptr(ws.total), None if exhaustive else dptr(ws.fallbacks), dptr(ws.scratch),
-         _stream(stream))
-    _written(ws, stream)
+         raw)
+    _written(ws, stream, raw)
 
 
 def mixed_pack(d_in, n, ws, stream=None):
-    call("fls_mixed_pack_device", dptr(d_in), n, dptr(ws.vmeta), dptr(ws.aux), dptr(ws.words), _stream(stream))
-    _written(ws, stream)
+    raw = _stream(stream)
+    call("fls_mixed_pack_device", dptr(d_in), n, dptr(ws.vmeta), dptr(ws.aux), dptr(ws.words), raw)
+    _written(ws, stream, raw)
 
 
 def mixed_encode(d_in, n, ws, conf=None, conf_min=0.0, stream=None):
@@ -302,10 +306,10 @@ def mixed_encode(d_in, n, ws, conf=None, conf_min=0.0, stream=None):
     120M rows (see mixed_encode_classes), kept for callers that want one
     launch."""
     ws.stats_n = None
+    raw = _stream(stream)
     call("fls_mixed_encode_device", dptr(d_in), n, dptr(ws.cls), dptr(conf), ctypes.c_float(conf_min),
-         dptr(ws.vmeta), dptr(ws.aux), dptr(ws.words), dptr(ws.total), dptr(ws.fallbacks), dptr(ws.scratch),
-         _stream(stream))
-    _written(ws, stream)
+         dptr(ws.vmeta), dptr(ws.aux), dptr(ws.words), dptr(ws.total), dptr(ws.fallbacks), dptr(ws.scratch), raw)
+    _written(ws, stream, raw)
 
 
 def mixed_encode_classes(d_in, n, ws, stream=None):
@@ -337,9 +341,10 @@ def mixed_encode_trial(d_in, n, ws, stream=None, buf=None):
     if buf is None:
         raise ValueError("no trial workspace: build with trial=True or pass buf=trial_buffer(n)")
     ws.stats_n = None
+    raw = _stream(stream)
     call("fls_mixed_encode_trial", dptr(d_in), n, dptr(ws.cls), dptr(ws.vmeta), dptr(ws.aux), dptr(ws.words),
-         dptr(ws.total), dptr(buf), _stream(stream))
-    _written(ws, stream)
+         dptr(ws.total), dptr(buf), raw)
+    _written(ws, stream, raw)
 
 
 def mixed_decode(col, out=None, stream=None):

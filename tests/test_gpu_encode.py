@@ -195,6 +195,13 @@ def test_encodes_on_another_stream(how):
         assert col.n_words == want[2].n_words, encode.__name__
         for k in ("words", "vmeta", "aux"):
             assert torch.equal(getattr(col, k), getattr(want[2], k)), (encode.__name__, k)
+    for stream in (0, torch.cuda.current_stream()):  # the stream that is current anyway, as an argument
+        ws.words.zero_()
+        sel.mixed_encode_exhaustive(x, n, ws, stream=stream)
+        assert torch.equal(ws.column(n).words, want[2].words)
+        with torch.cuda.stream(side):
+            busy()
+            assert torch.equal(ws.column(n).words, want[2].words)
     fresh = [fls.delta_encode_device(x, n, stream=0), fls.rle_encode_device(x, n, stream=torch.cuda.default_stream())]
     for g, w in zip(fresh, want):
         for a, b in zip(g, w):
