@@ -151,6 +151,46 @@ def test_offsets_over_several_scan_blocks(n_vec):
     assert int(ws.fallbacks.item()) == 2 * int((conf < 0.3).sum())
 
 
+def test_offsets_over_more_scan_blocks_than_run_at_once():
+    """More blocks than are resident together, which their tickets put in order,
+    and more than 1,024 of them before the last, whose sums it adds in two trips:
+    the delta plan's offsets against its widths, and the resolve's against the
+    sizes of the exhaustive search (both plans only, nothing is packed)."""
+    import fastlanesgpu_amd.selector as sel
+    torch = T.torch_cuda()
+    n_vec = 1024 * 1024 + 1025
+    n = n_vec * 1024
+    g = torch.Generator(device="cuda")
+    g.manual_seed(5)
+    step = torch.randint(0, 8, (n_vec,), generator=g, device="cuda", dtype=torch.int32)
+    ramp = torch.arange(1024, device="cuda", dtype=torch.int32) & 31  # every chain 0, s, 2s, ..., 31s
+    x = (step[:, None] * ramp[None, :]).reshape(-1)
+    vmeta, aux, total = (torch.empty(k, dtype=torch.int64, device="cuda") for k in (n_vec, n_vec, 1))
+    bases = torch.empty(32 * n_vec, dtype=torch.int32, device="cuda")
+    scratch = torch.empty(int(fls.load().fls_encode_scratch_bytes(n)), dtype=torch.uint8, device="cuda")
+    cls = torch.empty(n_vec, dtype=torch.uint8, device="cuda")
+
+    def offsets(sizes):
+        ends = torch.cumsum(sizes, 0)
+        return ends - sizes, int(ends[-1])
+
+    fls.call("fls_delta_plan_device", fls.dptr(x), n, fls.dptr(vmeta), fls.dptr(bases), fls.dptr(total),
+             fls.dptr(scratch), fls.current_stream())
+    width = torch.zeros_like(step) + (step >= 1) + (step >= 2) + (step >= 4)
+    off, end = offsets(32 * width.long())
+    assert torch.equal(vmeta & 255, width.long())
+    assert torch.equal(vmeta >> 8, off)
+    assert int(total.item()) == end
+    _, sizes4 = sel.exhaustive_select(x, n)
+    off, end = offsets((sizes4[:n_vec].min(1).values.long() - 16) // 4)
+    fls.call("fls_mixed_stats_device", fls.dptr(x), n, None, fls.dptr(vmeta), fls.dptr(aux), fls.dptr(scratch),
+             fls.current_stream())
+    fls.call("fls_mixed_resolve_device", n, fls.dptr(cls), None, 0.0, 1, fls.dptr(vmeta), fls.dptr(aux),
+             fls.dptr(total), None, fls.dptr(scratch), fls.current_stream())
+    assert torch.equal(vmeta >> 8, off)
+    assert int(total.item()) == end
+
+
 @pytest.mark.parametrize("how", ["explicit", "current"])
 def test_encodes_on_another_stream(how):
     """Encodes on a stream that has other work queued first: the size is read in
