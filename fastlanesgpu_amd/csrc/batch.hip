@@ -533,9 +533,9 @@ constexpr uint32_t kQueues = 8, kQueueStride = 32;
 // Eight waves per SIMD (64 VGPRs): the fast paths are latency-bound, and
 // measured 2.32 ms at five waves against 1.99 ms at eight over the
 // 4096-segment batch (a few loop-invariant values spill; no spill in a row loop).
-// That batch (9.3 GB) takes 1,770 us now, 5.25 TB/s, against 1,930 with one
-// queue, non-temporal loads and an instruction more per delta and RLE row;
-// 1,024 segments of up to 2^18 values in 64-vector tiles 49 against 61.
+// That batch (9.3 GB, 128-vector tiles) takes 1,672 us, 5.56 TB/s; with one queue,
+// non-temporal loads and an instruction more per delta and RLE row 1,832.  1,024
+// segments of up to 2^18 values in 64-vector tiles 49 against 61.
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) void batch_kernel(const SegDev* __restrict segs, const TileDev* __restrict tiles,
                                                       uint32_t n_tiles, uint64_t* __restrict counts,
@@ -1170,7 +1170,8 @@ int fls_batch_graph_launch(fls_batch* b, const fls_tune* tune, uint64_t* d_count
     if (!b || !d_counts) return FLS_ERR_NULL;
     int st;
     if ((st = check_tune(tune)) != FLS_OK) return st;
-    const bool same = b->exec && b->graph_tiles == b->tile_lists && b->graph_counts == d_counts && b->graph_tune.tile_vectors == tune->tile_vectors &&
+    const bool same = b->exec && b->graph_tiles == b->tile_lists && b->graph_counts == d_counts &&
+                      b->graph_tune.tile_vectors == tune->tile_vectors &&
                       b->graph_tune.block_threads == tune->block_threads && b->graph_tune.schedule == tune->schedule &&
                       b->graph_tune.class_tiles == tune->class_tiles;
     if (!same) {

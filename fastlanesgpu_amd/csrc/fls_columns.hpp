@@ -553,11 +553,6 @@ __device__ __forceinline__ uint32_t delta_mask_pre(const ColDev& c, fls_vmeta m,
     }
 }
 
-template <typename Pred>
-__device__ __forceinline__ uint32_t delta_mask(const ColDev& c, uint64_t v, Pred pred) {
-    return delta_mask_pre(c, c.vmeta[v], c.bases[v * 32u + dev::lane32()], pred);
-}
-
 // ------------------------------------------------------------------ row walks
 // One lane of one vector visited row by row: f(r, value) is called once per
 // register row r (a compile-time constant after unrolling, so a caller's

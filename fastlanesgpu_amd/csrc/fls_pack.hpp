@@ -8,10 +8,12 @@ namespace fls {
 
 // rows (row order) -> the lane's BW words at vec_out + lane + 32*k.  Stores are
 // non-temporal: an encoded column is larger than the caches, and left dirty in
-// them it is written back under the next kernel's reads (120M prices, learned:
-// 283 -> 250 us a pass; the first Q2.1 over columns just packed 222 -> 173 us,
-// Q4.1 190 -> 176, Q1.1 120 -> 111; only a 24-bit transposed pack by itself is
-// slower, 63.5 -> 67.4 us at 60M values).
+// them it is written back under the next kernel's reads.  Through the caches and
+// past them: 120M prices, learned, 283 and 250 us a pass; the first query over
+// columns just packed, Q2.1 198 and 147 us, Q4.1 158 and 143, Q1.1 101 and 87.  A
+// pack by itself gains at narrow widths and pays at wide ones, in either row
+// order: 60M values at 4 bits 47.0 and 43.1 us, 11 bits 50.3 and 48.9, 24 bits 63.3
+// and 66.5, 32 bits 70.2 and 78.9.
 template <int BW>
 __device__ __forceinline__ void pack_lane(const uint32_t (&x)[32], uint32_t* __restrict vec_out) {
     if constexpr (BW == 0) {

@@ -19,7 +19,7 @@ namespace fls {
 // one-block scan of the sums and an apply pass.  (With 4,096 entries per block,
 // too few to keep the loads moving, 7 us; mixed columns, which resolve their
 // plan in it, 6.6 against 9.6 for 117,188 vectors.)
-constexpr int kScanBlock = 1024, kScanPer = (int)kScanChunk / kScanBlock;
+constexpr int kScanBlock = (int)kScanChunk;  // a work-item per entry
 constexpr int kScanWaves = kScanBlock / 64;
 constexpr unsigned long long kScanReady = 1ull << 63;  // a published sum
 
@@ -60,17 +60,11 @@ __device__ __forceinline__ void scan_vectors(Load load, uint64_t n, unsigned lon
     const uint32_t b = s_ticket;
     if (b == kNoTicket) return;  // the whole block
     unsigned long long* sums = state + 1;
-    const uint64_t i0 = (uint64_t)b * kScanChunk + (uint64_t)kScanPer * t;
-    uint32_t w[kScanPer], bw[kScanPer], mine = 0, flags = 0;
-#pragma unroll
-    for (int k = 0; k < kScanPer; ++k) {
-        w[k] = bw[k] = 0u;
-        if (i0 + k < n) load(i0 + k, w[k], bw[k]);
-        mine += w[k];
-        flags += bw[k] >> 31;
-    }
+    const uint64_t i = (uint64_t)b * kScanChunk + t;
+    uint32_t w = 0, bw = 0;
+    if (i < n) load(i, w, bw);
     uint32_t total;
-    const uint32_t ex = block_exclusive_scan32(mine, sh, total);
+    const uint32_t ex = block_exclusive_scan32(w, sh, total);
     if (t == 0) atomicExch(&sums[b], kScanReady | total);
     asm volatile("" : : : "memory");  // published before the waits below
     uint64_t before = 0;
@@ -81,7 +75,7 @@ __device__ __forceinline__ void scan_vectors(Load load, uint64_t n, unsigned lon
         before += x & ~kScanReady;
     }
     before = dev::wave_sum(before);
-    flags = dev::wave_sum(flags);
+    const uint32_t flags = dev::wave_sum(bw >> 31);
     if (dev::is_wave_leader()) {
         sh64[t >> 6] = before;
         s_flags[t >> 6] = flags;
@@ -98,12 +92,7 @@ __device__ __forceinline__ void scan_vectors(Load load, uint64_t n, unsigned lon
         if (b == gridDim.x - 1u) *total_out = off + total;
         if (flagged && n_flags) atomicAdd(flagged, n_flags);
     }
-    off += ex;
-#pragma unroll
-    for (int k = 0; k < kScanPer; ++k) {
-        if (i0 + k < n) vmeta[i0 + k] = FLS_VMETA(off, bw[k] & 0xffu);
-        off += w[k];
-    }
+    if (i < n) vmeta[i] = FLS_VMETA(off + ex, bw & 0xffu);
 }
 
 }  // namespace fls

@@ -273,7 +273,7 @@ auto pick(const ColDev& c) {
 template <bool ROWS>
 int launch_order(const ColDev& c, uint64_t n_rows, uint32_t* d_out, hipStream_t s) {
     const uint64_t n_vec = ceil_div(n_rows, 1024);
-    const uint64_t work = ceil_div(n_vec, kMatVecs);  // a grid of every group: the grid-stride loop runs once
+    const uint64_t work = ceil_div(n_vec, kMatVecs);  // a grid of every group
     FLS_RETURN_IF(work > 0x7fffffffu, FLS_ERR_SIZE);
     const bool vec = reinterpret_cast<uintptr_t>(d_out) % 16u == 0;  // 16-byte stores where the output allows them
     auto k = vec ? rle_kernel<ROWS, true> : rle_kernel<ROWS, false>;
@@ -302,7 +302,7 @@ int fls_transpose_u32(const uint32_t* d_in, uint64_t n_vec, uint32_t inverse, ui
     FLS_RETURN_IF(d_in == d_out, FLS_ERR_ARG);
     FLS_RETURN_IF((reinterpret_cast<uintptr_t>(d_in) | reinterpret_cast<uintptr_t>(d_out)) % 16u, FLS_ERR_ARG);
     uint32_t grid = 0;
-    const uint64_t work = ceil_div(n_vec, kTrVecs);  // a grid of every group: the grid-stride loop runs once
+    const uint64_t work = ceil_div(n_vec, kTrVecs);  // a grid of every group
     FLS_RETURN_IF(work > 0x7fffffffu, FLS_ERR_SIZE);
     if (inverse) {
         grid = (uint32_t)work;

@@ -561,7 +561,7 @@ int fls_mixed_decode_u32(const uint32_t* d_words, const fls_vmeta* d_vmeta, cons
  *            (n rows of 16 floats) must be 16-byte aligned (FLS_ERR_ARG).
  *   grad: adds the gradient of the mean cross-entropy (inv_batch = 1/batch)
  *         over n rows into d_grad, the summed loss into *d_loss (may be NULL);
- *         d_work holds fls_mlp_grad_workspace_bytes(n) bytes.  Per-wave
+ *         d_work holds fls_mlp_grad_workspace_bytes(n) bytes.  Per-block
  *         partial sums are added in a fixed order: the result is
  *         bit-reproducible.
  *   adam: one Adam step (step >= 1) on the FP32 weights; refreshes d_wb and
