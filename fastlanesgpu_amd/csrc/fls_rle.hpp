@@ -62,24 +62,24 @@ __device__ __forceinline__ void rle_emit_wide(const RleVector& r, uint32_t last,
 
 // Decode the half-wave's vector to dst: rows 0..rows-1 in original order
 // (ROWS), or all 1,024 stored positions (rows = 1024).  VEC: dst is 16-byte
-// aligned.  ALIGNED: it is whether or not VEC is used; its stores are
-// non-temporal, those to other outputs are not, because they end in the middle
-// of a line (120M rows of mean run 8, unaligned: 199 us non-temporal, 144 this
-// way).  `lds` is this half-wave's; every exchange stays inside it.
-template <bool ROWS, bool VEC, bool ALIGNED = VEC>
+// aligned; otherwise stores go through the caches, because they end in the middle
+// of a line (120M rows of mean run 8: 199 us non-temporal, 144 this way).  LONG:
+// the form for waves with a vector of more runs than the stage holds.  `lds` is
+// this half-wave's; every exchange stays inside it.
+template <bool ROWS, bool VEC, bool LONG = false>
 __device__ __forceinline__ void rle_emit(const RleVector& r, RleLds& lds, uint32_t rows, uint32_t* __restrict dst) {
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     const uint32_t l = dev::lane32();
     const uint32_t nr = r.n_runs < 1024u ? r.n_runs : 1024u, last = nr ? nr - 1u : 0u;
     if (r.ibw > 1u) return rle_emit_wide<ROWS>(r, last, rows, dst);
-    if constexpr (VEC) {
+    if constexpr (!LONG) {
         // Two passes over the stage store only what each holds, so a word per
         // work-item at consecutive places: the words of a 16-byte store taken
         // one at a time touched four lines each (60M rows of 1,024 runs a
         // vector: row order 134 us, stored order 202; this way 94 and 143).  The
         // wave's two vectors go the same way, or both ways' code runs in turn
         // (vectors of about 512 runs 69 and 72 us apart, 64 and 70 together).
-        if (__any(last >= kRunStage)) return rle_emit<ROWS, false, ALIGNED>(r, lds, rows, dst);
+        if (__any(last >= kRunStage)) return rle_emit<ROWS, false, true>(r, lds, rows, dst);
     }
     // through the cache: RLE vectors end anywhere in a line, which the next one
     // shares (with non-temporal loads here a line was read twice: 62.2 us
@@ -167,13 +167,13 @@ __device__ __forceinline__ void rle_emit(const RleVector& r, RleLds& lds, uint32
             }
             const uint32_t p = VEC ? 4u * l + 128u * (uint32_t)j : 128u * (uint32_t)j + l;
             constexpr uint32_t step = VEC ? 1u : 32u;  // place of output 4j + i: p + step * i
-            if ((VEC || last < kRunStage) && p + 3u * step < rows) {
+            if ((!LONG || last < kRunStage) && p + 3u * step < rows) {
                 if constexpr (VEC) {
                     __builtin_nontemporal_store(u32x4{x[0], x[1], x[2], x[3]}, reinterpret_cast<u32x4*>(dst + p));
                 } else {
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        if constexpr (ALIGNED) __builtin_nontemporal_store(x[i], dst + p + step * i);
+                        if constexpr (LONG) __builtin_nontemporal_store(x[i], dst + p + step * i);
                         else dst[p + step * i] = x[i];
                     }
                 }
@@ -185,7 +185,7 @@ __device__ __forceinline__ void rle_emit(const RleVector& r, RleLds& lds, uint32
             __builtin_amdgcn_sched_barrier(0);  // few outputs in flight: their registers cost more waves than they hide
         }
         from += kRunStage;
-        if (VEC || from > last) break;
+        if (!LONG || from > last) break;
         fence();
         stage(from, min(last + 1u, from + kRunStage));
         fence();
