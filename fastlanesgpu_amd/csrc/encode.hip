@@ -24,8 +24,10 @@ constexpr int kVecPerBlock = kBlock / 32;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // ------------------------------------------------------------------ bitpack
-// Rows 32j + l of vector v minus base, rows past n zero.  In normal order
-// these are the lane's own rows; TRANSPOSED sends them through the LDS tile
+// Rows 32j + l of vector v minus base, rows past n zero (loaded as the last row
+// and then cleared: a load under a condition is waited for before the next one,
+// 32 round trips, and 100,003 values not read before took 14.0 us instead of 6.2).
+// In normal order these are the lane's own rows; TRANSPOSED sends them through the LDS tile
 // (the lane's row rsum_row(j) is element j of its chain).
 template <int BW, bool TRANSPOSED>
 __global__ __launch_bounds__(kBlock) void pack_kernel(const uint32_t* __restrict in, uint64_t n, uint32_t base,
@@ -42,7 +44,9 @@ __global__ __launch_bounds__(kBlock) void pack_kernel(const uint32_t* __restrict
             for (int r = 0; r < 32; ++r) x[r] = __builtin_nontemporal_load(in + i0 + 32u * r) - base;
         } else {
 #pragma unroll
-            for (int r = 0; r < 32; ++r) x[r] = i0 + 32u * r < n ? in[i0 + 32u * r] - base : 0u;
+            for (int r = 0; r < 32; ++r) x[r] = padded(in, n, i0 + 32u * r) - base;
+#pragma unroll
+            for (int r = 0; r < 32; ++r) x[r] = i0 + 32u * r < n ? x[r] : 0u;
         }
     }
     if constexpr (TRANSPOSED) {
